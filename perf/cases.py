@@ -263,6 +263,90 @@ def run(state):
     return _run_stack(state) if state["case"]["path"] == "stack" else _run_scan(state)
 
 
+# ---------------------------------------------------------------------------------- the same in 64 bits
+def _scan64(u, x, weight_c, bias, c0, hidden, dirs, k, tanh, scale, mask_c, pad):
+    """The recurrence written out step by step: u (L, B, D * k), x (L, B, D) or None -> h, last state."""
+    L, B = u.shape[:2]
+    D = hidden * dirs
+    u = u.view(L, B, D, k)
+    w1, w2, b1, b2 = weight_c[:D], weight_c[D:], bias[:D], bias[D:]
+    skip = u[..., 3] if k == 4 else x.view(L, B, D) * scale
+    c0 = u.new_zeros(B, D) if c0 is None else c0
+    hs, lasts = [], []
+    for i in range(dirs):
+        cols = slice(i * hidden, (i + 1) * hidden)
+        reverse = (lambda t: t.flip(0)) if i else (lambda t: t)
+        uu, ss = reverse(u[:, :, cols]), reverse(skip[:, :, cols])
+        keep = None if pad is None else reverse(pad)[..., None]
+        c, prev, cur = c0[:, cols], [], []
+        u0, u1 = uu[..., 0].unbind(0), (uu[..., 1] + b1[cols]).unbind(0)
+        for t in range(L):
+            prev.append(c)
+            new = torch.lerp(u0[t], c, torch.sigmoid(torch.addcmul(u1[t], w1[cols], c)))
+            c = new if keep is None else torch.where(keep[t], c, new)
+            cur.append(c)
+        prev, cur = torch.stack(prev), torch.stack(cur)
+        out = torch.sigmoid(uu[..., 2] + w2[cols] * prev + b2[cols])
+        if mask_c is not None:
+            out = out * mask_c[:, cols]
+        h = ss + ((torch.tanh(cur) if tanh else cur) - ss) * out
+        hs.append(reverse(h if keep is None else h.masked_fill(keep, 0.0)))
+        lasts.append(c)
+    return torch.cat(hs, -1), torch.cat(lasts, -1)
+
+
+def _stack64(case, named, x, c0, pad):
+    dirs = 2 if case["bidirectional"] else 1
+    L, B, D = case["length"], case["batch"], case["hidden"] * dirs
+    finals = []
+    for i in range(case["layers"]):
+        get = lambda n: named.get(f"rnn_lst.{i}.{n}")
+        k = get("weight").size(1) // D
+        y = x
+        if get("layer_norm.weight") is not None:
+            y = torch.nn.functional.layer_norm(x, x.shape[-1:], get("layer_norm.weight"), get("layer_norm.bias"), 1e-5)
+        y = y.reshape(L * B, -1)
+        if get("weight_proj") is not None:
+            y = y @ get("weight_proj")
+        scale = get("scale_x") if case["rescale"] else 1.0
+        x, last = _scan64((y @ get("weight")).view(L, B, -1), x, get("weight_c"), get("bias"),
+                          None if c0 is None else c0[i], case["hidden"], dirs, k, False, scale, None, pad)
+        finals.append(last)
+    return x, torch.stack(finals)
+
+
+def exact(case, seed):
+    s = prepare(case, seed)
+    wide = lambda t: None if t is None else t.detach().double().requires_grad_(t.requires_grad)
+    if case["path"] == "scan":
+        t = {n: wide(s[n]) for n in ("u", "x", "weight_c", "bias", "c0", "scale", "mask_c")}
+        h, last = _scan64(t["u"], t["x"], t["weight_c"], t["bias"], t["c0"], case["hidden"],
+                          2 if case["bidirectional"] else 1, case["k"], case["tanh"],
+                          1.0 if t["scale"] is None else t["scale"], t["mask_c"], s["mask"])
+        inputs = {n: t[n] for n in ("u", "x", "weight_c", "bias", "c0") if t[n] is not None and t[n].requires_grad}
+        outputs, seeds = [h], [s["grad_h"].double()]
+        if s["grad_last"] is not None:
+            outputs.append(last)
+            seeds.append(s["grad_last"].double())
+        grads = torch.autograd.grad(outputs, list(inputs.values()), seeds)
+        out = {"h": h.detach(), "last": last.detach()}
+        out.update(("grad_" + n, g) for n, g in zip(inputs, grads))
+        return out
+    params = {n: wide(p) for n, p in s["model"].named_parameters()}
+    named = dict(params, **{n: b.double() for n, b in s["model"].named_buffers()})
+    x, c0 = wide(s["x"]), wide(s["c0"])
+    if case["mode"] == "infer":
+        with torch.no_grad():
+            h, c = _stack64(case, named, x, c0, s["mask"])
+        return {"h": h, "c": c}
+    h, c = _stack64(case, named, x, c0, s["mask"])
+    wanted = dict(params, x=x) if x.requires_grad else params
+    grads = torch.autograd.grad([h], list(wanted.values()), [s["probe"].double()])
+    out = {"h": h.detach(), "c": c.detach()}
+    out.update(("grad_" + n, g) for n, g in zip(wanted, grads))
+    return out
+
+
 # ---------------------------------------------------------------------------------- what a pass needs
 def _bytes(name):
     return DTYPES[name].itemsize
