@@ -143,6 +143,26 @@ int sru_amd_forward(const sru_amd_shape *shape,
                     const uint8_t *mask_pad, const void *scale_x,
                     void *h, void *c, void *c_last, void *stream);
 
+/* Which small tensors are held in shape->dtype instead of float, for the two calls below: one bit
+ * each. Beside 16-bit streams only (BAD_FLAGS otherwise); SRU_AMD_SMALL_WEIGHT_C needs is_custom 0.
+ * A tensor held in 16 bits needs 2-byte alignment. The kernels decode the values as they read them:
+ * results are those of converting the tensor to float first. */
+#define SRU_AMD_SMALL_WEIGHT_C 1u
+#define SRU_AMD_SMALL_BIAS 2u
+#define SRU_AMD_SMALL_INIT 4u     /* c_init; forward only */
+#define SRU_AMD_SMALL_MASK 8u     /* mask_c */
+#define SRU_AMD_SMALL_SCALE 16u   /* scale_x */
+#define SRU_AMD_SMALL_LAST 32u    /* c_last (forward, rounded to nearest even), grad_last (backward) */
+#define SRU_AMD_SMALL_ALL 63u
+
+/* sru_amd_forward with the small tensors named in `small16` in shape->dtype. No counterpart in the
+ * reference, whose callers convert (sru/ops.py:116-127). */
+int sru_amd_forward_small(const sru_amd_shape *shape, uint32_t small16,
+                          const void *u, const void *x, const void *weight_c,
+                          const void *bias, const void *c_init, const void *mask_c,
+                          const uint8_t *mask_pad, const void *scale_x,
+                          void *h, void *c, void *c_last, void *stream);
+
 /* Bytes of the state buffer `c` that sru_amd_forward fills and sru_amd_backward reads for
  * `shape`, according to shape->state_interval (0 on a bad shape). */
 size_t sru_amd_state_bytes(const sru_amd_shape *shape);
@@ -176,6 +196,17 @@ int sru_amd_backward(const sru_amd_shape *shape,
                      void *grad_u, void *grad_x, void *grad_wc, void *grad_bias,
                      void *grad_init, void *workspace, size_t workspace_bytes,
                      void *stream);
+
+/* sru_amd_backward with the small inputs named in `small16` in shape->dtype (SRU_AMD_SMALL_INIT is
+ * refused; the gradients written are float as above). */
+int sru_amd_backward_small(const sru_amd_shape *shape, uint32_t small16,
+                           const void *u, const void *x, const void *weight_c,
+                           const void *bias, const void *c_init, const void *mask_c,
+                           const uint8_t *mask_pad, const void *scale_x,
+                           const void *c, const void *grad_h, const void *grad_last,
+                           void *grad_u, void *grad_x, void *grad_wc, void *grad_bias,
+                           void *grad_init, void *workspace, size_t workspace_bytes,
+                           void *stream);
 
 /* sru_amd_backward without the workspace argument, for callers that cannot allocate device
  * memory at all: code under HIP graph capture, tight serving loops, harnesses that forbid

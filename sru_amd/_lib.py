@@ -16,6 +16,8 @@ NORM_MAX_FEATURES = 4096       # SRU_AMD_NORM_MAX_FEATURES
 
 F32, F16, BF16, F64 = 0, 1, 2, 3
 X_AS_STREAMS, X_F32 = 0, 1   # SRU_AMD_X_AS_STREAMS, SRU_AMD_X_F32
+# SRU_AMD_SMALL_*: small tensors held in the stream type
+SMALL_WEIGHT_C, SMALL_BIAS, SMALL_INIT, SMALL_MASK, SMALL_SCALE, SMALL_LAST = 1, 2, 4, 8, 16, 32
 
 
 class Shape(ctypes.Structure):
@@ -39,9 +41,11 @@ _P = ctypes.c_void_p
 SIGNATURES = {
     # name: (restype, argtypes) exactly as declared in include/sru_amd.h
     "sru_amd_forward": (ctypes.c_int, [ctypes.POINTER(Shape)] + [_P] * 12),
+    "sru_amd_forward_small": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32] + [_P] * 12),
     "sru_amd_state_bytes": (ctypes.c_size_t, [ctypes.POINTER(Shape)]),
     "sru_amd_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Shape)]),
     "sru_amd_backward": (ctypes.c_int, [ctypes.POINTER(Shape)] + [_P] * 17 + [ctypes.c_size_t, _P]),
+    "sru_amd_backward_small": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32] + [_P] * 17 + [ctypes.c_size_t, _P]),
     "sru_amd_backward_static": (ctypes.c_int, [ctypes.POINTER(Shape)] + [_P] * 17),
     "sru_amd_layer_norm_forward": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, _P, ctypes.c_int, _P, _P,
                                                   ctypes.c_float, _P, ctypes.c_int, _P, _P, _P]),

@@ -92,6 +92,17 @@ int check_shape(const sru_amd_shape *s) {
     return SRU_AMD_OK;
 }
 
+// Small tensors in the stream type: only beside 16-bit streams, and weight_c only as a vector (a
+// per-step weight_c is a stream).
+int check_small(const sru_amd_shape &s, uint32_t small16) {
+    if (small16 & ~(uint32_t)SRU_AMD_SMALL_ALL) return SRU_AMD_ERR_BAD_FLAGS;
+    if (small16 && elem_size(s.dtype) != 2) return SRU_AMD_ERR_BAD_FLAGS;
+    if ((small16 & SRU_AMD_SMALL_WEIGHT_C) && s.is_custom) return SRU_AMD_ERR_BAD_FLAGS;
+    return SRU_AMD_OK;
+}
+static_assert(SRU_AMD_SMALL_WEIGHT_C == kSmallWeightC && SRU_AMD_SMALL_BIAS == kSmallBias && SRU_AMD_SMALL_INIT == kSmallInit &&
+              SRU_AMD_SMALL_MASK == kSmallMask && SRU_AMD_SMALL_SCALE == kSmallScale && SRU_AMD_SMALL_LAST == kSmallLast, "header and kernels disagree");
+
 // Everything sru_amd_backward and sru_amd_backward_static share: pointer checks, then the
 // scan and the batch reduction enqueued on `stream`, with the per-column partial sums in
 // `partial` (4 * B * D' floats of device memory).
@@ -99,8 +110,10 @@ int backward_core(const sru_amd_shape *shape, const void *u, const void *x, cons
                   const void *bias, const void *c_init, const void *mask_c, const uint8_t *mask_pad,
                   const void *scale_x, const void *c, const void *grad_h, const void *grad_last,
                   void *grad_u, void *grad_x, void *grad_wc, void *grad_bias, void *grad_init,
-                  void *partial, void *stream) {
+                  void *partial, void *stream, uint32_t small16 = 0) {
     const sru_amd_shape &s = *shape;
+    if (const int rc = check_small(s, small16)) return rc;
+    if (small16 & SRU_AMD_SMALL_INIT) return SRU_AMD_ERR_BAD_FLAGS;   // the chunk kernels select between it and a float checkpoint
     if (!u || !weight_c || !bias || !c || !grad_h || !grad_u || !grad_wc || !grad_bias || !grad_init)
         return SRU_AMD_ERR_NULL_POINTER;
     if (s.skip_type == 1 && (!x || !grad_x)) return SRU_AMD_ERR_NULL_POINTER;
@@ -110,11 +123,13 @@ int backward_core(const sru_amd_shape *shape, const void *u, const void *x, cons
     const bool x_float = x_is_float_beside_16bit(s);
     if (x_float && !ckpt) return SRU_AMD_ERR_BAD_FLAGS;
     const size_t xs = x_float ? 4 : es;
+    auto small_align = [&](uint32_t bit) { return (small16 & bit) ? es : ss; };
     if (!aligned(u, group) || !aligned(grad_u, group) || !aligned(c, ckpt ? 4 : es) || !aligned(grad_h, es) ||
         (s.skip_type == 1 && (!aligned(x, xs) || !aligned(grad_x, xs))) ||
-        !aligned(weight_c, s.is_custom ? 2 * es : ss) || !aligned(grad_wc, s.is_custom ? 2 * es : ss) ||
-        !aligned(bias, ss) || (c_init && !aligned(c_init, ss)) || (grad_last && !aligned(grad_last, ss)) || !aligned(grad_bias, ss) ||
-        !aligned(grad_init, ss) || (mask_c && !aligned(mask_c, ss)) || (scale_x && !aligned(scale_x, ss)))
+        !aligned(weight_c, s.is_custom ? 2 * es : small_align(SRU_AMD_SMALL_WEIGHT_C)) || !aligned(grad_wc, s.is_custom ? 2 * es : ss) ||
+        !aligned(bias, small_align(SRU_AMD_SMALL_BIAS)) || (c_init && !aligned(c_init, ss)) ||
+        (grad_last && !aligned(grad_last, small_align(SRU_AMD_SMALL_LAST))) || !aligned(grad_bias, ss) || !aligned(grad_init, ss) ||
+        (mask_c && !aligned(mask_c, small_align(SRU_AMD_SMALL_MASK))) || (scale_x && !aligned(scale_x, small_align(SRU_AMD_SMALL_SCALE))))
         return SRU_AMD_ERR_MISALIGNED;
 
     if (ckpt && es == 2 &&
@@ -123,11 +138,10 @@ int backward_core(const sru_amd_shape *shape, const void *u, const void *x, cons
          (s.skip_type == 1 && (!aligned(x, 4) || !aligned(grad_x, 4)))))
         return SRU_AMD_ERR_MISALIGNED;
 
-    // (the parameter block types the small tensors as float; the double kernels know better)
-    auto small = [](const void *q) { return static_cast<const float *>(q); };
+    // (the parameter block types what is always float or double as float; the double kernels know better)
     BwdParams p{};
-    p.u = u; p.x = x; p.wc = weight_c; p.bias = small(bias); p.c0 = small(c_init); p.mask_c = small(mask_c);
-    p.pad = mask_pad; p.scale_x = small(scale_x); p.gh = grad_h; p.glast = small(grad_last);
+    p.u = u; p.x = x; p.wc = weight_c; p.bias = bias; p.c0 = static_cast<const float *>(c_init); p.mask_c = mask_c;
+    p.pad = mask_pad; p.scale_x = scale_x; p.gh = grad_h; p.glast = grad_last; p.small16 = small16;
     p.c = ckpt ? nullptr : c;
     p.ckpt = ckpt ? static_cast<const float *>(c) : nullptr;
     p.gu = grad_u; p.gx = grad_x; p.gwc_steps = s.is_custom ? grad_wc : nullptr;
@@ -177,11 +191,20 @@ int sru_amd_forward(const sru_amd_shape *shape, const void *u, const void *x, co
                     const void *bias, const void *c_init, const void *mask_c,
                     const uint8_t *mask_pad, const void *scale_x, void *h, void *c, void *c_last,
                     void *stream) {
+    return sru_amd_forward_small(shape, 0, u, x, weight_c, bias, c_init, mask_c, mask_pad, scale_x, h, c, c_last, stream);
+}
+
+int sru_amd_forward_small(const sru_amd_shape *shape, uint32_t small16, const void *u, const void *x, const void *weight_c,
+                          const void *bias, const void *c_init, const void *mask_c,
+                          const uint8_t *mask_pad, const void *scale_x, void *h, void *c, void *c_last,
+                          void *stream) {
     if (const int rc = check_shape(shape)) return rc;
     const sru_amd_shape &s = *shape;
+    if (const int rc = check_small(s, small16)) return rc;
     if (!u || !weight_c || !bias || !h || !c_last) return SRU_AMD_ERR_NULL_POINTER;
     if (s.skip_type == 1 && !x) return SRU_AMD_ERR_NULL_POINTER;
     const size_t es = elem_size(s.dtype), ss = small_size(s.dtype);
+    auto small_align = [&](uint32_t bit) { return (small16 & bit) ? es : ss; };
     const size_t group = (s.k == 4) ? (es == 8 ? 16 : 4 * es) : es;  // a k=4 group moves as one vector (doubles: as two)
     const bool ckpt = s.state_interval == SRU_AMD_STATE_INTERVAL;
     const bool x_float = x_is_float_beside_16bit(s);
@@ -189,9 +212,10 @@ int sru_amd_forward(const sru_amd_shape *shape, const void *u, const void *x, co
     // (a float x still travels with 16-bit streams that move two columns at a time)
     if (x_float && (!aligned(u, s.k == 4 ? 16 : 4) || !aligned(h, 4))) return SRU_AMD_ERR_MISALIGNED;
     if (!aligned(u, group) || !aligned(h, es) || (c && !aligned(c, ckpt ? 4 : es)) ||
-        (s.skip_type == 1 && !aligned(x, x_float ? 4 : es)) || !aligned(weight_c, s.is_custom ? 2 * es : ss) ||
-        !aligned(bias, ss) || (c_init && !aligned(c_init, ss)) || !aligned(c_last, ss) ||
-        (mask_c && !aligned(mask_c, ss)) || (scale_x && !aligned(scale_x, ss)))
+        (s.skip_type == 1 && !aligned(x, x_float ? 4 : es)) ||
+        !aligned(weight_c, s.is_custom ? 2 * es : small_align(SRU_AMD_SMALL_WEIGHT_C)) || !aligned(bias, small_align(SRU_AMD_SMALL_BIAS)) ||
+        (c_init && !aligned(c_init, small_align(SRU_AMD_SMALL_INIT))) || !aligned(c_last, small_align(SRU_AMD_SMALL_LAST)) ||
+        (mask_c && !aligned(mask_c, small_align(SRU_AMD_SMALL_MASK))) || (scale_x && !aligned(scale_x, small_align(SRU_AMD_SMALL_SCALE))))
         return SRU_AMD_ERR_MISALIGNED;
 
     // 16-bit streams with checkpoints move two columns at a time
@@ -200,11 +224,9 @@ int sru_amd_forward(const sru_amd_shape *shape, const void *u, const void *x, co
          (s.skip_type == 1 && !aligned(x, 4))))
         return SRU_AMD_ERR_MISALIGNED;
 
-    // (the parameter block types the small tensors as float; the double kernels know better)
-    auto small = [](const void *q) { return static_cast<const float *>(q); };
     FwdParams p{};
-    p.u = u; p.x = x; p.wc = weight_c; p.bias = small(bias); p.c0 = small(c_init); p.mask_c = small(mask_c);
-    p.pad = mask_pad; p.scale_x = small(scale_x); p.h = h; p.c_last = static_cast<float *>(c_last);
+    p.u = u; p.x = x; p.wc = weight_c; p.bias = bias; p.c0 = c_init; p.mask_c = mask_c;
+    p.pad = mask_pad; p.scale_x = scale_x; p.h = h; p.c_last = c_last; p.small16 = small16;
     p.c = ckpt ? nullptr : c;
     p.ckpt = ckpt ? static_cast<float *>(c) : nullptr;
     p.L = s.length; p.B = s.batch; p.d = (int32_t)s.hidden; p.Dp = (int32_t)(s.hidden * s.dirs);
@@ -239,12 +261,22 @@ int sru_amd_backward(const sru_amd_shape *shape, const void *u, const void *x, c
                      const void *grad_h, const void *grad_last, void *grad_u, void *grad_x,
                      void *grad_wc, void *grad_bias, void *grad_init, void *workspace,
                      size_t workspace_bytes, void *stream) {
+    return sru_amd_backward_small(shape, 0, u, x, weight_c, bias, c_init, mask_c, mask_pad, scale_x, c, grad_h, grad_last,
+                                  grad_u, grad_x, grad_wc, grad_bias, grad_init, workspace, workspace_bytes, stream);
+}
+
+int sru_amd_backward_small(const sru_amd_shape *shape, uint32_t small16, const void *u, const void *x, const void *weight_c,
+                           const void *bias, const void *c_init, const void *mask_c,
+                           const uint8_t *mask_pad, const void *scale_x, const void *c,
+                           const void *grad_h, const void *grad_last, void *grad_u, void *grad_x,
+                           void *grad_wc, void *grad_bias, void *grad_init, void *workspace,
+                           size_t workspace_bytes, void *stream) {
     if (const int rc = check_shape(shape)) return rc;
     if (!workspace || !aligned(workspace, 16) ||
         workspace_bytes < sru_amd_backward_workspace_bytes(shape))
         return SRU_AMD_ERR_WORKSPACE;
     return backward_core(shape, u, x, weight_c, bias, c_init, mask_c, mask_pad, scale_x, c, grad_h, grad_last,
-                         grad_u, grad_x, grad_wc, grad_bias, grad_init, workspace, stream);
+                         grad_u, grad_x, grad_wc, grad_bias, grad_init, workspace, stream, small16);
 }
 
 int sru_amd_backward_static(const sru_amd_shape *shape, const void *u, const void *x, const void *weight_c,

@@ -365,28 +365,101 @@ __device__ __forceinline__ arith_t<T> tanh_of(arith_t<T> v) {
 template <typename A> __device__ __forceinline__ const A *as_arith(const float *q) { return reinterpret_cast<const A *>(q); }
 template <typename A> __device__ __forceinline__ A *as_arith(float *q) { return reinterpret_cast<A *>(q); }
 
+// A small tensor beside 16-bit streams may itself be held in the stream type (a layer whose
+// parameters and states are 16-bit): `small16` says which ones are, one bit each. The kernels read
+// them as they are, once per column: converting them in front of every call took a launch of
+// 2-5 us per tensor (ten layers decoding one token: 40 of 71 launches). The element is fetched
+// first and decoded when it is used, so that the prologue's loads stay in flight together.
+constexpr uint32_t kSmallWeightC = 1, kSmallBias = 2, kSmallInit = 4, kSmallMask = 8, kSmallScale = 16, kSmallLast = 32;
+template <typename T> struct SmallElem {
+    arith_t<T> v;
+    __device__ __forceinline__ void fetch(const void *q, int64_t i, bool) { v = static_cast<const arith_t<T> *>(q)[i]; }
+    __device__ __forceinline__ arith_t<T> get(bool) const { return v; }
+};
+template <typename T> struct SmallElem16 {
+    uint32_t v;
+    __device__ __forceinline__ void fetch(const void *q, int64_t i, bool narrow) {
+        if (narrow) v = static_cast<const uint16_t *>(q)[i];
+        else v = static_cast<const uint32_t *>(q)[i];
+    }
+    __device__ __forceinline__ float get(bool narrow) const {
+        return narrow ? bits_to_float<T>(v & 0xffffu) : __builtin_bit_cast(float, v);
+    }
+};
+template <> struct SmallElem<half_bits> : SmallElem16<half_bits> {};
+template <> struct SmallElem<bf16_bits> : SmallElem16<bf16_bits> {};
+
+// the state after the last step, written in the type the caller asked for
+template <typename T>
+__device__ __forceinline__ void put_last(void *q, int64_t i, arith_t<T> v, bool narrow) {
+    if constexpr (sizeof(T) == 2) {
+        if (narrow) {
+            static_cast<uint16_t *>(q)[i] = (uint16_t)float_to_bits<T>(v);
+            return;
+        }
+    }
+    static_cast<arith_t<T> *>(q)[i] = v;
+}
+// The per-column operands every kernel starts from. All loads are issued before the first value is
+// decoded.
+template <typename T, int COLS> struct ColumnOperands {
+    arith_t<T> w1[COLS], w2[COLS], b1[COLS], b2[COLS], m[COLS], start[COLS], sx;
+    // j: first column inside a row, col: first column of all; start: initial state or last-state gradient
+    template <typename P>
+    __device__ __forceinline__ void fetch(const P &p, const void *start_of, bool start16, bool vector_wc, bool scaled, int j, int64_t col) {
+        using A = arith_t<T>;
+        SmallElem<T> ew1[COLS], ew2[COLS], eb1[COLS], eb2[COLS], em[COLS], es[COLS], ex;
+        const bool wc16 = (p.small16 & kSmallWeightC) != 0, bias16 = (p.small16 & kSmallBias) != 0;
+        const bool mask16 = (p.small16 & kSmallMask) != 0, scale16 = (p.small16 & kSmallScale) != 0;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            if (vector_wc) {
+                ew1[c].fetch(p.wc, j + c, wc16);
+                ew2[c].fetch(p.wc, p.Dp + j + c, wc16);
+            }
+            eb1[c].fetch(p.bias, j + c, bias16);
+            eb2[c].fetch(p.bias, p.Dp + j + c, bias16);
+            if (p.mask_c) em[c].fetch(p.mask_c, col + c, mask16);
+            if (start_of) es[c].fetch(start_of, col + c, start16);
+        }
+        if (scaled && p.scale_x) ex.fetch(p.scale_x, 0, scale16);
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            w1[c] = vector_wc ? ew1[c].get(wc16) : A(0);
+            w2[c] = vector_wc ? ew2[c].get(wc16) : A(0);
+            b1[c] = eb1[c].get(bias16);
+            b2[c] = eb2[c].get(bias16);
+            m[c] = p.mask_c ? em[c].get(mask16) : A(1);
+            start[c] = start_of ? es[c].get(start16) : A(0);   // not given: zeros
+        }
+        sx = (scaled && p.scale_x) ? ex.get(scale16) : A(1);
+    }
+};
+
 struct FwdParams {
     const void *u, *x, *wc;
-    const float *bias, *c0, *mask_c;
+    const void *bias, *c0, *mask_c;
     const uint8_t *pad;
-    const float *scale_x;
+    const void *scale_x;
     void *h, *c;
-    float *c_last;
+    void *c_last;
     float *ckpt;          // (L / kCkptInterval, B, D') float state checkpoints, or nullptr
     int64_t L, B, ncols;  // ncols = B * D'
     int32_t d, Dp;        // hidden per direction, D' = dirs * d
     int32_t act, custom;  // act: host-side kernel selection and the general kernels; custom: general kernels
     int32_t x_float;      // host-side kernel selection: x is float next to 16-bit streams
+    uint32_t small16;     // which small tensors are held in the stream type (16-bit streams only)
 };
 
 struct BwdParams {
     const void *u, *x, *wc;
-    const float *bias, *c0, *mask_c;
+    const void *bias, *mask_c;
+    const float *c0;
     const uint8_t *pad;
-    const float *scale_x;
+    const void *scale_x;
     const void *c, *gh;
     const float *ckpt;    // state checkpoints written by the forward pass (checkpoint kernels)
-    const float *glast;
+    const void *glast;
     void *gu, *gx, *gwc_steps;  // gwc_steps: per-step weight_c gradient (custom only)
     float *ginit;
     float *partial;  // (4, ncols): per-column sums gwc1, gwc2, gbias1, gbias2
@@ -394,6 +467,7 @@ struct BwdParams {
     int32_t d, Dp;
     int32_t act, custom;
     int32_t x_float;      // host-side kernel selection: x and grad_x are float next to 16-bit streams
+    uint32_t small16;     // which small tensors are held in the stream type (16-bit streams only)
 };
 
 // Every field of the parameter block is read at the top of a kernel. Left alone, the compiler
@@ -405,14 +479,14 @@ __device__ __forceinline__ void fetch_params_early(const FwdParams &p) {
     SRU_AMD_PIN(p.u); SRU_AMD_PIN(p.x); SRU_AMD_PIN(p.wc); SRU_AMD_PIN(p.bias); SRU_AMD_PIN(p.c0);
     SRU_AMD_PIN(p.mask_c); SRU_AMD_PIN(p.pad); SRU_AMD_PIN(p.scale_x); SRU_AMD_PIN(p.h); SRU_AMD_PIN(p.c);
     SRU_AMD_PIN(p.c_last); SRU_AMD_PIN(p.ckpt); SRU_AMD_PIN(p.L); SRU_AMD_PIN(p.B); SRU_AMD_PIN(p.ncols);
-    SRU_AMD_PIN(p.d); SRU_AMD_PIN(p.Dp);
+    SRU_AMD_PIN(p.d); SRU_AMD_PIN(p.Dp); SRU_AMD_PIN(p.small16);
 }
 __device__ __forceinline__ void fetch_params_early(const BwdParams &p) {
     SRU_AMD_PIN(p.u); SRU_AMD_PIN(p.x); SRU_AMD_PIN(p.wc); SRU_AMD_PIN(p.bias); SRU_AMD_PIN(p.c0);
     SRU_AMD_PIN(p.mask_c); SRU_AMD_PIN(p.pad); SRU_AMD_PIN(p.scale_x); SRU_AMD_PIN(p.c); SRU_AMD_PIN(p.gh);
     SRU_AMD_PIN(p.ckpt); SRU_AMD_PIN(p.glast); SRU_AMD_PIN(p.gu); SRU_AMD_PIN(p.gx); SRU_AMD_PIN(p.gwc_steps);
     SRU_AMD_PIN(p.ginit); SRU_AMD_PIN(p.partial); SRU_AMD_PIN(p.L); SRU_AMD_PIN(p.B); SRU_AMD_PIN(p.ncols);
-    SRU_AMD_PIN(p.d); SRU_AMD_PIN(p.Dp);
+    SRU_AMD_PIN(p.d); SRU_AMD_PIN(p.Dp); SRU_AMD_PIN(p.small16);
 }
 
 // The loop body must stay one straight line of code for the compiler to keep the ring
@@ -487,17 +561,11 @@ __global__ void __launch_bounds__(kBlock * 4) forward_scan(const FwdParams p) {
     const bool has_pad = GENERAL ? (p.pad != nullptr) : ((MODE & kHasPad) != 0);
     const bool keep_c = GENERAL ? (p.c != nullptr) : ((MODE & kKeepC) != 0);
 
-    A wc1[COLS], wc2[COLS], b1[COLS], b2[COLS], m[COLS], cur[COLS];
-#pragma unroll
-    for (int c = 0; c < COLS; ++c) {
-        wc1[c] = custom ? A(0) : static_cast<const A *>(p.wc)[j + c];
-        wc2[c] = custom ? A(0) : static_cast<const A *>(p.wc)[Dp + j + c];
-        b1[c] = as_arith<A>(p.bias)[j + c];
-        b2[c] = as_arith<A>(p.bias)[Dp + j + c];
-        m[c] = p.mask_c ? as_arith<A>(p.mask_c)[col + c] : A(1);
-        cur[c] = p.c0 ? as_arith<A>(p.c0)[col + c] : A(0);   // no initial state given: zeros
-    }
-    const A sx = (SKIP == 1 && p.scale_x) ? *as_arith<A>(p.scale_x) : A(1);
+    ColumnOperands<T, COLS> op;
+    op.fetch(p, p.c0, (p.small16 & kSmallInit) != 0, !custom, SKIP == 1, j, col);
+    const auto &wc1 = op.w1, &wc2 = op.w2, &b1 = op.b1, &b2 = op.b2, &m = op.m;
+    auto &cur = op.start;
+    const A sx = op.sx;
 
     const int64_t L = p.L;
     const int64_t e0 = (flip ? (L - 1) : 0) * p.ncols + col;  // element of the first walk step
@@ -592,7 +660,7 @@ __global__ void __launch_bounds__(kBlock * 4) forward_scan(const FwdParams p) {
         }
     }
 #pragma unroll
-    for (int c = 0; c < COLS; ++c) as_arith<A>(p.c_last)[col + c] = cur[c];
+    for (int c = 0; c < COLS; ++c) put_last<T>(p.c_last, col + c, cur[c], (p.small16 & kSmallLast) != 0);
 }
 
 // Window of a wavefront's walk outside of which every step is padded, for wavefronts whose lanes
@@ -668,17 +736,11 @@ __global__ void __launch_bounds__(kBlock * max_waves_per_group<T>(MODE)) forward
     const int j = ju + (int)lane;
     const bool flip = ju >= p.d;
 
-    float wc1[COLS], wc2[COLS], b1[COLS], b2[COLS], m[COLS], cur[COLS];
-#pragma unroll
-    for (int c = 0; c < COLS; ++c) {
-        wc1[c] = CUSTOM ? 0.f : static_cast<const float *>(p.wc)[j + c];
-        wc2[c] = CUSTOM ? 0.f : static_cast<const float *>(p.wc)[Dp + j + c];
-        b1[c] = p.bias[j + c];
-        b2[c] = p.bias[Dp + j + c];
-        m[c] = p.mask_c ? p.mask_c[col + c] : 1.0f;
-        cur[c] = p.c0 ? p.c0[col + c] : 0.0f;   // no initial state given: zeros
-    }
-    const float sx = (SKIP == 1 && p.scale_x) ? *p.scale_x : 1.0f;
+    ColumnOperands<T, COLS> op;
+    op.fetch(p, p.c0, (p.small16 & kSmallInit) != 0, !CUSTOM, SKIP == 1, j, col);
+    const auto &wc1 = op.w1, &wc2 = op.w2, &b1 = op.b1, &b2 = op.b2, &m = op.m;
+    auto &cur = op.start;
+    const float sx = op.sx;
 
     const int64_t L = p.L;
     const int64_t ef = (flip ? (L - 1) : 0) * p.ncols + colu;  // element of walk step 0 (column colu)
@@ -818,7 +880,7 @@ __global__ void __launch_bounds__(kBlock * max_waves_per_group<T>(MODE)) forward
     }
     if constexpr (HAS_PAD && UNI) fill(with_tail ? L : nend * TC, L);
 #pragma unroll
-    for (int c = 0; c < COLS; ++c) p.c_last[col + c] = cur[c];
+    for (int c = 0; c < COLS; ++c) put_last<T>(p.c_last, col + c, cur[c], (p.small16 & kSmallLast) != 0);
 }
 
 // ================================================================= backward scan
@@ -843,8 +905,12 @@ __global__ void __launch_bounds__(kBlock * 4) backward_scan(const BwdParams p) {
     const bool use_tanh = GENERAL ? (p.act != 0) : ((MODE & kTanh) != 0);
     const bool has_pad = GENERAL ? (p.pad != nullptr) : ((MODE & kHasPad) != 0);
 
-    A wc1[COLS], wc2[COLS], b1[COLS], b2[COLS], m[COLS], c_init[COLS];
-    A cur[COLS];  // d loss / d state
+    ColumnOperands<T, COLS> op;
+    op.fetch(p, p.glast, (p.small16 & kSmallLast) != 0, !custom, SKIP == 1, j, col);
+    const auto &wc1 = op.w1, &wc2 = op.w2, &b1 = op.b1, &b2 = op.b2, &m = op.m;
+    auto &cur = op.start;   // d loss / d state
+    const A sx = op.sx;
+    A c_init[COLS];
     A gw1[COLS], gw2[COLS], gb1[COLS], gb2[COLS];  // sums of the current ring round
     CompensatedSumOf<A> sw1[COLS], sw2[COLS], sb1[COLS], sb2[COLS];  // sums over the whole walk
     auto fold_round = [&]() {
@@ -859,16 +925,9 @@ __global__ void __launch_bounds__(kBlock * 4) backward_scan(const BwdParams p) {
     };
 #pragma unroll
     for (int c = 0; c < COLS; ++c) {
-        wc1[c] = custom ? A(0) : static_cast<const A *>(p.wc)[j + c];
-        wc2[c] = custom ? A(0) : static_cast<const A *>(p.wc)[Dp + j + c];
-        b1[c] = as_arith<A>(p.bias)[j + c];
-        b2[c] = as_arith<A>(p.bias)[Dp + j + c];
-        m[c] = p.mask_c ? as_arith<A>(p.mask_c)[col + c] : A(1);
         c_init[c] = p.c0 ? as_arith<A>(p.c0)[col + c] : A(0);          // no initial state given: zeros
-        cur[c] = p.glast ? as_arith<A>(p.glast)[col + c] : A(0);      // no gradient of the last state given: zeros
         gw1[c] = gw2[c] = gb1[c] = gb2[c] = A(0);
     }
-    const A sx = (SKIP == 1 && p.scale_x) ? *as_arith<A>(p.scale_x) : A(1);
 
     const int64_t L = p.L;
     // The backward walk starts where the forward walk ended.
@@ -1052,19 +1111,12 @@ __global__ void __launch_bounds__(kBlock * max_waves_per_group<T>(MODE)) backwar
     const int j = ju + (int)lane;
     const bool flip = ju >= p.d;
 
-    float wc1[COLS], wc2[COLS], b1[COLS], b2[COLS], m[COLS];
-    float cur[COLS];  // d loss / d state
+    ColumnOperands<T, COLS> op;
+    op.fetch(p, p.glast, (p.small16 & kSmallLast) != 0, !CUSTOM, SKIP == 1, j, col);
+    const auto &wc1 = op.w1, &wc2 = op.w2, &b1 = op.b1, &b2 = op.b2, &m = op.m;
+    auto &cur = op.start;   // d loss / d state
+    const float sx = op.sx;
     CompensatedSum sw1[COLS], sw2[COLS], sb1[COLS], sb2[COLS];  // weight_c / bias gradient sums over the walk
-#pragma unroll
-    for (int c = 0; c < COLS; ++c) {
-        wc1[c] = CUSTOM ? 0.f : static_cast<const float *>(p.wc)[j + c];
-        wc2[c] = CUSTOM ? 0.f : static_cast<const float *>(p.wc)[Dp + j + c];
-        b1[c] = p.bias[j + c];
-        b2[c] = p.bias[Dp + j + c];
-        m[c] = p.mask_c ? p.mask_c[col + c] : 1.0f;
-        cur[c] = p.glast ? p.glast[col + c] : 0.0f;      // no gradient of the last state given: zeros
-    }
-    const float sx = (SKIP == 1 && p.scale_x) ? *p.scale_x : 1.0f;
 
     const int64_t L = p.L;
     // forward-walk step s of this column sits at element ef + s * es

@@ -102,11 +102,18 @@ forward_scan_split(const FwdParams p) {
     const bool flip = ju >= p.d;
 
     // the lane's gate: role 0 the forget gate, role 1 the reset gate (operands folded as in gate())
-    const float knw = kNegLog2e * static_cast<const float *>(p.wc)[role * Dp + j];
-    const float knb = kNegLog2e * p.bias[role * Dp + j];
-    const float m = p.mask_c ? p.mask_c[col] : 1.0f;
-    const float sa = (SKIP == 1 && role == 1 && p.scale_x) ? *p.scale_x : 1.0f;   // scale of operand A (x * scale_x)
-    float cur = p.c0 ? p.c0[col] : 0.0f;   // no initial state given: zeros
+    SmallElem<T> ew, eb, em, ex, e0;
+    const bool wc16 = (p.small16 & kSmallWeightC) != 0, bias16 = (p.small16 & kSmallBias) != 0;
+    const bool mask16 = (p.small16 & kSmallMask) != 0, scale16 = (p.small16 & kSmallScale) != 0, init16 = (p.small16 & kSmallInit) != 0;
+    ew.fetch(p.wc, role * Dp + j, wc16);
+    eb.fetch(p.bias, role * Dp + j, bias16);
+    if (p.mask_c) em.fetch(p.mask_c, col, mask16);
+    if (SKIP == 1 && p.scale_x) ex.fetch(p.scale_x, 0, scale16);
+    if (p.c0) e0.fetch(p.c0, col, init16);
+    const float knw = kNegLog2e * ew.get(wc16), knb = kNegLog2e * eb.get(bias16);
+    const float m = p.mask_c ? em.get(mask16) : 1.0f;
+    const float sa = (SKIP == 1 && role == 1 && p.scale_x) ? ex.get(scale16) : 1.0f;   // scale of operand A (x * scale_x)
+    float cur = p.c0 ? e0.get(init16) : 0.0f;   // no initial state given: zeros
 
     const int64_t L = p.L;
     const int64_t ef = (flip ? (L - 1) : 0) * p.ncols + colu;
@@ -221,7 +228,7 @@ forward_scan_split(const FwdParams p) {
         stage_to_lds(last);
         compute_chunk(nfull, tail);
     }
-    p.c_last[col] = cur;
+    put_last<T>(p.c_last, col, cur, (p.small16 & kSmallLast) != 0);
 }
 
 // ================================================================= backward scan from checkpoints, lane pairs
@@ -259,14 +266,22 @@ backward_scan_split(const BwdParams p) {
     const int j = ju + c;
     const bool flip = ju >= p.d;
 
-    const float w = static_cast<const float *>(p.wc)[role * Dp + j];   // the lane's own gate
-    const float knw = kNegLog2e * w, knb = kNegLog2e * p.bias[role * Dp + j];
-    const float m = p.mask_c ? p.mask_c[col] : 1.0f;
-    const float sx = (SKIP == 1 && p.scale_x) ? *p.scale_x : 1.0f;
+    SmallElem<T> ew, eb, em, ex, el;
+    const bool wc16 = (p.small16 & kSmallWeightC) != 0, bias16 = (p.small16 & kSmallBias) != 0;
+    const bool mask16 = (p.small16 & kSmallMask) != 0, scale16 = (p.small16 & kSmallScale) != 0, last16 = (p.small16 & kSmallLast) != 0;
+    ew.fetch(p.wc, role * Dp + j, wc16);
+    eb.fetch(p.bias, role * Dp + j, bias16);
+    if (p.mask_c) em.fetch(p.mask_c, col, mask16);
+    if (SKIP == 1 && p.scale_x) ex.fetch(p.scale_x, 0, scale16);
+    if (p.glast) el.fetch(p.glast, col, last16);
+    const float w = ew.get(wc16);   // the lane's own gate
+    const float knw = kNegLog2e * w, knb = kNegLog2e * eb.get(bias16);
+    const float m = p.mask_c ? em.get(mask16) : 1.0f;
+    const float sx = (SKIP == 1 && p.scale_x) ? ex.get(scale16) : 1.0f;
     // scale of operand A: role 1's skip operand is x * scale_x, U[..., 3], or nothing (times zero)
     const float sa = role ? (SKIP == 0 ? 0.0f : sx) : 1.0f;
     const float oa_a = role ? m * sx : 1.0f, oa_b = role ? sx : 1.0f;   // see out_a below (sx is 1 unless the skip term is x)
-    float cur = p.glast ? p.glast[col] : 0.0f;   // d loss / d state (meaningful in role 0); not given: zeros
+    float cur = p.glast ? el.get(last16) : 0.0f;   // d loss / d state (meaningful in role 0); not given: zeros
     CompensatedSum sw, sb;      // the lane's gate: sums of its weight_c and bias gradients
 
     const int64_t L = p.L;

@@ -35,6 +35,7 @@ from torch.autograd import Function
 
 from . import _lib
 
+_NARROW = (torch.float16, torch.bfloat16)
 _DTYPES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float64: _lib.F64}
 
 
@@ -152,7 +153,18 @@ def _problem(u: Tensor, x: Tensor, weight_c: Tensor, d_out: int, bidirectional: 
                            x.dtype == torch.float32, bool(state_kept))
 
 
-def _prepare_inputs(pb: _Problem, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad):
+def _prepare_inputs(pb: _Problem, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad, narrow_small=False):
+    """The tensors as the kernels read them, and which small ones stay in the 16-bit stream type
+    (`narrow_small`: those that have it are handed over as they are; otherwise all become float)."""
+    small16 = 0
+
+    def small(t, bit):
+        nonlocal small16
+        if t is not None and narrow_small and t.dtype == pb.dtype and pb.dtype in _NARROW:
+            small16 |= bit
+            return t.contiguous()
+        return _small(t, pb.small_dtype)
+
     # (16-bit k=4 groups of two columns move as one 16-byte vector in the checkpointed kernels)
     u_ = _aligned(u, 16)
     x_ = None
@@ -165,19 +177,19 @@ def _prepare_inputs(pb: _Problem, u, x, weight_c, bias, init, scale_x, mask_c, m
         if wc_.numel() != pb.length * pb.batch * pb.Dp * 2:
             raise ValueError("per-step weight_c must have length*batch*output_size*2 elements")
     else:
-        wc_ = _small(weight_c, pb.small_dtype)
+        wc_ = small(weight_c, _lib.SMALL_WEIGHT_C)
         if wc_.numel() != 2 * pb.Dp:
             raise ValueError("weight_c must have 2*output_size elements")
-    bias_ = _small(bias, pb.small_dtype)
-    init_ = _small(init, pb.small_dtype)         # None: the kernels start from zeros
+    bias_ = small(bias, _lib.SMALL_BIAS)
+    init_ = small(init, _lib.SMALL_INIT)         # None: the kernels start from zeros
     if bias_.numel() != 2 * pb.Dp or (init_ is not None and init_.numel() != pb.batch * pb.Dp):
         raise ValueError("bias must have 2*output_size and init batch*output_size elements")
-    mask_c_ = _small(mask_c, pb.small_dtype)
+    mask_c_ = small(mask_c, _lib.SMALL_MASK)
     if mask_c_ is not None and mask_c_.numel() != pb.batch * pb.Dp:
         raise ValueError("mask_c must have batch*output_size elements")
     scale_ = None
     if scale_x is not None and pb.skip_type == 1:
-        scale_ = _small(scale_x.reshape(-1)[:1], pb.small_dtype)
+        scale_ = small(scale_x if scale_x.numel() == 1 else scale_x.reshape(-1)[:1], _lib.SMALL_SCALE)
     pad_ = None
     if mask_pad is not None:
         pad_ = mask_pad.contiguous()
@@ -185,10 +197,10 @@ def _prepare_inputs(pb: _Problem, u, x, weight_c, bias, init, scale_x, mask_c, m
         assert pad_.size(0) == pb.length
         assert pad_.size(1) == pb.batch
         pad_ = (pad_ if pad_.dtype == torch.bool else pad_.bool()).view(torch.uint8)
-    return u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_
+    return (u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_), small16
 
 
-def _run_forward(pb, u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_, keep_c: bool):
+def _run_forward(pb, u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_, keep_c: bool, small16: int = 0):
     dev = u_.device
     lib = _lib.load()
     h = torch.empty(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
@@ -197,12 +209,15 @@ def _run_forward(pb, u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_, keep_c: b
         c = torch.empty(pb.state_rows, pb.batch, pb.Dp, dtype=torch.float32, device=dev)
     elif keep_c:
         c = torch.empty(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
-    c_last = torch.empty(pb.batch, pb.Dp, dtype=pb.small_dtype, device=dev)
+    # (the last state comes back in U's type: 16-bit streams have the kernel round it)
+    if pb.dtype in _NARROW:
+        small16 |= _lib.SMALL_LAST
+    c_last = torch.empty(pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
     with _on_device(dev) as stream:
-        rc = lib.sru_amd_forward(ctypes.byref(pb.shape), _ptr(u_), _ptr(x_), _ptr(wc_), _ptr(bias_),
-                                 _ptr(init_), _ptr(mask_c_), _ptr(pad_), _ptr(scale_), _ptr(h),
-                                 _ptr(c), _ptr(c_last), stream)
-    _lib.check(rc, "sru_amd_forward")
+        rc = lib.sru_amd_forward_small(ctypes.byref(pb.shape), small16, _ptr(u_), _ptr(x_), _ptr(wc_),
+                                       _ptr(bias_), _ptr(init_), _ptr(mask_c_), _ptr(pad_), _ptr(scale_), _ptr(h),
+                                       _ptr(c), _ptr(c_last), stream)
+    _lib.check(rc, "sru_amd_forward_small")
     return h, c, c_last
 
 
@@ -227,8 +242,8 @@ def elementwise_recurrence_forward(
     if u.dtype != _kernel_dtype(u):
         u = u.to(_kernel_dtype(u))
     pb = _problem(u, x, weight_c, d_out, bidirectional, has_skip_term, activation_type, state_kept=keep_c)
-    prepared = _prepare_inputs(pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
-    h, c, c_last = _run_forward(pb, *prepared, keep_c=keep_c)
+    prepared, small16 = _prepare_inputs(pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad, narrow_small=True)
+    h, c, c_last = _run_forward(pb, *prepared, keep_c=keep_c, small16=small16)
     last_hidden = c_last if out_dtype == c_last.dtype else c_last.to(out_dtype)
     if out_dtype != pb.dtype:
         h = h.to(out_dtype)
@@ -257,7 +272,7 @@ class ElementwiseRecurrence(Function):
             u = u.to(_kernel_dtype(u))
         pb = _problem(u, x, weight_c, d_out, bidirectional, has_skip_term, activation_type,
                       checkpoint_state=True)
-        prepared = _prepare_inputs(pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
+        prepared, _ = _prepare_inputs(pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
         h, c, c_last = _run_forward(pb, *prepared, keep_c=True)
         ctx.problem = pb
         ctx.in_dtypes = (u_dtype, x.dtype, weight_c.dtype, bias.dtype, None if init is None else init.dtype)
@@ -283,7 +298,9 @@ class ElementwiseRecurrence(Function):
             gh = torch.zeros(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
         else:
             gh = _aligned(grad_h if grad_h.dtype == pb.dtype else grad_h.to(pb.dtype), 4)
-        gl = _small(grad_last, pb.small_dtype)   # None: the kernels start from a zero state gradient
+        # (None: the kernels start from a zero state gradient; 16 bits are read as they are)
+        narrow_last = grad_last is not None and grad_last.dtype == pb.dtype and pb.dtype in _NARROW
+        gl = grad_last.contiguous() if narrow_last else _small(grad_last, pb.small_dtype)
         grad_u = torch.empty_like(u_)
         grad_x = torch.empty_like(x_) if pb.skip_type == 1 else None
         grad_wc = torch.empty_like(wc_) if pb.is_custom else \
@@ -294,12 +311,12 @@ class ElementwiseRecurrence(Function):
         ws_bytes = pb.workspace_bytes
         workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=dev)
         with _on_device(dev) as stream:
-            rc = _lib.load().sru_amd_backward(
-                ctypes.byref(pb.shape), _ptr(u_), _ptr(x_), _ptr(wc_), _ptr(bias_), _ptr(init_),
+            rc = _lib.load().sru_amd_backward_small(
+                ctypes.byref(pb.shape), _lib.SMALL_LAST if narrow_last else 0, _ptr(u_), _ptr(x_), _ptr(wc_), _ptr(bias_), _ptr(init_),
                 _ptr(mask_c_), _ptr(pad_), _ptr(scale_), _ptr(c), _ptr(gh), _ptr(gl),
                 _ptr(grad_u), _ptr(grad_x), _ptr(grad_wc), _ptr(grad_bias), _ptr(grad_init),
                 _ptr(workspace), ctypes.c_size_t(ws_bytes), stream)
-        _lib.check(rc, "sru_amd_backward")
+        _lib.check(rc, "sru_amd_backward_small")
         u_dt, x_dt, wc_dt, bias_dt, init_dt = ctx.in_dtypes
         u_sh, x_sh, wc_sh, bias_sh, init_sh = ctx.in_shapes
         grad_u = grad_u.view(u_sh).to(u_dt)
