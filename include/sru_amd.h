@@ -230,6 +230,30 @@ int sru_amd_backward_static(const sru_amd_shape *shape,
                             void *grad_u, void *grad_x, void *grad_wc, void *grad_bias,
                             void *grad_init, void *stream);
 
+/* A whole layer without gradients: U = x weight, or (x weight_proj) weight, and the recurrence
+ * behind it, where kernels exist that do both (sru/modules.py:252-304: compute_U, then
+ * apply_recurrence). The reference runs two or three library calls here.
+ *
+ * sru_amd_layer_route says whether they exist for a problem: 0 = no (project with a library and call
+ * sru_amd_forward), SRU_AMD_LAYER_STEP = one time step of up to 64 rows. `shape` is that of the
+ * recurrence (16-bit streams, is_custom 0); in_features and n_proj (0: no projection) are the inner
+ * sizes, which together with the width have to be multiples of 32. */
+#define SRU_AMD_LAYER_STEP 1
+int sru_amd_layer_route(const sru_amd_shape *shape, int64_t in_features, int64_t n_proj);
+
+/* The layer itself, on a route that sru_amd_layer_route gave (BAD_SHAPE otherwise).
+ *   x           (L, B, in_features) in shape->dtype
+ *   skip        (L, B, D') in shape->dtype, what the skip term reads; required iff skip_type == 1
+ *   weight_proj (in_features, n_proj); NULL iff n_proj is 0
+ *   weight      (n_proj or in_features, D' * k), both in shape->dtype, row-major
+ *   projected   (L, B, n_proj) scratch; NULL iff n_proj is 0
+ *   the rest    as in sru_amd_forward_small; every stream and weight 16-byte aligned */
+int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t in_features, int64_t n_proj,
+                          const void *x, const void *skip, const void *weight_proj, const void *weight,
+                          const void *weight_c, const void *bias, const void *c_init,
+                          const uint8_t *mask_pad, const void *scale_x, void *projected,
+                          void *h, void *c_last, void *stream);
+
 /* Layer normalisation of the rows of a (rows, cols) matrix, the operation the reference applies to a
  * layer's input before the projection or to its output after the recurrence with
  * torch.nn.LayerNorm (sru/modules.py:155-162 created, :250-253 and :278-279 applied):

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include "sru_launch.h"
+#include "sru_layer.h"
 #include "sru_reduce.h"
 
 #include <mutex>
@@ -291,6 +292,47 @@ int sru_amd_backward_static(const sru_amd_shape *shape, const void *u, const voi
     if (!partial) return SRU_AMD_ERR_LAUNCH;
     return backward_core(shape, u, x, weight_c, bias, c_init, mask_c, mask_pad, scale_x, c, grad_h, grad_last,
                          grad_u, grad_x, grad_wc, grad_bias, grad_init, partial, stream);
+}
+
+int sru_amd_layer_route(const sru_amd_shape *shape, int64_t in_features, int64_t n_proj) {
+    if (check_shape(shape) != SRU_AMD_OK || in_features < 1 || n_proj < 0) return 0;
+    const sru_amd_shape &s = *shape;
+    // (16-bit streams throughout; four streams per column only with the skip term among them)
+    if (elem_size(s.dtype) != 2 || s.is_custom || x_is_float_beside_16bit(s) || (s.k == 4 && s.skip_type != 2)) return 0;
+    if (s.length == 1 && step_sizes_ok(s.batch, s.hidden * s.dirs, in_features, n_proj)) return SRU_AMD_LAYER_STEP;
+    return 0;
+}
+
+int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t in_features, int64_t n_proj,
+                          const void *x, const void *skip, const void *weight_proj, const void *weight,
+                          const void *weight_c, const void *bias, const void *c_init,
+                          const uint8_t *mask_pad, const void *scale_x, void *projected,
+                          void *h, void *c_last, void *stream) {
+    if (const int rc = check_shape(shape)) return rc;
+    const sru_amd_shape &s = *shape;
+    const int route = sru_amd_layer_route(shape, in_features, n_proj);
+    if (!route) return SRU_AMD_ERR_BAD_SHAPE;
+    if (const int rc = check_small(s, small16)) return rc;
+    if (!x || !weight || !weight_c || !bias || !h || !c_last || (s.skip_type == 1 && !skip) ||
+        (n_proj > 0 && (!weight_proj || !projected)))
+        return SRU_AMD_ERR_NULL_POINTER;
+    for (const void *q : {x, s.skip_type == 1 ? skip : nullptr, weight_proj, weight, static_cast<const void *>(projected), static_cast<const void *>(h)})
+        if (q && !aligned(q, 16)) return SRU_AMD_ERR_MISALIGNED;
+    auto small_align = [&](uint32_t bit) { return (small16 & bit) ? (size_t)2 : (size_t)4; };
+    if (!aligned(weight_c, small_align(SRU_AMD_SMALL_WEIGHT_C)) || !aligned(bias, small_align(SRU_AMD_SMALL_BIAS)) ||
+        (c_init && !aligned(c_init, small_align(SRU_AMD_SMALL_INIT))) || !aligned(c_last, small_align(SRU_AMD_SMALL_LAST)) ||
+        (scale_x && !aligned(scale_x, small_align(SRU_AMD_SMALL_SCALE))))
+        return SRU_AMD_ERR_MISALIGNED;
+
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    StepParams p{}, proj{};
+    p.x = n_proj ? projected : x; p.weight = weight; p.wc = weight_c; p.bias = bias; p.c0 = c_init; p.scale_x = scale_x;
+    p.skip = skip; p.pad = mask_pad; p.h = h; p.c_last = c_last; p.Dp = s.hidden * s.dirs; p.cols = p.Dp * s.k;
+    p.rows = (int32_t)s.batch; p.inner = (int32_t)(n_proj ? n_proj : in_features); p.act = s.activation_type; p.small16 = small16;
+    proj.x = x; proj.weight = weight_proj; proj.h = projected; proj.cols = n_proj;
+    proj.rows = p.rows; proj.inner = (int32_t)in_features;
+    const hipError_t err = launch_layer_step(p, n_proj ? &proj : nullptr, s.dtype == SRU_AMD_F16, s.k, s.skip_type, st);
+    return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
 }
 
 }  // extern "C"

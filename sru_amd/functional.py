@@ -254,6 +254,61 @@ def elementwise_recurrence_forward(
     return h, last_hidden, c
 
 
+@functools.lru_cache(maxsize=256)
+def _layer_plan(dtype, x_dim, length, batch, in_features, n_proj, d_out, dirs, k, has_skip_term, activation_type):
+    """Problem and route of a whole layer; route 0: no kernel for it."""
+    D = d_out * dirs
+    pb = _problem_cached(dtype, x_dim, length, batch, length * batch * D * k, D * k, 0, d_out, dirs == 2, has_skip_term,
+                         activation_type, False, False, False)
+    return pb, _lib.load().sru_amd_layer_route(ctypes.byref(pb.shape), in_features, n_proj)
+
+
+def layer_forward(x: Tensor, residual: Tensor, weight_proj: Optional[Tensor], weight: Tensor, weight_c: Tensor,
+                  bias: Tensor, init: Optional[Tensor], activation_type: int, d_out: int, bidirectional: bool,
+                  has_skip_term: bool, scale_x: Optional[Tensor] = None,
+                  mask_pad: Optional[Tensor] = None) -> Optional[Tuple[Tensor, Tensor]]:
+    """A layer's dense products and its recurrence without gradients, in kernels that do both: (h,
+    last_hidden), or None where there are none for the problem (dtypes, sizes, alignment) and the
+    caller has to project first. `residual` is what the skip term reads, `x` what is projected."""
+    dtype = x.dtype
+    dirs = 2 if bidirectional else 1
+    k = weight.size(-1) // (d_out * dirs)
+    three = x.dim() == 3
+    n_proj = 0 if weight_proj is None else weight_proj.size(1)
+    if dtype not in _NARROW or not x.is_cuda:
+        return None
+    inner = x.size(-1)
+    for w in (weight_proj, weight):
+        if w is not None:
+            if w.dtype != dtype or w.device != x.device or w.dim() != 2 or w.size(0) != inner:
+                return None
+            inner = w.size(1)
+    if inner != d_out * dirs * k:
+        return None
+    pb, route = _layer_plan(dtype, x.dim(), x.size(0) if three else 1, x.size(-2), x.size(-1), n_proj, d_out, dirs, k,
+                            bool(has_skip_term), int(activation_type))
+    if not route or (pb.skip_type == 1 and residual.dtype != dtype):
+        return None
+    for w in (weight_proj, weight):
+        if w is not None and not (w.is_contiguous() and w.data_ptr() % 16 == 0):
+            return None
+    x_ = _aligned(x, 16)
+    (_, _, wc_, bias_, init_, scale_, _, pad_), small16 = _prepare_inputs(
+        pb, x_, residual, weight_c, bias, init, scale_x, None, mask_pad, narrow_small=True)
+    skip_ = None if pb.skip_type != 1 else x_ if residual is x else _aligned(residual, 16)
+    dev = x.device
+    projected = torch.empty(pb.length * pb.batch, n_proj, dtype=dtype, device=dev) if n_proj else None
+    h = torch.empty((pb.length, pb.batch, pb.Dp) if three else (pb.batch, pb.Dp), dtype=dtype, device=dev)
+    c_last = torch.empty(pb.batch, pb.Dp, dtype=dtype, device=dev)
+    with _on_device(dev) as stream:
+        rc = _lib.load().sru_amd_layer_forward(
+            ctypes.byref(pb.shape), small16 | _lib.SMALL_LAST, x.size(-1), n_proj, _ptr(x_), _ptr(skip_), _ptr(weight_proj),
+            _ptr(weight), _ptr(wc_), _ptr(bias_), _ptr(init_), _ptr(pad_), _ptr(scale_), _ptr(projected), _ptr(h),
+            _ptr(c_last), stream)
+    _lib.check(rc, "sru_amd_layer_forward")
+    return h, c_last
+
+
 class ElementwiseRecurrence(Function):
     """Drop-in for sru/cuda_functional.py:156-261.
 

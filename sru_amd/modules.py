@@ -18,6 +18,7 @@ import torch.nn as nn
 from torch import Tensor
 from torch.nn.utils.rnn import PackedSequence, pad_packed_sequence, pack_padded_sequence
 
+from .functional import layer_forward
 from .norm import layer_norm as fused_layer_norm, supported as fused_layer_norm_supported
 from .ops import elementwise_recurrence_gpu
 
@@ -140,11 +141,32 @@ class SRUCell(nn.Module):
             mask_c = self._dropout_mask((batch, self.output_size), self.dropout)
         scale_val = self.scale_x if self.rescale else None
 
+        if mask_c is None and self._whole_layer(input, residual):
+            done = layer_forward(input, residual, self.weight_proj, self.weight, self.weight_c, self.bias, c0,
+                                 self.activation_type, self.hidden_size, self.bidirectional, self.has_skip_term,
+                                 scale_val, mask_pad)
+            if done is not None:
+                h, c = done
+                if self.layer_norm is not None and self.normalize_after:
+                    h = self._normalise(h, feeds_projection=False)
+                return h, c
+
         U, V = self.compute_UV(input, c0, mask_pad)
         h, c = self.apply_recurrence(U, V, residual, c0, scale_val, mask_c, mask_pad)
         if self.layer_norm is not None and self.normalize_after:
             h = self._normalise(h, feeds_projection=False)
         return h, c
+
+    def _whole_layer(self, input: Tensor, residual: Tensor) -> bool:
+        """Whether `layer_forward` may stand for compute_UV and apply_recurrence: nothing is
+        differentiated or autocast, the layer projects with its own weights, neither step is
+        overridden, and the tensors are plain ones that nothing records."""
+        cls = type(self)
+        return (not torch.is_grad_enabled() and self.custom_m is None and input.dtype in (torch.float16, torch.bfloat16)
+                and getattr(self, "native_16bit", True) and cls.compute_U is SRUCell.compute_U and cls.compute_UV is SRUCell.compute_UV
+                and cls.apply_recurrence is SRUCell.apply_recurrence and type(input) is Tensor and type(residual) is Tensor
+                and not torch.is_autocast_enabled("cuda") and not torch.jit.is_tracing()
+                and input.size(-1) == self.input_size)
 
     def _normalise(self, x: Tensor, feeds_projection: bool) -> Tensor:
         """self.layer_norm(x) (sru/modules.py:250-253, :278-279) through the layer-norm kernels of
