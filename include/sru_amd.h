@@ -235,10 +235,13 @@ int sru_amd_backward_static(const sru_amd_shape *shape,
  * apply_recurrence). The reference runs two or three library calls here.
  *
  * sru_amd_layer_route says whether they exist for a problem: 0 = no (project with a library and call
- * sru_amd_forward), SRU_AMD_LAYER_STEP = one time step of up to 64 rows. `shape` is that of the
+ * sru_amd_forward), SRU_AMD_LAYER_STEP = one time step of up to 64 rows, SRU_AMD_LAYER_ROWS = long
+ * sequences of many columns (n_proj 0; an input that was projected elsewhere counts as x). `shape` is that of the
  * recurrence (16-bit streams, is_custom 0); in_features and n_proj (0: no projection) are the inner
- * sizes, which together with the width have to be multiples of 32. */
+ * sizes, multiples of 32; a step wants the width one as well, long sequences a hidden size that is a
+ * multiple of 8. */
 #define SRU_AMD_LAYER_STEP 1
+#define SRU_AMD_LAYER_ROWS 2
 int sru_amd_layer_route(const sru_amd_shape *shape, int64_t in_features, int64_t n_proj);
 
 /* The layer itself, on a route that sru_amd_layer_route gave (BAD_SHAPE otherwise).

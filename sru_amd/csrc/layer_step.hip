@@ -19,8 +19,8 @@
 
 #include <hip/hip_runtime.h>
 
-#include "sru_scan.h"
 #include "sru_layer.h"
+#include "sru_mfma.h"
 
 namespace sru_amd {
 namespace {
@@ -28,22 +28,7 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kBlock;
 constexpr int kTileRows = 16;
-constexpr int kStepK = 32;      // inner indices per MFMA
 constexpr int kPitch = 17;      // floats per column of a partial tile in LDS: 16 rows + 1, every bank twice per access
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
-
-template <typename T> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c);
-template <> __device__ __forceinline__ f32x4 mfma<bf16_bits>(u32x4 a, u32x4 b, f32x4 c) {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-}
-template <> __device__ __forceinline__ f32x4 mfma<half_bits>(u32x4 a, u32x4 b, f32x4 c) {
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
-}
 
 // STREAMS: 0 stores the product, 3 / 4 run the recurrence step on it.
 // SKIP as in the scan kernels. DEPTH: MFMA steps whose loads are in flight together.

@@ -300,6 +300,9 @@ int sru_amd_layer_route(const sru_amd_shape *shape, int64_t in_features, int64_t
     // (16-bit streams throughout; four streams per column only with the skip term among them)
     if (elem_size(s.dtype) != 2 || s.is_custom || x_is_float_beside_16bit(s) || (s.k == 4 && s.skip_type != 2)) return 0;
     if (s.length == 1 && step_sizes_ok(s.batch, s.hidden * s.dirs, in_features, n_proj)) return SRU_AMD_LAYER_STEP;
+    // (the long-sequence kernel is built for the layers that a stack has: a skip term, the identity activation)
+    if (n_proj == 0 && s.skip_type != 0 && s.activation_type == 0 && rows_sizes_ok(s.length, s.batch, s.hidden, s.dirs, in_features, s.k))
+        return SRU_AMD_LAYER_ROWS;
     return 0;
 }
 
@@ -325,6 +328,14 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
         return SRU_AMD_ERR_MISALIGNED;
 
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (route == SRU_AMD_LAYER_ROWS) {
+        RowsParams p{};
+        p.x = x; p.weight = weight; p.wc = weight_c; p.bias = bias; p.c0 = c_init; p.scale_x = scale_x; p.skip = skip;
+        p.pad = mask_pad; p.h = h; p.c_last = c_last; p.B = s.batch; p.Dp = s.hidden * s.dirs; p.L = (int32_t)s.length;
+        p.d = (int32_t)s.hidden; p.dirs = s.dirs; p.inner = (int32_t)in_features; p.groups_per_dir = (p.d + 63) / 64;
+        p.small16 = small16;
+        return launch_layer_rows(p, s.dtype == SRU_AMD_F16, s.k, st) == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
+    }
     StepParams p{}, proj{};
     p.x = n_proj ? projected : x; p.weight = weight; p.wc = weight_c; p.bias = bias; p.c0 = c_init; p.scale_x = scale_x;
     p.skip = skip; p.pad = mask_pad; p.h = h; p.c_last = c_last; p.Dp = s.hidden * s.dirs; p.cols = p.Dp * s.k;

@@ -285,13 +285,21 @@ def layer_forward(x: Tensor, residual: Tensor, weight_proj: Optional[Tensor], we
             inner = w.size(1)
     if inner != d_out * dirs * k:
         return None
-    pb, route = _layer_plan(dtype, x.dim(), x.size(0) if three else 1, x.size(-2), x.size(-1), n_proj, d_out, dirs, k,
-                            bool(has_skip_term), int(activation_type))
+    sizes = (d_out, dirs, k, bool(has_skip_term), int(activation_type))
+    pb, route = _layer_plan(dtype, x.dim(), x.size(0) if three else 1, x.size(-2), x.size(-1), n_proj, *sizes)
+    if not route and n_proj:   # the projection by the library, the rest of the layer in one kernel
+        pb, route = _layer_plan(dtype, x.dim(), x.size(0) if three else 1, x.size(-2), n_proj, 0, *sizes)
+    project_first = bool(n_proj) and bool(route) and route != _lib.LAYER_STEP
     if not route or (pb.skip_type == 1 and residual.dtype != dtype):
         return None
     for w in (weight_proj, weight):
         if w is not None and not (w.is_contiguous() and w.data_ptr() % 16 == 0):
             return None
+    if project_first:
+        if residual is x:
+            residual = x = x.contiguous()
+        x = x.reshape(-1, x.size(-1)).mm(weight_proj).view(*x.shape[:-1], n_proj)
+        weight_proj, n_proj = None, 0
     x_ = _aligned(x, 16)
     (_, _, wc_, bias_, init_, scale_, _, pad_), small16 = _prepare_inputs(
         pb, x_, residual, weight_c, bias, init, scale_x, None, mask_pad, narrow_small=True)

@@ -87,6 +87,39 @@ def test_one_step(inp, d, kw, batch, dtype):
     check(cell, x, c0.float(), pad)
 
 
+# (input, hidden, batch, length): partial groups of batch elements and of cells, an inner size at, between
+# and above the register classes, a last tile of every remainder; up to 65536 columns tiles have four
+# steps, above two
+LONG = [(64, 64, 385, 257, dict(bidirectional=True)), (128, 64, 386, 258, dict(bidirectional=True)),
+        (160, 72, 683, 259, {}), (256, 256, 131, 257, dict(bidirectional=True)), (512, 256, 128, 256, dict(bidirectional=True)),
+        (512, 256, 133, 258, dict(bidirectional=True)), (288, 144, 171, 260, dict(bidirectional=True)),
+        (128, 128, 384, 256, dict(n_proj=32))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("inp,d,batch,length,kw", LONG)
+def test_long_sequences(inp, d, batch, length, kw, dtype):
+    cell = make(inp, d, dtype, **kw)
+    x = torch.randn(length, batch, inp, device="cuda").to(dtype)
+    c0 = torch.randn(batch, cell.output_size, device="cuda").to(dtype)
+    lens = torch.randint(1, length + 1, (batch,), device="cuda")
+    pad = torch.arange(length, device="cuda")[:, None] >= lens[None, :]
+    check(cell, x, c0, None)
+    check(cell, x, None, pad)
+    check(cell, x, c0.float(), pad)
+
+
+def test_long_sequences_outside_the_route():
+    big = dict(bidirectional=True)
+    for inp, d, batch, length, kw in [(64, 64, 383, 256, big), (64, 64, 384, 255, big), (64, 68, 1024, 256, {}), (72, 64, 1024, 256, {}),
+                                      (288, 64, 1024, 256, {}), (256, 256, 256, 256, dict(use_tanh=True)),
+                                      (256, 256, 256, 256, dict(has_skip_term=False))]:
+        k = 3 if not kw.get("has_skip_term", True) or inp == d * (1 + kw.get("bidirectional", False)) else 4
+        plan = functional._layer_plan(torch.float16, 3, length, batch, inp, 0, d, 2 if "bidirectional" in kw else 1, k,
+                                      kw.get("has_skip_term", True), int(kw.get("use_tanh", False)))
+        assert plan[1] == 0
+
+
 def test_one_step_outside_the_route():
     cell = make(64, 64, torch.bfloat16)
     check(cell, torch.randn(1, 65, 64, device="cuda").bfloat16(), None, None, route_expected=False)   # too many rows
