@@ -90,6 +90,22 @@ def load():
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host code (csrc/host.cpp): calls in the plain case, from torch tensors to the C ABI."""
+    global _host
+    if _host is None:
+        load()      # the library it calls, and the error where that is missing
+        try:
+            from . import _host as module
+        except ImportError as exc:
+            raise LibraryError(f"sru_amd/_host.so cannot be loaded ({exc}): build it with `python -m sru_amd.build`") from exc
+        _host = module
+    return _host
+
+
 def status_string(code):
     return load().sru_amd_status_string(code).decode()
 

@@ -13,6 +13,7 @@ SOURCES = [os.path.join(HERE, "csrc", n)
                      "layer_rows.hip")]
 OUTPUT = os.path.join(HERE, "libsru_amd.so")
 OBJ_DIR = os.path.join(HERE, "csrc", "build")
+HOST_MODULE = os.path.join(HERE, "_host.so")
 SERVE_FORWARD = os.path.join(HERE, "serve_forward")
 
 HIPCC_FLAGS = [
@@ -93,7 +94,35 @@ def build(verbose=True, output=OUTPUT, defines=(), max_scratch_bytes=MAX_SCRATCH
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", output], verbose)
     if output == OUTPUT:
         build_serve_forward(verbose)
+        build_host(verbose)
     return output
+
+
+def _host_compile(cmd, verbose):
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode:
+        print(proc.stdout, flush=True)
+        raise RuntimeError("host compiler failed: " + " ".join(cmd))
+
+
+def build_host(verbose=True):
+    """Compiles csrc/host.cpp, the native host side between torch tensors and the C ABI, as a Python
+    extension module linked to the library just built."""
+    import sysconfig
+
+    import torch
+    torch_dir = os.path.dirname(os.path.abspath(torch.__file__))
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    _host_compile([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                   "-I" + os.path.join(torch_dir, "include"), "-I" + os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+                   "-I" + os.path.join(rocm, "include"), "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(ROOT, "include"),
+                   os.path.join(HERE, "csrc", "host.cpp"), "-L" + HERE, "-lsru_amd", "-L" + os.path.join(torch_dir, "lib"),
+                   "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN",
+                   "-o", HOST_MODULE], verbose)
+    return HOST_MODULE
 
 
 def build_serve_forward(verbose=True):
@@ -105,12 +134,7 @@ def build_serve_forward(verbose=True):
            os.path.join(HERE, "csrc", "serve_forward.cpp"), "-L" + HERE, "-lsru_amd",
            "-L" + os.path.join(rocm, "lib"), "-lamdhip64", "-Wl,-rpath,$ORIGIN",
            "-Wl,-rpath," + os.path.join(rocm, "lib"), "-o", SERVE_FORWARD]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if proc.returncode:
-        print(proc.stdout, flush=True)
-        raise RuntimeError("host compiler failed: " + " ".join(cmd))
+    _host_compile(cmd, verbose)
     return SERVE_FORWARD
 
 

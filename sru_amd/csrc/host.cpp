@@ -1,0 +1,275 @@
+// The host side of a call in native code: what functional.py does between torch tensors and the C ABI,
+// for the plain case only (a contiguous, aligned, already converted set of tensors on one device, the
+// state kept as checkpoints or not at all). Every function answers None where anything is out of the
+// ordinary, before it has launched anything, and functional.py then goes its general way, which also
+// says what is wrong with a call. No state is kept between calls.
+//
+// Why: a forward and backward pass of the recurrence cost the host 145-175 us in Python, more than the
+// kernels of most sizes take. 128 x 32 x 1024 f32 with padding, 53 us of kernels: 159 us a pass then,
+// 101 us through here (the rest is torch's own autograd); one token through ten layers of 2048: 221
+// and 145 us.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "sru_amd.h"
+
+namespace {
+
+// An argument that has to be a tensor or None.
+struct Arg {
+    const at::Tensor *t = nullptr;   // null: None
+    explicit operator bool() const { return t != nullptr; }
+    const at::Tensor *operator->() const { return t; }
+    void *ptr() const { return t ? t->data_ptr() : nullptr; }
+};
+bool read(PyObject *o, Arg &a) {
+    if (o == Py_None) return true;
+    if (!THPVariable_Check(o)) return false;
+    a.t = &THPVariable_Unpack(o);
+    return a->defined() && a->layout() == at::kStrided;
+}
+bool read(PyObject *o, int64_t &v) {
+    if (!PyLong_Check(o)) return false;
+    v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+
+bool aligned(const at::Tensor &t, uintptr_t n) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % n == 0; }
+bool narrow(at::ScalarType t) { return t == at::kHalf || t == at::kBFloat16; }
+
+// contiguous, on the device of the call, so many elements, so aligned
+bool plain(const at::Tensor &t, const c10::Device &device, int64_t numel, uintptr_t alignment) {
+    return t.device() == device && t.numel() == numel && t.is_contiguous() && !t.is_conj() && !t.is_neg() && aligned(t, alignment);
+}
+
+// A small tensor as the kernels read it: float, or (where `may_narrow`) in the 16-bit stream type.
+bool small(const Arg &a, const c10::Device &device, int64_t numel, at::ScalarType stream, bool may_narrow, uint32_t bit, uint32_t &small16) {
+    if (!a) return true;
+    if (may_narrow && narrow(stream) && a->scalar_type() == stream) {
+        small16 |= bit;
+        return plain(*a.t, device, numel, 2);
+    }
+    return a->scalar_type() == at::kFloat && plain(*a.t, device, numel, 8);
+}
+
+struct Call {
+    Arg u, x, weight_c, bias, init, scale, mask_c, pad;
+    int64_t act = 0, d = 0, length = 0, batch = 0;
+    bool bidirectional = false, has_skip = false;
+    sru_amd_shape shape{};
+    uint32_t small16 = 0;
+    int64_t width() const { return shape.hidden * shape.dirs; }
+    const c10::Device device() const { return u->device(); }
+};
+
+bool dtype_code(at::ScalarType t, int32_t &code) {
+    code = t == at::kFloat ? SRU_AMD_F32 : t == at::kHalf ? SRU_AMD_F16 : SRU_AMD_BF16;
+    return t == at::kFloat || narrow(t);
+}
+
+bool plain_pad(const Arg &pad, const c10::Device &device, int64_t length, int64_t batch) {
+    return !pad || (pad->scalar_type() == at::kBool && pad->dim() == 2 && pad->size(0) == length && pad->size(1) == batch &&
+                    plain(*pad.t, device, length * batch, 1));
+}
+
+// Sizes and flags as _Problem derives them, and the checks of _prepare_inputs; length and batch are set.
+bool prepare(Call &c, bool checkpointed, bool may_narrow) {
+    if (!c.u || !c.weight_c || !c.bias || !c.u->is_cuda() || c.u->dim() < 1 || c.length < 1 || c.batch < 1 || c.d < 1) return false;
+    const at::ScalarType type = c.u->scalar_type();
+    const c10::Device device = c.u->device();
+    sru_amd_shape &s = c.shape;
+    if (!dtype_code(type, s.dtype) || c.weight_c->dim() != 1 || (c.act != 0 && c.act != 1)) return false;
+    s.length = c.length;
+    s.batch = c.batch;
+    s.hidden = c.d;
+    s.dirs = c.bidirectional ? 2 : 1;
+    const int64_t width = c.d * s.dirs, streams = c.u->size(-1) / width;
+    if ((streams != 3 && streams != 4) || c.u->size(-1) != streams * width) return false;
+    s.k = (int32_t)streams;
+    s.activation_type = (int32_t)c.act;
+    s.skip_type = !c.has_skip ? 0 : s.k == 3 ? 1 : 2;
+    s.is_custom = 0;
+    const int64_t cells = c.length * c.batch * width;
+    if (checkpointed && ((type != at::kFloat && c.d % 2 != 0) || (s.skip_type == 0 && s.k == 4))) return false;
+    s.state_interval = checkpointed ? SRU_AMD_STATE_INTERVAL : 1;
+    s.x_dtype = SRU_AMD_X_AS_STREAMS;
+    if (!plain(*c.u.t, device, cells * s.k, 16)) return false;
+    if (s.skip_type == 1) {
+        if (!c.x || !plain(*c.x.t, device, cells, 4)) return false;
+        if (c.x->scalar_type() != type) {
+            if (c.x->scalar_type() != at::kFloat || c.act != 0 || c.d % 2 != 0) return false;
+            s.x_dtype = SRU_AMD_X_F32;
+        }
+    } else {
+        c.x = Arg{};
+        c.scale = Arg{};
+    }
+    return small(c.weight_c, device, 2 * width, type, may_narrow, SRU_AMD_SMALL_WEIGHT_C, c.small16) &&
+           small(c.bias, device, 2 * width, type, may_narrow, SRU_AMD_SMALL_BIAS, c.small16) &&
+           small(c.init, device, c.batch * width, type, may_narrow, SRU_AMD_SMALL_INIT, c.small16) &&
+           small(c.scale, device, 1, type, may_narrow, SRU_AMD_SMALL_SCALE, c.small16) &&
+           small(c.mask_c, device, c.batch * width, type, may_narrow, SRU_AMD_SMALL_MASK, c.small16) &&
+           plain_pad(c.pad, device, c.length, c.batch);
+}
+
+void *stream_of(const c10::Device &device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
+
+PyObject *none() { Py_RETURN_NONE; }
+PyObject *wrap(const at::Tensor &t) {
+    if (!t.defined()) return none();
+    return THPVariable_Wrap(t);
+}
+
+// scan_forward(u, x, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_c, mask_pad, train)
+//   -> (h, last, checkpoints or None, whether x and scale are read)
+PyObject *scan_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Call c;
+    if (n != 13 || !read(a[0], c.u) || !read(a[1], c.x) || !read(a[2], c.weight_c) || !read(a[3], c.bias) || !read(a[4], c.init) ||
+        !read(a[5], c.act) || !read(a[6], c.d) || !read(a[9], c.scale) || !read(a[10], c.mask_c) || !read(a[11], c.pad))
+        return none();
+    c.bidirectional = PyObject_IsTrue(a[7]) == 1;
+    c.has_skip = PyObject_IsTrue(a[8]) == 1;
+    const bool train = a[12] == Py_True;
+    if (!c.x || c.x->dim() != 3) return none();
+    c.length = c.x->size(0);
+    c.batch = c.x->size(1);
+    if (!prepare(c, train, !train)) return none();
+    const c10::DeviceGuard guard(c.device());
+    const auto options = c.u->options();
+    const at::Tensor h = at::empty({c.length, c.batch, c.width()}, options);
+    const at::Tensor last = at::empty({c.batch, c.width()}, options);
+    at::Tensor kept;
+    if (train)
+        kept = at::empty({(int64_t)sru_amd_state_bytes(&c.shape) / (4 * c.batch * c.width()), c.batch, c.width()}, options.dtype(at::kFloat));
+    if (narrow(c.u->scalar_type())) c.small16 |= SRU_AMD_SMALL_LAST;
+    const int rc = sru_amd_forward_small(&c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(),
+                                         c.mask_c.ptr(), static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), h.data_ptr(),
+                                         train ? kept.data_ptr() : nullptr, last.data_ptr(), stream_of(c.device()));
+    if (rc != SRU_AMD_OK) return none();
+    return Py_BuildValue("(NNNO)", wrap(h), wrap(last), wrap(kept), c.shape.skip_type == 1 ? Py_True : Py_False);
+    END_HANDLE_TH_ERRORS
+}
+
+// scan_backward(u, x, weight_c, bias, init, scale, mask_c, mask_pad, checkpoints, grad_h, grad_last,
+//               act, d, bidirectional, has_skip, length, batch) -> (grad_u, grad_x, grad_weight_c, grad_bias, grad_init)
+PyObject *scan_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Call c;
+    Arg kept, grad_h, grad_last;
+    if (n != 17 || !read(a[0], c.u) || !read(a[1], c.x) || !read(a[2], c.weight_c) || !read(a[3], c.bias) || !read(a[4], c.init) ||
+        !read(a[5], c.scale) || !read(a[6], c.mask_c) || !read(a[7], c.pad) || !read(a[8], kept) || !read(a[9], grad_h) ||
+        !read(a[10], grad_last) || !read(a[11], c.act) || !read(a[12], c.d) || !read(a[15], c.length) || !read(a[16], c.batch))
+        return none();
+    c.bidirectional = PyObject_IsTrue(a[13]) == 1;
+    c.has_skip = PyObject_IsTrue(a[14]) == 1;
+    if (!kept || !grad_h || !prepare(c, true, false)) return none();
+    const c10::Device device = c.device();
+    const int64_t width = c.width(), columns = c.batch * width;
+    const at::ScalarType type = c.u->scalar_type();
+    if (kept->scalar_type() != at::kFloat || !plain(*kept.t, device, (int64_t)sru_amd_state_bytes(&c.shape) / 4, 4) ||
+        grad_h->scalar_type() != type || !plain(*grad_h.t, device, c.length * columns, 4) ||
+        !small(grad_last, device, columns, type, true, SRU_AMD_SMALL_LAST, c.small16))
+        return none();
+    const c10::DeviceGuard guard(device);
+    const auto floats = c.u->options().dtype(at::kFloat);
+    const at::Tensor grad_u = at::empty(c.u->sizes(), c.u->options());
+    at::Tensor grad_x, grad_init;
+    if (c.x) grad_x = at::empty(c.x->sizes(), c.x->options());
+    const at::Tensor grad_wc = at::empty({2 * width}, floats), grad_bias = at::empty(c.bias->sizes(), floats);
+    const int64_t need = (int64_t)sru_amd_backward_workspace_bytes(&c.shape);
+    // (the gradient of an initial state that was not given is written behind the workspace)
+    const at::Tensor workspace = at::empty({need / 4 + (c.init ? 0 : columns)}, floats);
+    if (c.init) grad_init = at::empty(c.init->sizes(), floats);
+    float *const init_out = c.init ? grad_init.data_ptr<float>() : workspace.data_ptr<float>() + need / 4;
+    const int rc = sru_amd_backward_small(
+        &c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(), c.mask_c.ptr(),
+        static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), kept.ptr(), grad_h.ptr(), grad_last.ptr(), grad_u.data_ptr(),
+        c.x ? grad_x.data_ptr() : nullptr, grad_wc.data_ptr(), grad_bias.data_ptr(), init_out, workspace.data_ptr(), (size_t)need,
+        stream_of(device));
+    if (rc != SRU_AMD_OK) return none();
+    return Py_BuildValue("(NNNNN)", wrap(grad_u), wrap(grad_x), wrap(grad_wc), wrap(grad_bias), wrap(grad_init));
+    END_HANDLE_TH_ERRORS
+}
+
+// layer_forward(x, residual, weight_proj, weight, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_pad)
+//   -> (h, last), False where no kernel takes the layer, None where the general way has to look
+PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Arg x, residual, weight_proj, weight, weight_c, bias, init, scale, pad;
+    int64_t act = 0, d = 0;
+    if (n != 13 || !read(a[0], x) || !read(a[1], residual) || !read(a[2], weight_proj) || !read(a[3], weight) || !read(a[4], weight_c) ||
+        !read(a[5], bias) || !read(a[6], init) || !read(a[7], act) || !read(a[8], d) || !read(a[11], scale) || !read(a[12], pad))
+        return none();
+    if (!x || !residual || !weight || !weight_c || !bias || !x->is_cuda() || x->dim() != 3 || d < 1) return none();
+    const at::ScalarType type = x->scalar_type();
+    if (!narrow(type)) Py_RETURN_FALSE;
+    const c10::Device device = x->device();
+    const int64_t length = x->size(0), batch = x->size(1), in = x->size(2), rows = length * batch;
+    const int64_t dirs = PyObject_IsTrue(a[9]) == 1 ? 2 : 1, width = d * dirs;
+    int64_t inner = in;
+    for (const Arg *w : {&weight_proj, &weight}) {
+        if (!*w) continue;
+        if ((*w)->scalar_type() != type || (*w)->dim() != 2 || (*w)->size(0) != inner || !plain(*w->t, device, (*w)->numel(), 16)) return none();
+        inner = (*w)->size(1);
+    }
+    const int64_t n_proj = weight_proj ? weight_proj->size(1) : 0, k = inner / width;
+    if ((k != 3 && k != 4) || inner != k * width || rows < 1 || weight_c->dim() != 1) return none();
+    sru_amd_shape s{};
+    s.length = length;
+    s.batch = batch;
+    s.hidden = d;
+    s.dirs = (int32_t)dirs;
+    s.k = (int32_t)k;
+    s.activation_type = (int32_t)act;
+    s.skip_type = PyObject_IsTrue(a[10]) != 1 ? 0 : k == 3 ? 1 : 2;
+    dtype_code(type, s.dtype);
+    s.state_interval = 1;
+    s.x_dtype = SRU_AMD_X_AS_STREAMS;
+    const bool whole = sru_amd_layer_route(&s, in, n_proj) != 0;
+    if (!whole && !(n_proj && sru_amd_layer_route(&s, n_proj, 0) != 0)) Py_RETURN_FALSE;
+    uint32_t small16 = SRU_AMD_SMALL_LAST;
+    if (s.skip_type != 1) scale = Arg{};
+    if (!plain(*x.t, device, rows * in, 16) ||
+        (s.skip_type == 1 && (residual->scalar_type() != type || !plain(*residual.t, device, rows * width, 16))) ||
+        !small(weight_c, device, 2 * width, type, true, SRU_AMD_SMALL_WEIGHT_C, small16) ||
+        !small(bias, device, 2 * width, type, true, SRU_AMD_SMALL_BIAS, small16) ||
+        !small(init, device, batch * width, type, true, SRU_AMD_SMALL_INIT, small16) ||
+        !small(scale, device, 1, type, true, SRU_AMD_SMALL_SCALE, small16) || !plain_pad(pad, device, length, batch))
+        return none();
+    const c10::DeviceGuard guard(device);
+    const auto options = x->options();
+    at::Tensor projected;
+    if (n_proj) projected = whole ? at::empty({rows, n_proj}, options) : at::mm(x->view({rows, in}), *weight_proj.t);
+    const at::Tensor h = at::empty({length, batch, width}, options), last = at::empty({batch, width}, options);
+    const bool inside = n_proj && whole;   // the projection is the kernels' business
+    const int rc = sru_amd_layer_forward(
+        &s, small16, n_proj && !whole ? n_proj : in, inside ? n_proj : 0, n_proj && !whole ? projected.data_ptr() : x.ptr(),
+        s.skip_type == 1 ? residual.ptr() : nullptr, inside ? weight_proj.ptr() : nullptr, weight.ptr(), weight_c.ptr(), bias.ptr(),
+        init.ptr(), static_cast<const uint8_t *>(pad.ptr()), scale.ptr(), inside ? projected.data_ptr() : nullptr, h.data_ptr(),
+        last.data_ptr(), stream_of(device));
+    if (rc != SRU_AMD_OK) return none();
+    return Py_BuildValue("(NN)", wrap(h), wrap(last));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},
+    {"scan_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_backward)), METH_FASTCALL, nullptr},
+    {"layer_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_forward)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Calls of the recurrence in the plain case.", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }

@@ -238,6 +238,11 @@ def elementwise_recurrence_forward(
     `keep_c=False` (no counterpart in the reference) skips storing the per-step
     state and returns None for it: the inference variant. `init=None` stands for zeros.
     """
+    if not keep_c:
+        done = _lib.host().scan_forward(u, x, weight_c, bias, init, activation_type, d_out, bidirectional, has_skip_term,
+                                        scale_x, mask_c, mask_pad, False)
+        if done is not None:
+            return done[0], done[1], None
     out_dtype = u.dtype
     if u.dtype != _kernel_dtype(u):
         u = u.to(_kernel_dtype(u))
@@ -270,6 +275,10 @@ def layer_forward(x: Tensor, residual: Tensor, weight_proj: Optional[Tensor], we
     """A layer's dense products and its recurrence without gradients, in kernels that do both: (h,
     last_hidden), or None where there are none for the problem (dtypes, sizes, alignment) and the
     caller has to project first. `residual` is what the skip term reads, `x` what is projected."""
+    done = _lib.host().layer_forward(x, residual, weight_proj, weight, weight_c, bias, init, activation_type, d_out,
+                                     bidirectional, has_skip_term, scale_x, mask_pad)
+    if done is not None:
+        return done or None
     dtype = x.dtype
     dirs = 2 if bidirectional else 1
     k = weight.size(-1) // (d_out * dirs)
@@ -330,6 +339,14 @@ class ElementwiseRecurrence(Function):
         # gradients that autograd does not have stay None instead of becoming zero tensors (one
         # fill kernel per layer for the usually unused gradient of the last state)
         ctx.set_materialize_grads(False)
+        done = _lib.host().scan_forward(u, x, weight_c, bias, init, activation_type, d_out, bidirectional, has_skip_term,
+                                        scale_x, mask_c, mask_pad, True)
+        if done is not None:
+            h, last_hidden, c, reads_x = done
+            ctx.problem = None
+            ctx.call = (activation_type, d_out, bidirectional, has_skip_term, x.size(0), x.size(1))
+            ctx.save_for_backward(u, x if reads_x else None, weight_c, bias, init, scale_x if reads_x else None, mask_c, mask_pad, c)
+            return h, last_hidden
         u_dtype = u.dtype
         if u.dtype != _kernel_dtype(u):
             u = u.to(_kernel_dtype(u))
@@ -353,9 +370,28 @@ class ElementwiseRecurrence(Function):
     def backward(ctx, grad_h, grad_last):
         pb = ctx.problem
         saved = list(ctx.saved_tensors)
-        c = saved.pop()
-        it = iter(saved)
-        u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_ = [next(it) if p else None for p in ctx.present]
+        if pb is None:
+            if grad_h is not None:
+                done = _lib.host().scan_backward(*saved, grad_h, grad_last, *ctx.call)
+                if done is not None:
+                    return done + (None,) * 7
+            # (a gradient that is missing, strided or of another dtype, or tensors that a saved-tensor
+            # hook gave back differently)
+            u, x, weight_c, bias, init, scale_x, mask_c, mask_pad, c = saved
+            activation_type, d_out, bidirectional, has_skip_term, length, batch = ctx.call
+            pb = _problem_cached(u.dtype, 3, length, batch, u.numel(), u.size(-1), 0, d_out, bool(bidirectional),
+                                 bool(has_skip_term), int(activation_type), True, x is not None and x.dtype == torch.float32, True)
+            (u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_), _ = _prepare_inputs(
+                pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
+            c = c.contiguous()
+            x_like = u if x is None else x     # (no gradient goes to an x that the skip term does not read)
+            in_dtypes = (u.dtype, x_like.dtype, weight_c.dtype, bias.dtype, None if init is None else init.dtype)
+            in_shapes = (u.shape, x_like.shape, weight_c.shape, bias.shape, None if init is None else init.shape)
+        else:
+            c = saved.pop()
+            it = iter(saved)
+            u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_ = [next(it) if p else None for p in ctx.present]
+            in_dtypes, in_shapes = ctx.in_dtypes, ctx.in_shapes
         dev = u_.device
         if grad_h is None:     # only last_hidden was used downstream
             gh = torch.zeros(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
@@ -380,8 +416,8 @@ class ElementwiseRecurrence(Function):
                 _ptr(grad_u), _ptr(grad_x), _ptr(grad_wc), _ptr(grad_bias), _ptr(grad_init),
                 _ptr(workspace), ctypes.c_size_t(ws_bytes), stream)
         _lib.check(rc, "sru_amd_backward_small")
-        u_dt, x_dt, wc_dt, bias_dt, init_dt = ctx.in_dtypes
-        u_sh, x_sh, wc_sh, bias_sh, init_sh = ctx.in_shapes
+        u_dt, x_dt, wc_dt, bias_dt, init_dt = in_dtypes
+        u_sh, x_sh, wc_sh, bias_sh, init_sh = in_shapes
         grad_u = grad_u.view(u_sh).to(u_dt)
         if grad_x is not None:
             grad_x = grad_x.view(x_sh).to(x_dt)
