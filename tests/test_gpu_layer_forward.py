@@ -70,7 +70,10 @@ def make(inp, d, dtype, **kw):
 
 STEP = [(64, 64, {}), (64, 64, dict(bidirectional=True)), (96, 32, dict(n_proj=32)), (256, 256, dict(n_proj=64)),
         (288, 288, dict(use_tanh=True)), (128, 128, dict(has_skip_term=False)), (2048, 2048, dict(n_proj=512)),
-        (2048, 96, {})]
+        (2048, 96, {}),
+        # the inner sizes where the number of steps in flight changes (512 with the recurrence, 1024 without)
+        (512, 512, {}), (544, 544, {}), (512, 512, dict(has_skip_term=False)), (544, 544, dict(has_skip_term=False)),
+        (1024, 96, dict(n_proj=32)), (1056, 96, dict(n_proj=64))]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
