@@ -5,8 +5,9 @@ Constructor arguments, parameter / buffer names (`weight`, `weight_proj`, `weigh
 `bias`, `scale_x`, `layer_norm.*`, `rnn_lst.{i}.*`, `input_to_hidden.weight`), the
 initialisation recipe and the forward semantics follow the reference, so a state_dict
 saved by it loads here and the same inputs give the same outputs. What differs is
-below the layer: the projection stays `torch.mm` (hipBLASLt) and the recurrence always
-runs the HIP kernels of this package; there is no CPU path (CPU tensors are refused).
+below the layer: the recurrence always runs the HIP kernels of this package, the projection
+is `torch.mm` (hipBLASLt) except where one kernel does both (`layer_forward`: 16-bit weights,
+no gradients); there is no CPU path (CPU tensors are refused).
 """
 import copy
 import math
