@@ -16,8 +16,8 @@ NORM_MAX_FEATURES = 4096       # SRU_AMD_NORM_MAX_FEATURES
 
 F32, F16, BF16, F64 = 0, 1, 2, 3
 X_AS_STREAMS, X_F32 = 0, 1   # SRU_AMD_X_AS_STREAMS, SRU_AMD_X_F32
-# SRU_AMD_SMALL_*: small tensors held in the stream type
 LAYER_STEP, LAYER_ROWS = 1, 2      # what sru_amd_layer_route answers
+# SRU_AMD_SMALL_*: small tensors held in the stream type
 SMALL_WEIGHT_C, SMALL_BIAS, SMALL_INIT, SMALL_MASK, SMALL_SCALE, SMALL_LAST = 1, 2, 4, 8, 16, 32
 
 
