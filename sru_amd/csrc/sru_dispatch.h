@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "sru_launch.h"
+#include "sru_relay.h"
 #include "sru_split.h"
 
 namespace sru_amd {
@@ -172,6 +173,36 @@ inline bool all_aligned_16(std::initializer_list<const void *> ptrs) {
     return true;
 }
 
+// Relay kernel (sru_relay.h): few columns, long enough a walk; whole 16-byte pieces of every stream lie in one
+// direction and batch row; the state is kept as checkpoints or not at all.
+// A workgroup of five wavefronts takes two register files' worth of a SIMD, so a compute unit holds one at a
+// time: beyond 256 workgroups (16384 columns) they follow each other (256 steps of 24576 columns bf16: 26.5 us,
+// lane pairs 20.7). The walk passes through five stages, 1-2.5 us more than the other kernels need to start.
+// Measured (us, the other kernel / this one; k = 3, two directions):
+//   bf16, 2048 columns     48 steps 5.6/5.5   96 8.7/7.6    192 14.8/10.9    padded: 48 6.0/7.5   96 9.6/8.8
+//   bf16, 16384 columns    48 steps 6.7/6.4   96 9.7/8.5    192 15.6/12.1    padded: 96 10.7/10.7 192 17.3/15.1
+//   bf16, d = 152          48 steps 7.5/6.2   96 11.8/8.2   192 20.4/11.9    padded: 48 8.3/8.4   96 13.2/10.6
+//   f32, 2048 columns      96 steps 9.5/9.1   192 16.5/13.6                  padded: 96 9.7/9.6   192 17.0/14.0
+//   f32, 16384 columns     96 steps 10.2/11.1 192 17.9/15.9                  padded: 96 11.9/12.9 192 20.0/18.1
+constexpr int64_t kRelayMaxColumns = 256 * kRelayCols;
+template <typename T> inline bool relay_wanted(const FwdParams &p) {
+    const int64_t least = (sizeof(T) == 4 ? 128 : 64) + (p.pad ? 40 : 0);
+    return !p.c && p.ncols <= kRelayMaxColumns && p.L >= least && p.L < (1 << 30) && p.d % (16 / (int)sizeof(T)) == 0 &&
+           all_aligned_16({p.u, p.x}) && aligned_to(p.h, 8) && aligned_to(p.ckpt, 8);
+}
+template <typename T, int K, int SKIP, typename TX = T, int X = 0, int STAGE = 0>
+hipError_t relay_forward(const FwdParams &p, hipStream_t st) {
+    if constexpr (STAGE == 0) {
+        return p.act ? relay_forward<T, K, SKIP, TX, X | kTanh, 1>(p, st) : relay_forward<T, K, SKIP, TX, X, 1>(p, st);
+    } else if constexpr (STAGE == 1) {
+        return p.pad ? relay_forward<T, K, SKIP, TX, X | kHasPad, 2>(p, st) : relay_forward<T, K, SKIP, TX, X, 2>(p, st);
+    } else {
+        void *args[] = {const_cast<FwdParams *>(&p)};
+        return hipLaunchKernel(reinterpret_cast<const void *>(forward_scan_relay<T, K, SKIP, X, kRelaySteps, TX>),
+                               dim3((unsigned)((p.ncols + kRelayCols - 1) / kRelayCols)), dim3(kRelayThreads), args, 0, st);
+    }
+}
+
 template <typename T, int K, int SKIP>
 hipError_t general_forward(const FwdParams &p, hipStream_t st) {
     return launch_grouped(forward_scan<T, K, SKIP, kGeneral | kNt, 1, general_ring_depth<T>()>, p.ncols, 1, 4, st, p);
@@ -186,10 +217,12 @@ hipError_t general_backward(const BwdParams &p, hipStream_t st) {
 // refuses checkpointed state for them.
 template <typename T, int K, int SKIP>
 hipError_t pick_forward(const sru_amd_shape &s, const FwdParams &p, hipStream_t st) {
+    if (!p.x_float && relay_wanted<T>(p)) return relay_forward<T, K, SKIP>(p, st);
     if constexpr (sizeof(T) == 2) {
         if constexpr (SKIP == 1) {
             if (p.x_float) {   // a float x next to 16-bit streams: chunked kernels only (the flag combinations were checked before)
                 if (p.act || p.c || !pair_ok<T, K>(s, {p.u}, {p.h}) || !aligned_to(p.x, 4)) return hipErrorInvalidValue;
+                if (relay_wanted<T>(p)) return relay_forward<T, K, SKIP, float, 0, 1>(p, st);
                 if (p.ncols / 2 < kPairBelow) return fast_forward<T, K, SKIP, 1, kPair, 1, float>(p, st);
                 return fast_forward<T, K, SKIP, 2, 0, 1, float>(p, st);
             }
