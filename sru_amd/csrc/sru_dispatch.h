@@ -17,6 +17,7 @@
 #include "sru_launch.h"
 #include "sru_relay.h"
 #include "sru_split.h"
+#include "sru_team.h"
 
 namespace sru_amd {
 
@@ -203,6 +204,46 @@ hipError_t relay_forward(const FwdParams &p, hipStream_t st) {
     }
 }
 
+// Team kernel (sru_team.h): wavefronts of a workgroup share the walk of 64 columns. A workgroup keeps to one
+// direction of one batch row where at most a fifth of its lanes is left over: addresses and flags are scalar then,
+// and padding at the ends is not walked.
+// Taken while its wavefronts are resident together (two to a SIMD; beyond that the chunked kernels have wavefronts
+// enough to hide their chain), from the third chunk on; eight wavefronts while that leaves one workgroup to a compute
+// unit, else four. Measured (us, backward call with its 4 us reduction, the other kernels / this one; k = 3):
+//   bf16, 16 steps   8192 columns 7.1/7.6   32768 8.4/9.0       24 steps   8192 10.1/7.8   32768 11.4/9.5
+//   bf16, 256 steps  8192 33.6/18.9   16384 34.3/23.2   40960 57.2/51.0   49152 57.4/56.0   57344 61.2/64.7
+//   padded           40960 68.2/51.4   49152 67.1/58.9   57344 71.8/62.0
+//   bf16, 512 steps  2048 59.8/28.4   32768 71.8/64.7 (float x 85.7/73.2)
+//   f32, 32 steps    8192 9.9/8.1      256 steps  12288 41.7/27.0   20480 47.2/47.5   24576 48.3/50.8
+//   f32, 512 steps   2048 77.1/31.2   8192 77.6/40.2   16384 79.1/61.2 (padded 97.3/62.5)
+//   any 64 columns: d = 40, 256 steps, 10240 columns bf16 54.7/30.9
+inline bool team_by_row(int32_t d) { return (d + kBlock - 1) / kBlock * kBlock * 4 <= d * 5; }
+inline int64_t team_groups(int64_t ncols, int32_t d) {
+    return team_by_row(d) ? ncols / d * ((d + kBlock - 1) / kBlock) : (ncols + kBlock - 1) / kBlock;
+}
+template <typename T> inline int team_waves(const BwdParams &p) {
+    const int64_t groups = team_groups(p.ncols, p.d), chunks = (p.L + kCkptInterval - 1) / kCkptInterval;
+    if (chunks < 3 || groups > (sizeof(T) == 4 ? 256 : p.pad ? 896 : 768)) return 1;
+    return groups <= 128 && chunks > 4 ? 8 : 4;
+}
+// X, STAGE, TX: as in fast_forward
+template <typename T, int K, int SKIP, int X = 0, int STAGE = 0, typename TX = T>
+hipError_t team_backward(const BwdParams &p, int waves, hipStream_t st) {
+    if constexpr (STAGE == 0) {
+        return p.act ? team_backward<T, K, SKIP, X | kTanh, 1, TX>(p, waves, st) : team_backward<T, K, SKIP, X, 1, TX>(p, waves, st);
+    } else if constexpr (STAGE == 1) {
+        return p.pad ? team_backward<T, K, SKIP, X | kHasPad, 2, TX>(p, waves, st) : team_backward<T, K, SKIP, X, 2, TX>(p, waves, st);
+    } else if constexpr (STAGE == 2) {
+        return team_by_row(p.d) ? team_backward<T, K, SKIP, X | kUniform, 3, TX>(p, waves, st)
+                                : team_backward<T, K, SKIP, X, 3, TX>(p, waves, st);
+    } else {
+        void *args[] = {const_cast<BwdParams *>(&p)};
+        constexpr int kLanes = sizeof(T) == 2 ? kPair : 0;
+        return hipLaunchKernel(reinterpret_cast<const void *>(backward_scan_team<T, K, SKIP, X | kLanes | kNt, TX>),
+                               dim3((unsigned)team_groups(p.ncols, p.d)), dim3((unsigned)(kBlock * waves)), args, 0, st);
+    }
+}
+
 template <typename T, int K, int SKIP>
 hipError_t general_forward(const FwdParams &p, hipStream_t st) {
     return launch_grouped(forward_scan<T, K, SKIP, kGeneral | kNt, 1, general_ring_depth<T>()>, p.ncols, 1, 4, st, p);
@@ -245,10 +286,13 @@ hipError_t pick_backward(const sru_amd_shape &s, const BwdParams &p, hipStream_t
             if (p.x_float) {
                 if (p.act || !p.ckpt || !pair_ok<T, K>(s, {p.u, p.gu}, {p.gh}) || !aligned_to(p.x, 4) || !aligned_to(p.gx, 4))
                     return hipErrorInvalidValue;
+                if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP, 0, 1, float>(p, w, st);
                 if (p.ncols / 2 < kPairBelow) return fast_backward<T, K, SKIP, 1, kPair, 1, float>(p, st);
                 return fast_backward<T, K, SKIP, 2, 0, 1, float>(p, st);
             }
         }
+        if (p.ckpt && pair_ok<T, K>(s, {p.u, p.gu}, {p.x, p.c, p.gh, p.gx}))
+            if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP>(p, w, st);
         if (p.ckpt && split_wanted(p.ncols, p.d) && all_aligned_16({p.u, p.x, p.gh, p.gu, p.gx}))
             return split_backward<T, K, SKIP>(p, st);
         if (!pair_ok<T, K>(s, {p.u, p.gu}, {p.x, p.c, p.gh, p.gx}))   // p.c is null with checkpoints
@@ -256,6 +300,8 @@ hipError_t pick_backward(const sru_amd_shape &s, const BwdParams &p, hipStream_t
         if (p.ckpt && p.ncols / 2 < kPairBelow) return fast_backward<T, K, SKIP, 1, kPair>(p, st);
         return fast_backward<T, K, SKIP, 2>(p, st);
     } else {
+        if (p.ckpt)
+            if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP>(p, w, st);
         return fast_backward<T, K, SKIP, 1>(p, st);
     }
 }

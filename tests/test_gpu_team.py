@@ -1,0 +1,76 @@
+"""The backward kernel whose wavefronts share a walk (sru_team.h) against the CPU oracle: walks from its shortest
+(17 steps) on, around chunks of 8 steps and rounds of 4 and 8 chunks; columns by direction and row (d near a
+multiple of 64), any 64 columns (other d), a last workgroup that is not full; the limits of its column counts.
+Tolerances as in test_gpu_parity.py: its sums are those of the other kernels but for the order of a chunk's factors."""
+import numpy as np
+import pytest
+import torch
+
+import sru_amd
+from tests.cases import Case
+from tests.test_gpu_parity import check_against_oracle
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    dict(L=17, B=1, d=8),
+    dict(L=24, B=3, d=56, dirs=2, pad="right", scale=1.7),
+    dict(L=31, B=5, d=152, dirs=2, pad="right", mask_c=True),
+    dict(L=33, B=130, d=64, k=4, pad="random"),
+    dict(L=64, B=3, d=120, dirs=2, k=4, act=1),
+    dict(L=65, B=2, d=64, dirs=2, skip=False, pad="right", mask_c=True),
+    dict(L=72, B=7, d=22, dirs=2, act=1, pad="random", scale=1.3),
+    dict(L=128, B=4, d=128, dirs=2, zero_c0=True),
+    dict(L=129, B=1, d=40, dirs=2, skip=False, act=1),
+    dict(L=201, B=3, d=304, dirs=2, k=4, pad="right"),
+]
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("cfg", SHAPES, ids=lambda g: "-".join(f"{k}{v}" for k, v in g.items()))
+def test_against_the_oracle(cfg, dt):
+    check_against_oracle(Case(seed=41, **cfg), dt, checkpointed=True)
+
+
+@pytest.mark.parametrize("pad", [None, "right"])
+@pytest.mark.parametrize("d", [72, 192])
+def test_float_x_beside_16_bit_streams(d, pad):
+    check_against_oracle(Case(L=57, B=3, d=d, dirs=2, scale=1.7, mask_c=True, pad=pad, seed=42), "bf16",
+                         checkpointed=True, x_f32=True)
+
+
+@pytest.mark.parametrize("dt,B", [("f32", 256), ("f32", 257), ("bf16", 128), ("bf16", 129), ("bf16", 768), ("bf16", 769)])
+def test_column_limits(dt, B):
+    check_against_oracle(Case(L=41, B=B, d=64, seed=43), dt, checkpointed=True)
+
+
+@pytest.mark.parametrize("d", [24, 64])
+@pytest.mark.parametrize("L", [32, 100])
+def test_factors_beyond_the_float_range(L, d):
+    # Every step but the first multiplies the state's gradient by about 4e5, eight of them by more than a float
+    # holds; the gradient itself is zero there (only the first output has one), and stays zero.
+    gen = np.random.default_rng(5)
+    B, D = 2, d
+    u = np.zeros((L, B, D, 3), np.float32)
+    c = np.zeros((B, D), np.float32)
+    for t in range(L):
+        u[t, ..., 0] = 4e6 * (-1) ** t * (1 + 0.1 * gen.random((B, D)))
+        u[t, ..., 1] = 2.0 - c
+        g = 1 / (1 + np.exp(-(u[t, ..., 1].astype(np.float64) + c)))
+        c = ((c - u[t, ..., 0]) * g + u[t, ..., 0]).astype(np.float32)
+    leaf = lambda a: torch.tensor(a, dtype=torch.float32, device="cuda", requires_grad=True)
+    U, x = leaf(u.reshape(L, B, 3 * D)), leaf(gen.standard_normal((L, B, D)))
+    wc, bias = leaf(np.ones(2 * D)), leaf(np.zeros(2 * D))
+    h, _ = sru_amd.ElementwiseRecurrence.apply(U, x, wc, bias, None, 0, d, False, True, None, None, None)
+    gh = torch.zeros_like(h)
+    gh[0] = 1.0
+    gu, gx, gwc, gbias = torch.autograd.grad(h, (U, x, wc, bias), gh)
+    gu = gu.view(L, B, D, 3).cpu()
+    assert (gu[1:] == 0).all() and (gx[1:] == 0).all()
+    # the first step: c = u0 (1 - g1), h = (c - x) g2 + x with g2 = 1/2
+    u0, x0 = torch.tensor(u[0, ..., 0]).double(), x[0].detach().cpu().double()
+    g1 = torch.sigmoid(torch.tensor(2.0, dtype=torch.float64))
+    expect = torch.stack([0.5 * (1 - g1).expand_as(u0), -0.5 * u0 * g1 * (1 - g1), 0.25 * (u0 * (1 - g1) - x0)], -1)
+    # (a gate is within 1e-7, relative to 1 - g1 = 0.12: 1e-6)
+    assert ((gu[0].double() - expect).abs() <= 2e-6 * expect.abs()).all()
+    assert (gwc == 0).all() and gbias.isfinite().all()
