@@ -258,6 +258,13 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
                           const uint8_t *mask_pad, const void *scale_x, void *projected,
                           void *h, void *c_last, void *stream);
 
+/* A dense product, out (rows, cols) = x (rows, inner) weight (inner, cols), all row-major in `dtype` (float, or 16
+ * bits with float sums) and 16-byte aligned: compute_U of a short sequence or a prompt (sru/modules.py:252-274,
+ * a library call there). sru_amd_product_wanted says whether the kernel takes a problem (a library product is
+ * faster for the others, or a size is not a multiple of 4 or 8); sru_amd_product answers BAD_SHAPE otherwise. */
+int sru_amd_product_wanted(int32_t dtype, int64_t rows, int64_t inner, int64_t cols);
+int sru_amd_product(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *weight, void *out, void *stream);
+
 /* Layer normalisation of the rows of a (rows, cols) matrix, the operation the reference applies to a
  * layer's input before the projection or to its output after the recurrence with
  * torch.nn.LayerNorm (sru/modules.py:155-162 created, :250-253 and :278-279 applied):

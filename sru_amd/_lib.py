@@ -50,6 +50,8 @@ SIGNATURES = {
     "sru_amd_backward_static": (ctypes.c_int, [ctypes.POINTER(Shape)] + [_P] * 17),
     "sru_amd_layer_route": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
     "sru_amd_layer_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 13),
+    "sru_amd_product_wanted": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3),
+    "sru_amd_product": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3 + [_P] * 4),
     "sru_amd_layer_norm_forward": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, _P, ctypes.c_int, _P, _P,
                                                   ctypes.c_float, _P, ctypes.c_int, _P, _P, _P]),
     "sru_amd_layer_norm_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64]),

@@ -243,6 +243,16 @@ PyObject *scan_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// x weight, with `own` by a kernel where that is the faster one (the device is set)
+at::Tensor product(const at::Tensor &x, const at::Tensor &weight, int32_t dtype, bool own) {
+    const int64_t rows = x.size(0), inner = x.size(1), cols = weight.size(1);
+    if (own && sru_amd_product_wanted(dtype, rows, inner, cols)) {
+        at::Tensor out = at::empty({rows, cols}, x.options());
+        if (sru_amd_product(dtype, rows, inner, cols, x.data_ptr(), weight.data_ptr(), out.data_ptr(), stream_of(x.device())) == SRU_AMD_OK) return out;
+    }
+    return at::mm(x, weight);
+}
+
 // layer_forward(x, residual, weight_proj, weight, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_pad)
 //   -> (h, last), False where no kernel takes the layer or a mode watches, None where the general way has to look
 PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
@@ -257,7 +267,7 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         return none();
     if (!x || !residual || !weight || !weight_c || !bias || !x->is_cuda() || x->dim() != 3 || d < 1) return none();
     const at::ScalarType type = x->scalar_type();
-    if (!narrow(type)) Py_RETURN_FALSE;
+    if (!narrow(type) && type != at::kFloat) Py_RETURN_FALSE;
     const c10::Device device = x->device();
     const int64_t length = x->size(0), batch = x->size(1), in = x->size(2), rows = length * batch;
     const int64_t dirs = bidirectional ? 2 : 1, width = d * dirs;
@@ -280,13 +290,17 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     dtype_code(type, s.dtype);
     s.state_interval = 1;
     s.x_dtype = SRU_AMD_X_AS_STREAMS;
-    // Both products in kernels, or the second one with the recurrence, or library products and the scan: the
-    // last for one step at sizes past the step kernels' only, where the host's time counts (4096 features,
-    // 16 rows: 29.9 us a layer, 29.7 of them kernels).
+    // Both products in kernels, or the second one with the recurrence, or products and the scan: the last where
+    // one of the products is a kernel (one step in 16 bits has the step kernels instead), and for one step at sizes
+    // past the step kernels', where the host's time counts (4096 features, 16 rows: 29.9 us a layer, 29.7 of them
+    // kernels). Two layers of 640 rows and 128 features in float take 69.6 us a pass as calls of torch and the
+    // scan, 32.9 this way.
     const bool whole = sru_amd_layer_route(&s, in, n_proj) != 0;
     const bool fused = whole || (n_proj && sru_amd_layer_route(&s, n_proj, 0) != 0);
-    if (!fused && !(length == 1 && batch <= 64 && width % 32 == 0 && in % 32 == 0 && n_proj % 32 == 0)) Py_RETURN_FALSE;
-    uint32_t small16 = SRU_AMD_SMALL_LAST;
+    const bool own = !fused && (length > 1 || !narrow(type)) &&
+                     (sru_amd_product_wanted(s.dtype, rows, n_proj ? n_proj : in, k * width) || (n_proj && sru_amd_product_wanted(s.dtype, rows, in, n_proj)));
+    if (!fused && !own && !(narrow(type) && length == 1 && batch <= 64 && width % 32 == 0 && in % 32 == 0 && n_proj % 32 == 0)) Py_RETURN_FALSE;
+    uint32_t small16 = narrow(type) ? SRU_AMD_SMALL_LAST : 0;
     if (s.skip_type != 1) scale = Arg{};
     if (!plain(*x.t, device, rows * in, 16) ||
         (s.skip_type == 1 && (residual->scalar_type() != type || !plain(*residual.t, device, rows * width, 16))) ||
@@ -302,7 +316,7 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const c10::DeviceGuard guard(device);
         const auto options = x->options();
         at::Tensor y = x->view({rows, in}), projected;
-        if (n_proj && !whole) y = at::mm(y, *weight_proj.t);
+        if (n_proj && !whole) y = product(y, *weight_proj.t, s.dtype, own);
         if (n_proj && whole) projected = at::empty({rows, n_proj}, options);   // the projection is the kernels' business
         h = at::empty({length, batch, width}, options);
         last = at::empty({batch, width}, options);
@@ -313,7 +327,7 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
                                        weight.ptr(), weight_c.ptr(), bias.ptr(), init.ptr(), mask, scale.ptr(),
                                        projected.defined() ? projected.data_ptr() : nullptr, h.data_ptr(), last.data_ptr(), stream_of(device));
         else
-            rc = sru_amd_forward_small(&s, small16, at::mm(y, *weight.t).data_ptr(), skip, weight_c.ptr(), bias.ptr(), init.ptr(), nullptr,
+            rc = sru_amd_forward_small(&s, small16, product(y, *weight.t, s.dtype, own).data_ptr(), skip, weight_c.ptr(), bias.ptr(), init.ptr(), nullptr,
                                        mask, scale.ptr(), h.data_ptr(), nullptr, last.data_ptr(), stream_of(device));
     }
     if (rc != SRU_AMD_OK) return none();

@@ -94,4 +94,40 @@ inline bool rows_sizes_ok(int64_t L, int64_t B, int64_t d, int64_t dirs, int64_t
 }
 hipError_t launch_layer_rows(const RowsParams &p, bool half, int k, hipStream_t st);
 
+// A product by itself (product.hip): x (rows, inner) times weight (inner, cols), all in one type.
+struct ProductParams {
+    const void *x, *weight;
+    void *out;
+    int32_t rows, inner, cols;
+};
+
+// The tile of a product's workgroups, 32 rows x 32 columns at the least, and whether they split the inner dimension
+// in two; none where the library's product is faster or a size is not a whole number of 16-byte pieces.
+//
+// Larger tiles read less, smaller ones leave a workgroup for more compute units: a larger one is taken from about
+// three workgroups to four compute units on (float, whose tiles take four times as long in the matrix cores, from
+// three workgroups to a unit). Two halves of the inner dimension where it is long and compute units are left over.
+// Measured (us in a graph, library / 32 x 32 / 32 x 64 / 64 x 64, the rule's choice marked *, with "2" where split):
+//   bf16   33 x 256 -> 768      4.5/3.1*/3.6/3.9      128 x 256 -> 3072    6.7/4.0/3.8*/4.4    512 x 512 -> 6144   12.9/17.1/13.4/11.3*
+//          128 x 1024 -> 256    10.5/4.8*2/6.3/7.4    512 x 2048 -> 512   10.8/8.8*2/10.3/12.6 128 x 2048 -> 6144  18.8/17.7/16.1/13.1*2
+//   f32    640 x 128 -> 384     4.3/3.4*/4.3/5.6      2048 x 256 -> 768   22.3/12.3/12.2*/14.0 1024 x 256 -> 3072  24.7/21.0/19.6/18.9*
+// Past 1.75e9 multiply-adds the library is faster (bf16 512 x 2048 -> 6144 26.4/30.5, 1024 x 512 -> 6144
+// 16.3/18.8, 2048 x 1024 -> 3072 21.9/30.8); below, 2048 x 256 -> 3072 (12.0/12.4) is the worst of those measured.
+// In float it is faster too where the inner dimension is long (128 x 2048 -> 512 10.0/14.3, 64 x 1536 -> 4608
+// 17.2/18.8) or longer than the result is wide (512 x 1024 -> 256 8.9/9.3); below 64 inner indices or columns it is not measured.
+// Launched one by one a library product costs
+// its caller 18 us, and this one 4.
+struct ProductTile { int m, n, split; };   // in units of 32; m 0: none
+inline ProductTile product_tile(int size, int64_t rows, int64_t inner, int64_t cols) {
+    const bool f32 = size == 4;
+    if (rows < 1 || inner < 1 || cols < 1 || inner % (f32 ? 4 : 8) != 0 || cols % 4 != 0 || rows > (1 << 20) || inner > (1 << 14) ||
+        cols > (1 << 16) || (f32 && (inner < 64 || cols < 64)) || rows * inner * cols > (int64_t)1750000000 || (f32 && inner > 512 && (inner > 1024 || cols < 2 * inner)))
+        return {0, 0, 0};
+    const auto tiles = [&](int m, int n) { return (rows + 32 * m - 1) / (32 * m) * ((cols + 32 * n - 1) / (32 * n)); };
+    ProductTile t = tiles(2, 2) >= (f32 ? 768 : 192) ? ProductTile{2, 2, 1} : tiles(1, 2) >= (f32 ? 384 : 192) ? ProductTile{1, 2, 1} : ProductTile{1, 1, 1};
+    if (inner >= (f32 ? 512 : 1024) && tiles(t.m, t.n) <= 256) t.split = 2;
+    return t;
+}
+hipError_t launch_product(const ProductParams &p, int32_t dtype, const ProductTile &tile, hipStream_t st);
+
 }  // namespace sru_amd

@@ -162,7 +162,8 @@ class SRUCell(nn.Module):
         """Whether `layer_forward` may stand for compute_UV and apply_recurrence: nothing is
         differentiated or autocast, the layer projects with its own weights, no step is overridden (by a
         subclass, on the instance or on the class), and the input is a plain tensor that nothing records."""
-        return (not torch.is_grad_enabled() and self.custom_m is None and input.dtype in (torch.float16, torch.bfloat16)
+        return (not torch.is_grad_enabled() and self.custom_m is None
+                and input.dtype in (torch.float16, torch.bfloat16, torch.float32)
                 and getattr(self, "native_16bit", True) and type(input) is Tensor and type(residual) is Tensor
                 and getattr(self.compute_UV, "__func__", None) is _COMPUTE_UV
                 and getattr(self.compute_U, "__func__", None) is _COMPUTE_U

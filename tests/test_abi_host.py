@@ -238,3 +238,20 @@ def test_long_sequence_route_goes_by_rounds_of_workgroups(inner, hidden, dirs, k
 def test_one_step_route_ends_where_library_products_are_faster(inner, n_proj, rows, taken):
     shape = _lib.Shape(1, rows, 512, 1, 4, 0, 2, 0, _lib.BF16, 1, _lib.X_AS_STREAMS)
     assert _lib.load().sru_amd_layer_route(ctypes.byref(shape), inner, n_proj) == (_lib.LAYER_STEP if taken else 0)
+
+
+@pytest.mark.parametrize("dtype,rows,inner,cols,taken", [
+    (_lib.F32, 640, 128, 384, 1), (_lib.F32, 640, 126, 384, 0), (_lib.F32, 640, 128, 382, 0), (_lib.F32, 640, 60, 384, 0), (_lib.F32, 640, 128, 60, 0), (_lib.F32, 128, 1024, 2048, 1),
+    (_lib.F32, 128, 1024, 2044, 0), (_lib.F32, 128, 1028, 4096, 0), (_lib.BF16, 512, 512, 6144, 1), (_lib.BF16, 512, 516, 6144, 0),
+    (_lib.F16, 1, 8, 4, 1), (_lib.F16, 512, 2048, 6144, 0), (_lib.F64, 64, 64, 64, 0), (_lib.BF16, 0, 64, 64, 0), (9, 64, 64, 64, 0)])
+def test_product_wanted(dtype, rows, inner, cols, taken):
+    lib = _lib.load()
+    assert lib.sru_amd_product_wanted(dtype, rows, inner, cols) == taken
+    # (nothing is launched: null pointers, or sizes that are not taken)
+    text = lib.sru_amd_status_string(lib.sru_amd_product(dtype, rows, inner, cols, None, None, None, None))
+    assert text == lib.sru_amd_status_string(_lib_status("NULL_POINTER" if taken else "BAD_SHAPE"))
+
+
+def _lib_status(name):
+    header = open(os.path.join(ROOT, "include", "sru_amd.h")).read()
+    return int(re.search(r"SRU_AMD_ERR_%s\s*=?\s*(\d+)" % name, header).group(1))
