@@ -265,6 +265,14 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
 int sru_amd_product_wanted(int32_t dtype, int64_t rows, int64_t inner, int64_t cols);
 int sru_amd_product(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *weight, void *out, void *stream);
 
+/* The weight's gradient of such a product over many rows, grad_weight (inner, cols) = x^T grad_out, x (rows, inner)
+ * and grad_out (rows, cols) in 16 bits, the result in grad_dtype: `dtype`, or float as a float parameter under
+ * autocast wants it. The workspace size is 0 where there is no kernel (the library's product is not slower, or a size
+ * is not a multiple of 8), and the call answers BAD_SHAPE. Everything 16-byte aligned. */
+size_t sru_amd_product_grad_workspace_bytes(int32_t dtype, int64_t rows, int64_t inner, int64_t cols);
+int sru_amd_product_grad(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *grad_out, int32_t grad_dtype,
+                         void *grad_weight, void *workspace, size_t workspace_bytes, void *stream);
+
 /* Layer normalisation of the rows of a (rows, cols) matrix, the operation the reference applies to a
  * layer's input before the projection or to its output after the recurrence with
  * torch.nn.LayerNorm (sru/modules.py:155-162 created, :250-253 and :278-279 applied):

@@ -52,6 +52,8 @@ SIGNATURES = {
     "sru_amd_layer_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 13),
     "sru_amd_product_wanted": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3),
     "sru_amd_product": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3 + [_P] * 4),
+    "sru_amd_product_grad_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int32] + [ctypes.c_int64] * 3),
+    "sru_amd_product_grad": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3 + [_P, _P, ctypes.c_int32, _P, _P, ctypes.c_size_t, _P]),
     "sru_amd_layer_norm_forward": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int64, _P, ctypes.c_int, _P, _P,
                                                   ctypes.c_float, _P, ctypes.c_int, _P, _P, _P]),
     "sru_amd_layer_norm_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int64]),
@@ -98,7 +100,7 @@ _host = None
 class GeneralHost:
     """Stands for the native host code where that cannot be used: nothing is plain, every call goes the
     general way of functional.py."""
-    scan_forward = scan_backward = staticmethod(lambda *args: None)
+    scan_forward = scan_backward = product = staticmethod(lambda *args: None)
     layer_forward = staticmethod(lambda *args: False)
 
 

@@ -267,7 +267,7 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         return none();
     if (!x || !residual || !weight || !weight_c || !bias || !x->is_cuda() || x->dim() != 3 || d < 1) return none();
     const at::ScalarType type = x->scalar_type();
-    if (!narrow(type) && type != at::kFloat) Py_RETURN_FALSE;
+    if (!narrow(type)) Py_RETURN_FALSE;
     const c10::Device device = x->device();
     const int64_t length = x->size(0), batch = x->size(1), in = x->size(2), rows = length * batch;
     const int64_t dirs = bidirectional ? 2 : 1, width = d * dirs;
@@ -293,14 +293,13 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     // Both products in kernels, or the second one with the recurrence, or products and the scan: the last where
     // one of the products is a kernel (one step in 16 bits has the step kernels instead), and for one step at sizes
     // past the step kernels', where the host's time counts (4096 features, 16 rows: 29.9 us a layer, 29.7 of them
-    // kernels). Two layers of 640 rows and 128 features in float take 69.6 us a pass as calls of torch and the
-    // scan, 32.9 this way.
+    // kernels).
     const bool whole = sru_amd_layer_route(&s, in, n_proj) != 0;
     const bool fused = whole || (n_proj && sru_amd_layer_route(&s, n_proj, 0) != 0);
-    const bool own = !fused && (length > 1 || !narrow(type)) &&
+    const bool own = !fused && length > 1 &&
                      (sru_amd_product_wanted(s.dtype, rows, n_proj ? n_proj : in, k * width) || (n_proj && sru_amd_product_wanted(s.dtype, rows, in, n_proj)));
-    if (!fused && !own && !(narrow(type) && length == 1 && batch <= 64 && width % 32 == 0 && in % 32 == 0 && n_proj % 32 == 0)) Py_RETURN_FALSE;
-    uint32_t small16 = narrow(type) ? SRU_AMD_SMALL_LAST : 0;
+    if (!fused && !own && !(length == 1 && batch <= 64 && width % 32 == 0 && in % 32 == 0 && n_proj % 32 == 0)) Py_RETURN_FALSE;
+    uint32_t small16 = SRU_AMD_SMALL_LAST;
     if (s.skip_type != 1) scale = Arg{};
     if (!plain(*x.t, device, rows * in, 16) ||
         (s.skip_type == 1 && (residual->scalar_type() != type || !plain(*residual.t, device, rows * width, 16))) ||
@@ -335,7 +334,29 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// product(x, weight) -> x weight in float, by the kernel where that is the faster one, else None
+PyObject *float_product(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Arg x, weight;
+    if (observed() || n != 2 || !read(a[0], x) || !read(a[1], weight) || !x || !weight || !x->is_cuda() || x->dim() != 2 || weight->dim() != 2 ||
+        x->scalar_type() != at::kFloat || weight->scalar_type() != at::kFloat || x->size(1) != weight->size(0))
+        return none();
+    const int64_t rows = x->size(0), inner = x->size(1), cols = weight->size(1);
+    const c10::Device device = x->device();
+    if (!sru_amd_product_wanted(SRU_AMD_F32, rows, inner, cols) || !plain(*x.t, device, rows * inner, 16) || !plain(*weight.t, device, inner * cols, 16))
+        return none();
+    at::Tensor out;
+    {
+        const Unlocked unlocked;
+        const c10::DeviceGuard guard(device);
+        out = product(*x.t, *weight.t, SRU_AMD_F32, true);
+    }
+    return wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"product", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(float_product)), METH_FASTCALL, nullptr},
     {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},
     {"scan_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_backward)), METH_FASTCALL, nullptr},
     {"layer_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_forward)), METH_FASTCALL, nullptr},

@@ -359,4 +359,23 @@ int sru_amd_product(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, co
     return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
 }
 
+size_t sru_amd_product_grad_workspace_bytes(int32_t dtype, int64_t rows, int64_t inner, int64_t cols) {
+    if (dtype != SRU_AMD_F16 && dtype != SRU_AMD_BF16) return 0;
+    return sizeof(float) * (size_t)product_grad_plan(rows, inner, cols).splits * (size_t)inner * (size_t)cols;
+}
+
+int sru_amd_product_grad(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *grad_out, int32_t grad_dtype,
+                         void *grad_weight, void *workspace, size_t workspace_bytes, void *stream) {
+    const size_t need = sru_amd_product_grad_workspace_bytes(dtype, rows, inner, cols);
+    if (need == 0) return SRU_AMD_ERR_BAD_SHAPE;
+    if (grad_dtype != SRU_AMD_F32 && grad_dtype != dtype) return SRU_AMD_ERR_BAD_DTYPE;
+    if (!x || !grad_out || !grad_weight) return SRU_AMD_ERR_NULL_POINTER;
+    if (!workspace || !aligned(workspace, 16) || workspace_bytes < need) return SRU_AMD_ERR_WORKSPACE;
+    if (!aligned(x, 16) || !aligned(grad_out, 16) || !aligned(grad_weight, 16)) return SRU_AMD_ERR_MISALIGNED;
+    const GradPlan plan = product_grad_plan(rows, inner, cols);
+    const GradParams p{x, grad_out, static_cast<float *>(workspace), (int32_t)rows, (int32_t)inner, (int32_t)cols, plan.splits};
+    const hipError_t err = launch_product_grad(p, plan, dtype == SRU_AMD_F16, grad_dtype, grad_weight, static_cast<hipStream_t>(stream));
+    return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
+}
+
 }  // extern "C"

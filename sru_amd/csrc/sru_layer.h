@@ -106,7 +106,8 @@ struct ProductParams {
 //
 // Larger tiles read less, smaller ones leave a workgroup for more compute units: a larger one is taken from about
 // three workgroups to four compute units on (float, whose tiles take four times as long in the matrix cores, from
-// three workgroups to a unit). Two halves of the inner dimension where it is long and compute units are left over.
+// three workgroups to a unit), unless that is just one round of them and a little of another, of many
+// inner indices each (bf16 200 x 1536 -> 4608, 288 workgroups: 17.8 us, 32 x 64 tiles 14.0, library 15.0). Two halves of the inner dimension where it is long and compute units are left over.
 // Measured (us in a graph, library / 32 x 32 / 32 x 64 / 64 x 64, the rule's choice marked *, with "2" where split):
 //   bf16   33 x 256 -> 768      4.5/3.1*/3.6/3.9      128 x 256 -> 3072    6.7/4.0/3.8*/4.4    512 x 512 -> 6144   12.9/17.1/13.4/11.3*
 //          128 x 1024 -> 256    10.5/4.8*2/6.3/7.4    512 x 2048 -> 512   10.8/8.8*2/10.3/12.6 128 x 2048 -> 6144  18.8/17.7/16.1/13.1*2
@@ -125,9 +126,55 @@ inline ProductTile product_tile(int size, int64_t rows, int64_t inner, int64_t c
         return {0, 0, 0};
     const auto tiles = [&](int m, int n) { return (rows + 32 * m - 1) / (32 * m) * ((cols + 32 * n - 1) / (32 * n)); };
     ProductTile t = tiles(2, 2) >= (f32 ? 768 : 192) ? ProductTile{2, 2, 1} : tiles(1, 2) >= (f32 ? 384 : 192) ? ProductTile{1, 2, 1} : ProductTile{1, 1, 1};
+    if (!f32 && inner >= 1024 && t.m == 2 && tiles(2, 2) > 256 && tiles(2, 2) <= 320) t.m = 1;
     if (inner >= (f32 ? 512 : 1024) && tiles(t.m, t.n) <= 256) t.split = 2;
     return t;
 }
 hipError_t launch_product(const ProductParams &p, int32_t dtype, const ProductTile &tile, hipStream_t st);
+
+// The gradient of a product's weight (product_grad.hip): x (rows, inner) transposed times g (rows, cols), both in 16
+// bits, as float slices (splits, inner, cols) of parts of the rows.
+struct GradParams {
+    const void *x, *g;
+    float *out;
+    int32_t rows, inner, cols, splits;
+};
+
+// The tile of the workgroups (128 columns of x by tile_n of g) and the number of parts of the rows; 0: the library's
+// product is not slower, or a size is not a whole number of 16-byte pieces.
+//
+// One round of workgroups, one to each of 256 compute units: a tile of 64 rows takes 0.66 us with 128 columns and
+// 0.88 with 192, the slices are written and read at 3.5 TB/s, and the sum of both is least. Measured (us, library
+// product with conversion / 128 columns / 192, with the best number of parts each, the rule's choice marked *):
+//   8192 rows   512 x 6144   111/83/71*     2048 x 512   57/33*/38    1024 x 3072  89/79/71*    256 x 1024  54/21*/24
+//   4096 rows   512 x 1536   31/24*/26      256 x 3072   32/22*/23    1024 x 3072  49/46/43*
+//   16384 rows  512 x 3072   153/79/73*     1024 x 8192  296/322/328
+//   2048 rows   512 x 3072   24/24/24       2048 x 512   20/19/22
+// More rows and smaller results are the library's worst (32768 rows, 512 x 512 157 -> 36; 16384 rows, 128 x 2048 130 ->
+// 25); where the rows are not split it is level or faster (4096 rows, 768 x 4096 47 / 50).
+struct GradPlan { int tile_n, splits; };
+// A call costs its host some 25 us more than torch's: taken from 8192 rows on, where the library loses more than that
+// (8192 rows, 256 x 256 50/16, 128 x 512 71/16; 16384 rows, 256 x 768 96/23), below where the products keep the GPU
+// busier than the host (from 3000 rows and 3e9 multiply-adds; 4096 rows, 256 x 1024 30/18 is left alone). More than 16
+// parts were no faster anywhere.
+constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384, kGradMaxResult = 1024 * 3072;
+inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {
+    if (rows < kGradMinRows || rows > (1 << 24) || inner > (1 << 16) || cols > (1 << 16) || inner < 128 || cols < 128 || inner % 8 != 0 || cols % 8 != 0 || inner * cols < kGradMinResult ||
+        inner * cols > kGradMaxResult || (rows < kGradManyRows && rows * inner * cols < kGradMinWork) || rows * inner >= (1 << 30) || rows * cols >= (1 << 30))   // (31-bit byte offsets)
+        return {0, 0};
+    GradPlan best{0, 0};
+    int64_t least = 0;
+    for (const int tile_n : {128, 192}) {
+        const int64_t tiles = (inner + 127) / 128 * ((cols + tile_n - 1) / tile_n);
+        for (int64_t splits = 1; splits == 1 || (splits <= 16 && tiles * splits <= 256 && splits * 256 <= rows); ++splits) {
+            const int64_t walk = ((rows + 63) / 64 + splits - 1) / splits * ((tiles * splits + 255) / 256) * (tile_n == 128 ? 660 : 880);   // ns
+            const int64_t cost = walk + splits * inner * cols * 8 / 3500;
+            if (best.splits == 0 || cost < least) best = GradPlan{tile_n, (int)splits}, least = cost;
+        }
+    }
+    return best.splits < 2 ? GradPlan{0, 0} : best;
+}
+// p.out: room for the slices; out: the result in out_dtype (float or the 16 bits of x and g)
+hipError_t launch_product_grad(const GradParams &p, const GradPlan &plan, bool half, int32_t out_dtype, void *out, hipStream_t st);
 
 }  // namespace sru_amd

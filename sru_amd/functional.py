@@ -337,6 +337,72 @@ def layer_forward(x: Tensor, residual: Tensor, weight_proj: Optional[Tensor], we
     return h, c_last
 
 
+@functools.lru_cache(maxsize=256)
+def _grad_workspace(dtype, rows, inner, cols):
+    return _lib.load().sru_amd_product_grad_workspace_bytes(_DTYPES[dtype], rows, inner, cols)
+
+
+def _observed() -> bool:
+    """Whether something records, transforms or compiles torch's calls: then a product is one of them."""
+    C = torch._C
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or C._len_torch_function_stack() > 0
+            or C._len_torch_dispatch_stack() > 0 or C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _weight_gradient(x: Tensor, grad: Tensor, dtype: torch.dtype) -> Tensor:
+    """x^T grad in `dtype`, summed in float."""
+    rows, inner, cols = x.size(0), x.size(1), grad.size(1)
+    if not (_plain(x) and _plain(grad) and x.dtype == grad.dtype and x.device == grad.device and x.is_contiguous()
+            and grad.is_contiguous() and x.data_ptr() % 16 == 0 and grad.data_ptr() % 16 == 0) or _observed():
+        return x.t().mm(grad).to(dtype)
+    nbytes = _grad_workspace(x.dtype, rows, inner, cols)
+    out = torch.empty(inner, cols, dtype=dtype, device=x.device)
+    workspace = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+    with _on_device(x.device) as stream:
+        rc = _lib.load().sru_amd_product_grad(_DTYPES[x.dtype], rows, inner, cols, _ptr(x), _ptr(grad), _DTYPES[dtype], _ptr(out),
+                                              _ptr(workspace), ctypes.c_size_t(nbytes), stream)
+    _lib.check(rc, "sru_amd_product_grad")
+    return out
+
+
+class _Product(Function):
+    """x.mm(narrow), `narrow` being `weight` in x's 16 bits; the weight's gradient by this package's kernel, straight in
+    the type of `weight` (None: that of x, and it is narrow's). Only x and narrow are kept, as mm keeps them."""
+
+    @staticmethod
+    def forward(ctx, x, narrow, weight):
+        ctx.save_for_backward(x, narrow)
+        ctx.weight_dtype = None if weight is None else weight.dtype
+        return x.mm(narrow)
+
+    @staticmethod
+    def backward(ctx, grad):
+        x, narrow = ctx.saved_tensors
+        grad_x = grad.mm(narrow.t()) if ctx.needs_input_grad[0] else None
+        if torch.is_grad_enabled():       # (to be differentiated again)
+            return grad_x, x.t().mm(grad), None
+        grad_w = _weight_gradient(x, grad, ctx.weight_dtype or narrow.dtype)
+        return (grad_x, grad_w, None) if ctx.weight_dtype is None else (grad_x, None, grad_w)
+
+
+def dense(x: Tensor, weight: Tensor) -> Tensor:
+    """x.mm(weight) as autocast makes it, by a kernel where that is the faster way: without gradients a short product in
+    float, with them the weight's gradient."""
+    autocast = torch.is_autocast_enabled("cuda")
+    if not torch.is_grad_enabled():
+        out = None if autocast or x.dtype != torch.float32 or _observed() else _lib.host().product(x, weight)
+        return x.mm(weight) if out is None else out
+    dtype = torch.get_autocast_dtype("cuda") if autocast else weight.dtype
+    if not (weight.requires_grad and dtype in _NARROW and x.is_cuda and weight.device == x.device
+            and x.dim() == 2 and weight.dim() == 2 and x.size(1) == weight.size(0) and _plain(x) and _plain(weight)
+            and (x.dtype in (torch.float32, *_NARROW) and weight.dtype in (torch.float32, dtype) if autocast else x.dtype == dtype)
+            and _grad_workspace(dtype, x.size(0), x.size(1), weight.size(1)) and not _observed()):
+        return x.mm(weight)
+    narrow = weight if weight.dtype == dtype else weight.to(dtype)
+    return _Product.apply(x.to(dtype), narrow, None if narrow is weight else weight)
+
+
 class ElementwiseRecurrence(Function):
     """Drop-in for sru/cuda_functional.py:156-261.
 

@@ -6,8 +6,8 @@ Constructor arguments, parameter / buffer names (`weight`, `weight_proj`, `weigh
 initialisation recipe and the forward semantics follow the reference, so a state_dict
 saved by it loads here and the same inputs give the same outputs. What differs is
 below the layer: the recurrence always runs the HIP kernels of this package, the projection
-is `torch.mm` (hipBLASLt) except where one kernel does both (`layer_forward`: 16-bit weights,
-no gradients); there is no CPU path (CPU tensors are refused).
+is `torch.mm` (hipBLASLt) except where kernels of this package are faster (`layer_forward`: 16-bit
+weights, no gradients; `dense`: short float products, weight gradients over many rows); there is no CPU path (CPU tensors are refused).
 """
 import copy
 import math
@@ -19,7 +19,7 @@ import torch.nn as nn
 from torch import Tensor
 from torch.nn.utils.rnn import PackedSequence, pad_packed_sequence, pack_padded_sequence
 
-from .functional import layer_forward
+from .functional import dense, layer_forward
 from .norm import layer_norm as fused_layer_norm, supported as fused_layer_norm_supported
 from .ops import elementwise_recurrence_gpu
 
@@ -162,8 +162,7 @@ class SRUCell(nn.Module):
         """Whether `layer_forward` may stand for compute_UV and apply_recurrence: nothing is
         differentiated or autocast, the layer projects with its own weights, no step is overridden (by a
         subclass, on the instance or on the class), and the input is a plain tensor that nothing records."""
-        return (not torch.is_grad_enabled() and self.custom_m is None
-                and input.dtype in (torch.float16, torch.bfloat16, torch.float32)
+        return (not torch.is_grad_enabled() and self.custom_m is None and input.dtype in (torch.float16, torch.bfloat16)
                 and getattr(self, "native_16bit", True) and type(input) is Tensor and type(residual) is Tensor
                 and getattr(self.compute_UV, "__func__", None) is _COMPUTE_UV
                 and getattr(self.compute_U, "__func__", None) is _COMPUTE_U
@@ -220,8 +219,8 @@ class SRUCell(nn.Module):
         """(length*batch, output_size*num_matrices): one dense GEMM (two with a projection)."""
         x = input if input.dim() == 2 else input.contiguous().view(-1, self.input_size)
         if self.weight_proj is not None:
-            x = x.mm(self.weight_proj)
-        return x.mm(self.weight)
+            x = dense(x, self.weight_proj)
+        return dense(x, self.weight)
 
     def _dropout_mask(self, size: Tuple[int, int], p: float) -> Tensor:
         return self.bias.new_empty(size).bernoulli_(1 - p).div_(1 - p)

@@ -255,3 +255,17 @@ def test_product_wanted(dtype, rows, inner, cols, taken):
 def _lib_status(name):
     header = open(os.path.join(ROOT, "include", "sru_amd.h")).read()
     return int(re.search(r"SRU_AMD_ERR_%s\s*=?\s*(\d+)" % name, header).group(1))
+
+
+@pytest.mark.parametrize("dtype,rows,inner,cols,taken", [
+    (_lib.BF16, 8192, 512, 6144, 1), (_lib.F16, 8192, 128, 384, 1), (_lib.F16, 3000, 512, 3072, 1), (_lib.F16, 4096, 256, 1024, 0), (_lib.F32, 8192, 512, 6144, 0), (_lib.BF16, 2999, 512, 6144, 0),
+    (_lib.BF16, 8192, 516, 6144, 0), (_lib.BF16, 8192, 512, 1540, 0), (_lib.BF16, 8192, 1032, 3072, 0), (_lib.BF16, 8192, 128, 376, 0),
+    (_lib.BF16, 1 << 20, 1024, 3072, 0), (_lib.BF16, 8192, -8, -8, 0), (_lib.BF16, 1 << 62, 1 << 62, 1 << 62, 0)])
+def test_product_grad_sizes(dtype, rows, inner, cols, taken):
+    lib = _lib.load()
+    assert (lib.sru_amd_product_grad_workspace_bytes(dtype, rows, inner, cols) > 0) == bool(taken)
+    rc = lib.sru_amd_product_grad(dtype, rows, inner, cols, FAKE, FAKE, dtype, None, None, 0, None)
+    assert lib.sru_amd_status_string(rc) == lib.sru_amd_status_string(_lib_status("NULL_POINTER" if taken else "BAD_SHAPE"))
+    if taken:
+        assert lib.sru_amd_product_grad(dtype, rows, inner, cols, FAKE, FAKE, dtype, FAKE, None, 0, None) == _lib_status("WORKSPACE")
+        assert lib.sru_amd_product_grad(dtype, rows, inner, cols, FAKE, FAKE, _lib.F64, FAKE, FAKE, 1 << 40, None) == _lib_status("BAD_DTYPE")
