@@ -386,21 +386,32 @@ class _Product(Function):
         return (grad_x, grad_w, None) if ctx.weight_dtype is None else (grad_x, None, grad_w)
 
 
+def _short_product(x: Tensor, weight: Tensor) -> Optional[Tensor]:
+    if x.dtype != torch.float32 or not x.is_cuda or torch.is_autocast_enabled("cuda") or _observed():
+        return None
+    return _lib.host().product(x, weight)
+
+
+def _product_for_gradients(x: Tensor, weight: Tensor) -> Optional[Tensor]:
+    # (the sizes as soon as they are numbers: they rule out the steps whose time is the host's)
+    if (not (_plain(x) and _plain(weight)) or torch.jit.is_tracing() or torch.compiler.is_compiling() or x.dim() != 2 or weight.dim() != 2
+            or not _grad_workspace(torch.bfloat16, x.size(0), x.size(1), weight.size(1))):
+        return None
+    autocast = torch.is_autocast_enabled("cuda")
+    dtype = torch.get_autocast_dtype("cuda") if autocast else weight.dtype
+    if not (weight.requires_grad and dtype in _NARROW and x.is_cuda and weight.device == x.device and x.size(1) == weight.size(0)
+            and (x.dtype in (torch.float32, *_NARROW) and weight.dtype in (torch.float32, dtype) if autocast else x.dtype == dtype)
+            and not _observed()):
+        return None
+    narrow = weight if weight.dtype == dtype else weight.to(dtype)
+    return _Product.apply(x.to(dtype), narrow, None if narrow is weight else weight)
+
+
 def dense(x: Tensor, weight: Tensor) -> Tensor:
     """x.mm(weight) as autocast makes it, by a kernel where that is the faster way: without gradients a short product in
     float, with them the weight's gradient."""
-    autocast = torch.is_autocast_enabled("cuda")
-    if not torch.is_grad_enabled():
-        out = None if autocast or x.dtype != torch.float32 or _observed() else _lib.host().product(x, weight)
-        return x.mm(weight) if out is None else out
-    dtype = torch.get_autocast_dtype("cuda") if autocast else weight.dtype
-    if not (weight.requires_grad and dtype in _NARROW and x.is_cuda and weight.device == x.device
-            and x.dim() == 2 and weight.dim() == 2 and x.size(1) == weight.size(0) and _plain(x) and _plain(weight)
-            and (x.dtype in (torch.float32, *_NARROW) and weight.dtype in (torch.float32, dtype) if autocast else x.dtype == dtype)
-            and _grad_workspace(dtype, x.size(0), x.size(1), weight.size(1)) and not _observed()):
-        return x.mm(weight)
-    narrow = weight if weight.dtype == dtype else weight.to(dtype)
-    return _Product.apply(x.to(dtype), narrow, None if narrow is weight else weight)
+    out = _product_for_gradients(x, weight) if torch.is_grad_enabled() else _short_product(x, weight)
+    return x.mm(weight) if out is None else out     # (in one place: a trace is compared with its repetition line by line)
 
 
 class ElementwiseRecurrence(Function):

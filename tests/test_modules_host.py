@@ -260,3 +260,11 @@ def test_flags_without_a_truth_value_are_refused_by_the_general_way(which):
     args[which] = torch.zeros(2)
     with pytest.raises(RuntimeError):      # (host tensors here; with device tensors the flag itself)
         elementwise_recurrence_forward(*args, keep_c=False)
+
+
+def test_a_layers_product_can_be_traced():
+    """With the tracer's own check, which repeats the call without gradients and compares line by line."""
+    from sru_amd.functional import dense
+    x, w = torch.randn(5000, 64), torch.randn(64, 192, requires_grad=True)
+    traced = torch.jit.trace(dense, (x, w))
+    assert torch.equal(traced(x[:7], w), x[:7] @ w)
