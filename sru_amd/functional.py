@@ -337,6 +337,9 @@ def layer_forward(x: Tensor, residual: Tensor, weight_proj: Optional[Tensor], we
     return h, c_last
 
 
+_GRAD_MIN_ROWS = 3000   # fewer rows are never taken (sru_amd_product_grad_workspace_bytes answers 0)
+
+
 @functools.lru_cache(maxsize=256)
 def _grad_workspace(dtype, rows, inner, cols):
     return _lib.load().sru_amd_product_grad_workspace_bytes(_DTYPES[dtype], rows, inner, cols)
@@ -393,9 +396,10 @@ def _short_product(x: Tensor, weight: Tensor) -> Optional[Tensor]:
 
 
 def _product_for_gradients(x: Tensor, weight: Tensor) -> Optional[Tensor]:
-    # (the sizes as soon as they are numbers: they rule out the steps whose time is the host's)
-    if (not (_plain(x) and _plain(weight)) or torch.jit.is_tracing() or torch.compiler.is_compiling() or x.dim() != 2 or weight.dim() != 2
-            or not _grad_workspace(torch.bfloat16, x.size(0), x.size(1), weight.size(1))):
+    # the sizes first: they rule out the steps whose time is the host's (while a trace is made they are no numbers)
+    shape = x.shape
+    if len(shape) != 2 or type(shape[0]) is not int or shape[0] < _GRAD_MIN_ROWS or not (_plain(x) and _plain(weight)) \
+            or weight.dim() != 2 or not _grad_workspace(torch.bfloat16, *shape, weight.size(1)):
         return None
     autocast = torch.is_autocast_enabled("cuda")
     dtype = torch.get_autocast_dtype("cuda") if autocast else weight.dtype
