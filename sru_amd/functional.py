@@ -369,6 +369,17 @@ def _weight_gradient(x: Tensor, grad: Tensor, dtype: torch.dtype) -> Tensor:
     return out
 
 
+def _asked_for(ctx, i: int) -> bool:
+    """Whether the backward pass that runs wants the gradient of input i. ctx.needs_input_grad says which inputs can have
+    one; torch.autograd.grad and backward(inputs=) may want fewer, and torch's own products leave the others out."""
+    if not ctx.needs_input_grad[i]:
+        return False
+    try:
+        return torch._C._will_engine_execute_node(ctx.next_functions[i][0])
+    except (RuntimeError, TypeError, AttributeError):   # a leaf that torch.autograd.grad wants; nothing to be asked
+        return True
+
+
 class _Product(Function):
     """x.mm(narrow), `narrow` being `weight` in x's 16 bits; the weight's gradient by this package's kernel, straight in
     the type of `weight` (None: that of x, and it is narrow's). Only x and narrow are kept, as mm keeps them."""
@@ -382,7 +393,9 @@ class _Product(Function):
     @staticmethod
     def backward(ctx, grad):
         x, narrow = ctx.saved_tensors
-        grad_x = grad.mm(narrow.t()) if ctx.needs_input_grad[0] else None
+        grad_x = grad.mm(narrow.t()) if _asked_for(ctx, 0) else None
+        if not _asked_for(ctx, 1 if ctx.weight_dtype is None else 2):
+            return grad_x, None, None
         if torch.is_grad_enabled():       # (to be differentiated again)
             return grad_x, x.t().mm(grad), None
         grad_w = _weight_gradient(x, grad, ctx.weight_dtype or narrow.dtype)

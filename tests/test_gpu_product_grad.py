@@ -134,3 +134,15 @@ def test_in_a_graph():
         graph.replay()
         replayed = out.clone()
         assert torch.equal(replayed, functional._weight_gradient(x, g, torch.float32))
+
+
+def test_the_inputs_gradient_alone(monkeypatch):
+    cell = SRUCell(512, 512).cuda().bfloat16()
+    x = torch.randn(260, 32, 512, device="cuda").bfloat16().requires_grad_()
+    calls, original = [], functional._weight_gradient
+    monkeypatch.setattr(functional, "_weight_gradient", lambda *a: calls.append(1) or original(*a))
+    h, _ = cell(x)
+    only, = torch.autograd.grad(h, x, torch.ones_like(h), retain_graph=True)
+    assert not calls
+    both = torch.autograd.grad(h, (x, cell.weight), torch.ones_like(h))
+    assert len(calls) == 1 and torch.equal(only, both[0])
