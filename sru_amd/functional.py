@@ -427,7 +427,10 @@ def _product_for_gradients(x: Tensor, weight: Tensor) -> Optional[Tensor]:
 def dense(x: Tensor, weight: Tensor) -> Tensor:
     """x.mm(weight) as autocast makes it, by a kernel where that is the faster way: without gradients a short product in
     float, with them the weight's gradient."""
-    out = _product_for_gradients(x, weight) if torch.is_grad_enabled() else _short_product(x, weight)
+    if torch.compiler.is_compiling():   # (before anything of this package: the compiler cannot follow into the library)
+        out = None
+    else:
+        out = _product_for_gradients(x, weight) if torch.is_grad_enabled() else _short_product(x, weight)
     return x.mm(weight) if out is None else out     # (in one place: a trace is compared with its repetition line by line)
 
 

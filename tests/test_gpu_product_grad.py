@@ -146,3 +146,13 @@ def test_the_inputs_gradient_alone(monkeypatch):
     assert not calls
     both = torch.autograd.grad(h, (x, cell.weight), torch.ones_like(h))
     assert len(calls) == 1 and torch.equal(only, both[0])
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("rows", [640, 8192])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_compiled_whole(dtype, rows, grad):
+    torch._dynamo.reset()
+    x, w = torch.randn(rows, 128, device="cuda").to(dtype), torch.randn(128, 384, device="cuda").to(dtype).requires_grad_()
+    with torch.set_grad_enabled(grad):
+        assert torch.equal(torch.compile(functional.dense, backend="eager", fullgraph=True)(x, w), x @ w)

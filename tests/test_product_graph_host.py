@@ -51,3 +51,12 @@ def test_gradients_that_nobody_asked_for_are_not_made(request_name, leaf, conver
         assert products_of_pass.count == products
     for a, b in zip(*got):
         assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("rows", [100, 5000])
+def test_a_product_is_compiled_whole(rows, grad):
+    torch._dynamo.reset()
+    x, w = torch.randn(rows, 64), torch.randn(64, 192, requires_grad=True)
+    with torch.set_grad_enabled(grad):
+        assert torch.equal(torch.compile(functional.dense, backend="eager", fullgraph=True)(x, w), x @ w)
