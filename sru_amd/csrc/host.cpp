@@ -13,6 +13,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -355,7 +356,22 @@ PyObject *float_product(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// autocast_operand(t) -> t as autocast hands it to a product: in the region's type, a parameter converted once in a region
+PyObject *autocast_operand(PyObject *, PyObject *o) {
+    HANDLE_TH_ERRORS
+    Arg t;
+    if (!read(o, t) || !t) return none();
+    at::Tensor out;
+    {
+        const Unlocked unlocked;
+        out = at::autocast::cached_cast(at::autocast::get_autocast_dtype(at::kCUDA), *t.t, at::kCUDA);
+    }
+    return wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"autocast_operand", autocast_operand, METH_O, nullptr},
     {"product", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(float_product)), METH_FASTCALL, nullptr},
     {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},
     {"scan_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_backward)), METH_FASTCALL, nullptr},

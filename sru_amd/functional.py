@@ -382,7 +382,8 @@ def _asked_for(ctx, i: int) -> bool:
 
 class _Product(Function):
     """x.mm(narrow), `narrow` being `weight` in x's 16 bits; the weight's gradient by this package's kernel, straight in
-    the type of `weight` (None: that of x, and it is narrow's). Only x and narrow are kept, as mm keeps them."""
+    the type of `weight` (None: that of x, and it is narrow's). Only x and narrow are kept, as mm keeps them. (A conversion
+    that autocast kept from a part of its region without gradients has no graph of its own to `weight`.)"""
 
     @staticmethod
     def forward(ctx, x, narrow, weight):
@@ -397,7 +398,8 @@ class _Product(Function):
         if not _asked_for(ctx, 1 if ctx.weight_dtype is None else 2):
             return grad_x, None, None
         if torch.is_grad_enabled():       # (to be differentiated again)
-            return grad_x, x.t().mm(grad), None
+            grad_w = x.t().mm(grad)
+            return (grad_x, grad_w, None) if ctx.needs_input_grad[1] else (grad_x, None, grad_w.to(ctx.weight_dtype))
         grad_w = _weight_gradient(x, grad, ctx.weight_dtype or narrow.dtype)
         return (grad_x, grad_w, None) if ctx.weight_dtype is None else (grad_x, None, grad_w)
 
@@ -406,6 +408,11 @@ def _short_product(x: Tensor, weight: Tensor) -> Optional[Tensor]:
     if x.dtype != torch.float32 or not x.is_cuda or torch.is_autocast_enabled("cuda") or _observed():
         return None
     return _lib.host().product(x, weight)
+
+
+def _autocast_operand(t: Tensor, dtype: torch.dtype) -> Tensor:
+    done = _lib.host().autocast_operand(t)
+    return t.to(dtype) if done is None else done
 
 
 def _product_for_gradients(x: Tensor, weight: Tensor) -> Optional[Tensor]:
@@ -420,8 +427,10 @@ def _product_for_gradients(x: Tensor, weight: Tensor) -> Optional[Tensor]:
             and (x.dtype in (torch.float32, *_NARROW) and weight.dtype in (torch.float32, dtype) if autocast else x.dtype == dtype)
             and not _observed()):
         return None
-    narrow = weight if weight.dtype == dtype else weight.to(dtype)
-    return _Product.apply(x.to(dtype), narrow, None if narrow is weight else weight)
+    if autocast:     # (its own conversions: those of parameters are kept for the region)
+        x, narrow = _autocast_operand(x, dtype), _autocast_operand(weight, dtype)
+        return _Product.apply(x, narrow, None if weight.dtype == dtype else weight)
+    return _Product.apply(x, weight, None)
 
 
 def dense(x: Tensor, weight: Tensor) -> Tensor:

@@ -156,3 +156,32 @@ def test_compiled_whole(dtype, rows, grad):
     x, w = torch.randn(rows, 128, device="cuda").to(dtype), torch.randn(128, 384, device="cuda").to(dtype).requires_grad_()
     with torch.set_grad_enabled(grad):
         assert torch.equal(torch.compile(functional.dense, backend="eager", fullgraph=True)(x, w), x @ w)
+
+
+def test_a_weight_is_converted_once_in_an_autocast_region():
+    x, w = torch.randn(8192, 512, device="cuda"), torch.randn(512, 512, device="cuda").requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        outs = [functional.dense(x, w) for _ in range(2)]
+        kept = [o.grad_fn.saved_tensors[1].data_ptr() for o in outs]
+        assert kept[0] == kept[1]
+        with torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=False):
+            other = functional.dense(x, w)
+            assert other.grad_fn.saved_tensors[1].data_ptr() != kept[0]
+    torch.autograd.backward(outs, [torch.ones_like(o) for o in outs])
+    twice, w.grad = w.grad, None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        functional.dense(x, w).backward(torch.ones_like(outs[0]))
+    assert torch.equal(twice, 2 * w.grad)
+
+
+@pytest.mark.parametrize("again", [False, True])
+def test_a_weight_converted_without_gradients_earlier_in_the_region(again):
+    x, w = torch.randn(8192, 512, device="cuda"), torch.randn(512, 512, device="cuda").requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        with torch.no_grad():
+            functional.dense(x, w)
+        out = functional.dense(x, w)
+    got, = torch.autograd.grad(out, w, torch.ones_like(out), create_graph=again)
+    want = x.bfloat16().double().t() @ torch.ones_like(out).double()
+    # a sum of 8192 rounded once to 16 bits, or none but its own float sums
+    assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * want.abs().max()).all()
