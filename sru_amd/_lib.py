@@ -104,6 +104,11 @@ class GeneralHost:
     autocast_operand = staticmethod(lambda t: None)
     layer_forward = staticmethod(lambda *args: False)
 
+    @staticmethod
+    def observed():
+        import torch
+        return torch._C._len_torch_function_stack() > 0 or torch._C._len_torch_dispatch_stack() > 0
+
 
 def host():
     """The native host code (csrc/host.cpp): calls in the plain case, from torch tensors to the C ABI. It

@@ -370,7 +370,14 @@ PyObject *autocast_operand(PyObject *, PyObject *o) {
     END_HANDLE_TH_ERRORS
 }
 
+PyObject *observed_now(PyObject *, PyObject *) {
+    HANDLE_TH_ERRORS
+    return PyBool_FromLong(observed());
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"observed", observed_now, METH_NOARGS, nullptr},
     {"autocast_operand", autocast_operand, METH_O, nullptr},
     {"product", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(float_product)), METH_FASTCALL, nullptr},
     {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},

@@ -347,10 +347,8 @@ def _grad_workspace(dtype, rows, inner, cols):
 
 def _observed() -> bool:
     """Whether something records, transforms or compiles torch's calls: then a product is one of them."""
-    C = torch._C
-    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or C._len_torch_function_stack() > 0
-            or C._len_torch_dispatch_stack() > 0 or C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0)
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or _lib.host().observed()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0)
 
 
 def _weight_gradient(x: Tensor, grad: Tensor, dtype: torch.dtype) -> Tensor:

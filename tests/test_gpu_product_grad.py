@@ -185,3 +185,12 @@ def test_a_weight_converted_without_gradients_earlier_in_the_region(again):
     want = x.bfloat16().double().t() @ torch.ones_like(out).double()
     # a sum of 8192 rounded once to 16 bits, or none but its own float sums
     assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * want.abs().max()).all()
+
+
+def test_a_default_device_changes_nothing():
+    x, w = torch.randn(8192, 512, device="cuda").bfloat16(), torch.randn(512, 512, device="cuda").bfloat16().requires_grad_()
+    floats = torch.randn(640, 128, device="cuda"), torch.randn(128, 384, device="cuda")
+    with torch.device("cuda"):
+        assert type(functional.dense(x, w).grad_fn).__name__ == "_ProductBackward"
+        with torch.no_grad():
+            assert functional._short_product(*floats) is not None

@@ -60,3 +60,20 @@ def test_a_product_is_compiled_whole(rows, grad):
     x, w = torch.randn(rows, 64), torch.randn(64, 192, requires_grad=True)
     with torch.set_grad_enabled(grad):
         assert torch.equal(torch.compile(functional.dense, backend="eager", fullgraph=True)(x, w), x @ w)
+
+
+def test_a_default_device_watches_nothing():
+    from torch.overrides import TorchFunctionMode
+    assert not functional._observed()
+    with torch.device("cpu"):
+        assert not functional._observed()
+        with CountProducts():
+            assert functional._observed()
+        with TorchFunctionMode():
+            assert functional._observed()
+    with torch.autograd.forward_ad.dual_level():
+        assert functional._observed()
+    seen = []
+    torch.func.vmap(lambda t: seen.append(functional._observed()) or t)(torch.zeros(2))
+    torch.jit.trace(lambda t: seen.append(functional._observed()) or t + 1, torch.zeros(2), check_trace=False)
+    assert seen == [True, True] and not functional._observed()
