@@ -207,23 +207,38 @@ hipError_t relay_forward(const FwdParams &p, hipStream_t st) {
 // Team kernel (sru_team.h): wavefronts of a workgroup share the walk of 64 columns. A workgroup keeps to one
 // direction of one batch row where at most a fifth of its lanes is left over: addresses and flags are scalar then,
 // and padding at the ends is not walked.
-// Taken while its wavefronts are resident together (two to a SIMD; beyond that the chunked kernels have wavefronts
-// enough to hide their chain), from the third chunk on; eight wavefronts while that leaves one workgroup to a compute
-// unit, else four. Measured (us, backward call with its 4 us reduction, the other kernels / this one; k = 3):
-//   bf16, 16 steps   8192 columns 7.1/7.6   32768 8.4/9.0       24 steps   8192 10.1/7.8   32768 11.4/9.5
-//   bf16, 256 steps  8192 33.6/18.9   16384 34.3/23.2   40960 57.2/51.0   49152 57.4/56.0   57344 61.2/64.7
-//   padded           40960 68.2/51.4   49152 67.1/58.9   57344 71.8/62.0
-//   bf16, 512 steps  2048 59.8/28.4   32768 71.8/64.7 (float x 85.7/73.2)
-//   f32, 32 steps    8192 9.9/8.1      256 steps  12288 41.7/27.0   20480 47.2/47.5   24576 48.3/50.8
-//   f32, 512 steps   2048 77.1/31.2   8192 77.6/40.2   16384 79.1/61.2 (padded 97.3/62.5)
-//   any 64 columns: d = 40, 256 steps, 10240 columns bf16 54.7/30.9
+// Eight wavefronts up to 128 workgroups, from the fifth chunk on; else four, up to where the kernels it stands before
+// are faster: those gain from more columns, while two of this one's wavefronts to a SIMD are 512 workgroups. Widths that
+// are not a multiple of 64 leave lanes over and split cache lines between workgroups, which memory minds the most: in long
+// walks without padding, and with a float x (not where the width is a multiple of 32: others there too are the slower
+// ones). A walk of few steps past its second chunk costs this kernel a whole chunk.
+// Measured (us, backward call with its 4 us reduction, the other kernels / this one; k = 3 and one direction if not said):
+//   bf16, d = 512   17 steps   8192 columns 9.3/7.6    32768 10.5/9.2    40960 10.0/12.3
+//                   64 steps   8192 13.4/9.2    32768 15.7/13.7   40960 19.3/18.5 (no skip term, padded 18.3/19.0)
+//                   96 steps   40960 25.8/23.7 (no skip term, padded 24.0/23.9)   49152 26.0/25.9 (k = 4 23.2/24.9)
+//                   256 steps  2048 33.4/18.0  32768 39.6/35.6   40960 55.3/49.5   49152 56.1/53.1 (k = 4, 128 steps 28.8/30.7)
+//   with a float x  256 steps  8192 44.1/17.9  32768 47.8/38.8   40960 48.1/52.9
+//   bf16, 400 steps d = 1000   25000 columns 80.9/70.8, 32000 78.1/85.8; padded, tanh, k = 4 84.1/60.0; float x 32000 67.9/92.2
+//                   d = 250    20000 columns with a float x 0.93 of the others' rate (d = 1014, 52 steps 18432 columns 16.4/13.9)
+//                   d = 96     20480 columns 0.93 of the others' rate; with a float x 32768 71.8/63.7
+//   bf16, 17 steps  d = 304    24320 columns padded, tanh, k = 4 10.3/10.7
+//   f32, d = 512    17 steps 16384 columns 7.9/7.8   64 steps 14.6/11.4   512 steps 77.9/55.1 (padded 96.0/60.9)
+//   f32, d = 250    17 steps 16000 columns 8.4/8.9   24 steps 9.0/9.3   64 steps 15.3/13.5   400 steps 61.5/64.5 (12000 61.0/47.9)
 inline bool team_by_row(int32_t d) { return (d + kBlock - 1) / kBlock * kBlock * 4 <= d * 5; }
 inline int64_t team_groups(int64_t ncols, int32_t d) {
     return team_by_row(d) ? ncols / d * ((d + kBlock - 1) / kBlock) : (ncols + kBlock - 1) / kBlock;
 }
-template <typename T> inline int team_waves(const BwdParams &p) {
+inline int team_waves(const BwdParams &p, bool narrow) {   // narrow: 16-bit streams
     const int64_t groups = team_groups(p.ncols, p.d), chunks = (p.L + kCkptInterval - 1) / kCkptInterval;
-    if (chunks < 3 || groups > (sizeof(T) == 4 ? 256 : p.pad ? 896 : 768)) return 1;
+    const bool whole = p.d % kBlock == 0, rows32 = p.d % 32 == 0;
+    if (p.L < (narrow || whole ? 17 : 18)) return 1;
+    int64_t most;
+    if (!narrow) most = whole || p.pad || p.L < 256 ? 256 : 224;
+    else if (whole) most = p.x_float || p.L <= 88 ? 512 : 640;
+    else if (p.L < 20) most = 256;
+    else if (p.x_float) most = rows32 ? 512 : 288;
+    else most = p.pad || p.L < (rows32 ? 64 : 128) ? 512 : rows32 ? 256 : 384;
+    if (groups > most) return 1;
     return groups <= 128 && chunks > 4 ? 8 : 4;
 }
 // X, STAGE, TX: as in fast_forward
@@ -286,13 +301,13 @@ hipError_t pick_backward(const sru_amd_shape &s, const BwdParams &p, hipStream_t
             if (p.x_float) {
                 if (p.act || !p.ckpt || !pair_ok<T, K>(s, {p.u, p.gu}, {p.gh}) || !aligned_to(p.x, 4) || !aligned_to(p.gx, 4))
                     return hipErrorInvalidValue;
-                if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP, 0, 1, float>(p, w, st);
+                if (const int w = team_waves(p, sizeof(T) == 2); w > 1) return team_backward<T, K, SKIP, 0, 1, float>(p, w, st);
                 if (p.ncols / 2 < kPairBelow) return fast_backward<T, K, SKIP, 1, kPair, 1, float>(p, st);
                 return fast_backward<T, K, SKIP, 2, 0, 1, float>(p, st);
             }
         }
         if (p.ckpt && pair_ok<T, K>(s, {p.u, p.gu}, {p.x, p.c, p.gh, p.gx}))
-            if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP>(p, w, st);
+            if (const int w = team_waves(p, sizeof(T) == 2); w > 1) return team_backward<T, K, SKIP>(p, w, st);
         if (p.ckpt && split_wanted(p.ncols, p.d) && all_aligned_16({p.u, p.x, p.gh, p.gu, p.gx}))
             return split_backward<T, K, SKIP>(p, st);
         if (!pair_ok<T, K>(s, {p.u, p.gu}, {p.x, p.c, p.gh, p.gx}))   // p.c is null with checkpoints
@@ -301,7 +316,7 @@ hipError_t pick_backward(const sru_amd_shape &s, const BwdParams &p, hipStream_t
         return fast_backward<T, K, SKIP, 2>(p, st);
     } else {
         if (p.ckpt)
-            if (const int w = team_waves<T>(p); w > 1) return team_backward<T, K, SKIP>(p, w, st);
+            if (const int w = team_waves(p, sizeof(T) == 2); w > 1) return team_backward<T, K, SKIP>(p, w, st);
         return fast_backward<T, K, SKIP, 1>(p, st);
     }
 }

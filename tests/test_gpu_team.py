@@ -74,3 +74,33 @@ def test_factors_beyond_the_float_range(L, d):
     # (a gate is within 1e-7, relative to 1 - g1 = 0.12: 1e-6)
     assert ((gu[0].double() - expect).abs() <= 2e-6 * expect.abs()).all()
     assert (gwc == 0).all() and gbias.isfinite().all()
+
+
+# (streams, steps, rows, d, options, taken): both sides of each line of the rule, beyond which other kernels are the faster ones
+LINES = [
+    ("bf16", 16, 4, 512, {}, False), ("bf16", 17, 4, 512, {}, True), ("bf16", 24, 64, 512, {}, True), ("bf16", 24, 65, 512, {}, False),
+    ("f16", 89, 80, 512, {}, True), ("f16", 89, 81, 512, {}, False), ("bf16", 88, 80, 512, {}, False), ("bf16", 89, 80, 512, dict(x_f32=True), False),
+    ("bf16", 19, 52, 304, {}, False), ("bf16", 20, 52, 304, {}, True), ("bf16", 127, 102, 304, {}, True), ("bf16", 127, 103, 304, {}, False),
+    ("bf16", 128, 76, 304, {}, True), ("bf16", 128, 77, 304, {}, False), ("bf16", 128, 102, 304, dict(pad=True), True), ("bf16", 128, 103, 304, dict(pad=True), False),
+    ("bf16", 64, 85, 160, {}, True), ("bf16", 64, 86, 160, {}, False), ("bf16", 63, 170, 160, {}, True), ("bf16", 40, 57, 304, dict(x_f32=True), True),
+    ("bf16", 40, 58, 304, dict(x_f32=True), False), ("bf16", 40, 170, 160, dict(x_f32=True), True), ("bf16", 40, 171, 160, dict(x_f32=True), False),
+    ("f32", 17, 32, 512, {}, True), ("f32", 17, 33, 512, {}, False), ("f32", 17, 4, 250, {}, False), ("f32", 18, 64, 250, {}, True),
+    ("f32", 256, 56, 250, {}, True), ("f32", 256, 57, 250, {}, False), ("f32", 256, 64, 250, dict(pad=True), True), ("f32", 256, 65, 250, dict(pad=True), False),
+]
+
+
+@pytest.mark.parametrize("dt,L,B,d,kw,taken", LINES, ids=lambda v: "-".join(v) if isinstance(v, dict) else str(v))
+def test_where_it_is_taken(dt, L, B, d, kw, taken):
+    from torch.profiler import ProfilerActivity, profile
+    t = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dt]
+    leaf = lambda *size, dtype=t: torch.randn(*size, device="cuda", dtype=dtype).requires_grad_()
+    u, x = leaf(L, B, 3 * d), leaf(L, B, d, dtype=torch.float32 if "x_f32" in kw else t)
+    wc, bias = leaf(2 * d, dtype=torch.float32), leaf(2 * d, dtype=torch.float32)
+    pad = torch.zeros(L, B, dtype=torch.bool, device="cuda") if "pad" in kw else None
+    h, _ = sru_amd.ElementwiseRecurrence.apply(u, x, wc, bias, None, 0, d, False, True, None, None, pad)
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        torch.autograd.grad(h, (u, x, wc, bias), torch.ones_like(h))
+        torch.cuda.synchronize()
+    scans = [e.name for e in seen.events() if "backward_scan" in e.name]
+    assert len(scans) == 1 and ("backward_scan_team" in scans[0]) == taken, scans
