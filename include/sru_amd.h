@@ -260,8 +260,9 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
 
 /* A dense product, out (rows, cols) = x (rows, inner) weight (inner, cols), all row-major in `dtype` (float, or 16
  * bits with float sums) and 16-byte aligned: compute_U of a short sequence or a prompt (sru/modules.py:252-274,
- * a library call there). sru_amd_product_wanted says whether the kernel takes a problem (a library product is
- * faster for the others, or a size is not a multiple of 4 or 8); sru_amd_product answers BAD_SHAPE otherwise. */
+ * a library call there). sru_amd_product_wanted says whether the kernel is the better choice for a problem (a library
+ * product is faster for the others); sru_amd_product takes larger ones as well, and answers BAD_SHAPE where there is no
+ * kernel: past 1.75e9 multiply-adds, or where a size is not a multiple of 4 or 8. */
 int sru_amd_product_wanted(int32_t dtype, int64_t rows, int64_t inner, int64_t cols);
 int sru_amd_product(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *weight, void *out, void *stream);
 

@@ -347,15 +347,17 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
 }
 
 int sru_amd_product_wanted(int32_t dtype, int64_t rows, int64_t inner, int64_t cols) {
-    return (dtype == SRU_AMD_F32 || dtype == SRU_AMD_F16 || dtype == SRU_AMD_BF16) && product_tile((int)elem_size(dtype), rows, inner, cols).m != 0;
+    return (dtype == SRU_AMD_F32 || dtype == SRU_AMD_F16 || dtype == SRU_AMD_BF16) && product_wanted((int)elem_size(dtype), rows, inner, cols);
 }
 
 int sru_amd_product(int32_t dtype, int64_t rows, int64_t inner, int64_t cols, const void *x, const void *weight, void *out, void *stream) {
-    if (!sru_amd_product_wanted(dtype, rows, inner, cols)) return SRU_AMD_ERR_BAD_SHAPE;
+    if (dtype != SRU_AMD_F32 && dtype != SRU_AMD_F16 && dtype != SRU_AMD_BF16) return SRU_AMD_ERR_BAD_SHAPE;
+    const ProductTile tile = product_tile((int)elem_size(dtype), rows, inner, cols);
+    if (tile.m == 0) return SRU_AMD_ERR_BAD_SHAPE;
     if (!x || !weight || !out) return SRU_AMD_ERR_NULL_POINTER;
     if (!aligned(x, 16) || !aligned(weight, 16) || !aligned(out, 16)) return SRU_AMD_ERR_MISALIGNED;
     const ProductParams p{x, weight, out, (int32_t)rows, (int32_t)inner, (int32_t)cols};
-    const hipError_t err = launch_product(p, dtype, product_tile((int)elem_size(dtype), rows, inner, cols), static_cast<hipStream_t>(stream));
+    const hipError_t err = launch_product(p, dtype, tile, static_cast<hipStream_t>(stream));
     return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
 }
 

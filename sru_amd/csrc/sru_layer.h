@@ -102,22 +102,21 @@ struct ProductParams {
 };
 
 // The tile of a product's workgroups, 32 rows x 32 columns at the least, and whether they split the inner dimension
-// in two; none where the library's product is faster or a size is not a whole number of 16-byte pieces.
+// in two; none where a size is not a whole number of 16-byte pieces or the library's product is the faster one by far.
 //
 // Larger tiles read less, smaller ones leave a workgroup for more compute units: a larger one is taken from about
 // three workgroups to four compute units on (float, whose tiles take four times as long in the matrix cores, from
-// three workgroups to a unit), unless that is just one round of them and a little of another, of many
-// inner indices each (bf16 200 x 1536 -> 4608, 288 workgroups: 17.8 us, 32 x 64 tiles 14.0, library 15.0). Two halves of the inner dimension where it is long and compute units are left over.
+// three workgroups to a unit), unless that is just one round of them and a little of another, of many inner indices
+// each: tiles of 32 x 64 then are two rounds (bf16 200 x 1024 -> 4416, 276 workgroups 12.7 us, 32 x 64 tiles 10.1, library 11.5;
+// 136 x 1792 -> 5632 19.4, 16.8, 17.3) or more, and level. Two halves of the inner dimension where it is long and compute units are left over.
 // Measured (us in a graph, library / 32 x 32 / 32 x 64 / 64 x 64, the rule's choice marked *, with "2" where split):
 //   bf16   33 x 256 -> 768      4.5/3.1*/3.6/3.9      128 x 256 -> 3072    6.7/4.0/3.8*/4.4    512 x 512 -> 6144   12.9/17.1/13.4/11.3*
 //          128 x 1024 -> 256    10.5/4.8*2/6.3/7.4    512 x 2048 -> 512   10.8/8.8*2/10.3/12.6 128 x 2048 -> 6144  18.8/17.7/16.1/13.1*2
 //   f32    640 x 128 -> 384     4.3/3.4*/4.3/5.6      2048 x 256 -> 768   22.3/12.3/12.2*/14.0 1024 x 256 -> 3072  24.7/21.0/19.6/18.9*
 // Past 1.75e9 multiply-adds the library is faster (bf16 512 x 2048 -> 6144 26.4/30.5, 1024 x 512 -> 6144
-// 16.3/18.8, 2048 x 1024 -> 3072 21.9/30.8); below, 2048 x 256 -> 3072 (12.0/12.4) is the worst of those measured.
-// In float it is faster too where the inner dimension is long (128 x 2048 -> 512 10.0/14.3, 64 x 1536 -> 4608
-// 17.2/18.8) or longer than the result is wide (512 x 1024 -> 256 8.9/9.3); below 64 inner indices or columns it is not measured.
-// Launched one by one a library product costs
-// its caller 18 us, and this one 4.
+// 16.3/18.8, 2048 x 1024 -> 3072 21.9/30.8). In float it is faster too where the inner dimension is long (128 x 2048 -> 512
+// 10.0/14.3, 64 x 1536 -> 4608 17.2/18.8) or longer than the result is wide (512 x 1024 -> 256 8.9/9.3); below 64 inner
+// indices or columns it is not measured.
 struct ProductTile { int m, n, split; };   // in units of 32; m 0: none
 inline ProductTile product_tile(int size, int64_t rows, int64_t inner, int64_t cols) {
     const bool f32 = size == 4;
@@ -129,6 +128,17 @@ inline ProductTile product_tile(int size, int64_t rows, int64_t inner, int64_t c
     if (!f32 && inner >= 1024 && t.m == 2 && tiles(2, 2) > 256 && tiles(2, 2) <= 320) t.m = 1;
     if (inner >= (f32 ? 512 : 1024) && tiles(t.m, t.n) <= 256) t.split = 2;
     return t;
+}
+// Whether a layer's product is made by the kernel: up to where, over sizes drawn at random, its time in a graph is still the
+// shorter one on average. In 16 bits that is a matter of the result's size, the sooner the more inner indices there are:
+// 375 sizes on this side 0.77 of the library's time, the worst 1.30 (4502 x 320 -> 768 9.6/12.5); 196 beyond level, the worst
+// 1.66 (777 x 640 -> 1920 9.6/10.5, 3007 x 128 -> 3584 12.1/17.1). In float it is one of work at more than 384 inner indices:
+// 216 sizes 0.78, the worst 1.26 (2855 x 512 -> 384 15.9/20.0), beyond 1.03 and 1.35. Launched one by one a library product
+// costs its caller 18 us, and this one 4, which is why the line lies no lower.
+inline bool product_wanted(int size, int64_t rows, int64_t inner, int64_t cols) {
+    if (product_tile(size, rows, inner, cols).m == 0) return false;
+    if (size == 4) return inner <= 384 || rows * inner * cols <= 600000000;
+    return rows * cols <= (inner <= 512 ? 3500000 : 1000000);
 }
 hipError_t launch_product(const ProductParams &p, int32_t dtype, const ProductTile &tile, hipStream_t st);
 

@@ -252,6 +252,16 @@ def test_product_wanted(dtype, rows, inner, cols, taken):
     assert text == lib.sru_amd_status_string(_lib_status("NULL_POINTER" if taken else "BAD_SHAPE"))
 
 
+@pytest.mark.parametrize("dtype,rows,inner,cols,wanted", [
+    (_lib.BF16, 512, 512, 6144, 1), (_lib.BF16, 1000, 256, 3500, 1), (_lib.BF16, 1001, 256, 3500, 0), (_lib.F16, 3007, 128, 3584, 0),
+    (_lib.BF16, 1000, 520, 1000, 1), (_lib.BF16, 1001, 520, 1000, 0), (_lib.BF16, 777, 640, 1920, 0), (_lib.F32, 2000, 384, 1000, 1),
+    (_lib.F32, 500, 500, 2400, 1), (_lib.F32, 501, 500, 2400, 0)])
+def test_a_product_may_be_taken_and_not_wanted(dtype, rows, inner, cols, wanted):
+    lib = _lib.load()
+    assert lib.sru_amd_product_wanted(dtype, rows, inner, cols) == wanted
+    assert lib.sru_amd_product(dtype, rows, inner, cols, None, None, None, None) == _lib_status("NULL_POINTER")
+
+
 def _lib_status(name):
     header = open(os.path.join(ROOT, "include", "sru_amd.h")).read()
     return int(re.search(r"SRU_AMD_ERR_%s\s*=?\s*(\d+)" % name, header).group(1))
