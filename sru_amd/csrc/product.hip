@@ -228,8 +228,10 @@ template <typename T, int TM, int TN, int G> hipError_t launch(const ProductPara
                            dim3(kGroupThreads * G), args, 0, st);
 }
 template <typename T> hipError_t product_of(const ProductParams &p, const ProductTile &t, hipStream_t st) {
-    if (t.m == 2) return t.split == 2 ? launch<T, 2, 2, 2>(p, st) : launch<T, 2, 2, 1>(p, st);
-    if (t.n == 2) return t.split == 2 ? launch<T, 1, 2, 2>(p, st) : launch<T, 1, 2, 1>(p, st);
+    if constexpr (sizeof(T) == 2) {   // (in float larger tiles come with more workgroups than a split wants)
+        if (t.split == 2 && t.n == 2) return t.m == 2 ? launch<T, 2, 2, 2>(p, st) : launch<T, 1, 2, 2>(p, st);
+    }
+    if (t.n == 2) return t.m == 2 ? launch<T, 2, 2, 1>(p, st) : launch<T, 1, 2, 1>(p, st);
     return t.split == 2 ? launch<T, 1, 1, 2>(p, st) : launch<T, 1, 1, 1>(p, st);
 }
 

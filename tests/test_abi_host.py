@@ -279,3 +279,12 @@ def test_product_grad_sizes(dtype, rows, inner, cols, taken):
     if taken:
         assert lib.sru_amd_product_grad(dtype, rows, inner, cols, FAKE, FAKE, dtype, FAKE, None, 0, None) == _lib_status("WORKSPACE")
         assert lib.sru_amd_product_grad(dtype, rows, inner, cols, FAKE, FAKE, _lib.F64, FAKE, FAKE, 1 << 40, None) == _lib_status("BAD_DTYPE")
+
+
+def test_every_product_kernel_in_the_library_can_be_chosen():
+    # (rows and columns of the tile in 32, parts of the inner dimension; float splits small tiles only: larger ones start
+    # at 384 workgroups, and a split wants at most 256)
+    built = set(re.findall(rb"product_tileI(f|NS_9bf16_bitsE|NS_9half_bitsE)Li(\d)ELi(\d)ELi(\d)EEEvNS_13ProductParamsE", open(_lib.LIB_PATH, "rb").read()))
+    tiles = {(1, 1, 1), (1, 1, 2), (1, 2, 1), (2, 2, 1)}
+    for name, chosen in ((b"f", tiles), (b"NS_9bf16_bitsE", tiles | {(1, 2, 2), (2, 2, 2)}), (b"NS_9half_bitsE", tiles | {(1, 2, 2), (2, 2, 2)})):
+        assert {tuple(map(int, b[1:])) for b in built if b[0] == name} == chosen
