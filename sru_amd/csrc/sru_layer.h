@@ -167,10 +167,10 @@ struct GradPlan { int tile_n, splits; };
 // (8192 rows, 256 x 256 50/16, 128 x 512 71/16; 16384 rows, 256 x 768 96/23), below where the products keep the GPU
 // busier than the host (from 3000 rows and 3e9 multiply-adds; 4096 rows, 256 x 1024 30/18 is left alone). More than 16
 // parts were no faster anywhere.
-constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384, kGradMaxResult = 1024 * 3072;
+constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384;
 inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {
     if (rows < kGradMinRows || rows > (1 << 24) || inner > (1 << 16) || cols > (1 << 16) || inner < 128 || cols < 128 || inner % 8 != 0 || cols % 8 != 0 || inner * cols < kGradMinResult ||
-        inner * cols > kGradMaxResult || (rows < kGradManyRows && rows * inner * cols < kGradMinWork) || rows * inner >= (1 << 30) || rows * cols >= (1 << 30))   // (31-bit byte offsets)
+        (rows < kGradManyRows && rows * inner * cols < kGradMinWork) || rows * inner >= (1 << 30) || rows * cols >= (1 << 30))   // (31-bit byte offsets)
         return {0, 0};
     GradPlan best{0, 0};
     int64_t least = 0;
@@ -182,7 +182,7 @@ inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {
             if (best.splits == 0 || cost < least) best = GradPlan{tile_n, (int)splits}, least = cost;
         }
     }
-    return best.splits < 2 ? GradPlan{0, 0} : best;
+    return best.splits < 2 ? GradPlan{0, 0} : best;   // (no two parts of a result beyond 128 tiles of 128 x 192 fit a round)
 }
 // p.out: room for the slices; out: the result in out_dtype (float or the 16 bits of x and g)
 hipError_t launch_product_grad(const GradParams &p, const GradPlan &plan, bool half, int32_t out_dtype, void *out, hipStream_t st);
