@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from sru_amd import SRU, SRUCell, _lib, modules
+from tests.test_abi_host import _lib_status
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +19,10 @@ SIZES = [(1, 8, 4), (31, 24, 36), (33, 64, 100), (65, 72, 132), (7, 1032, 36), (
          (160, 200, 2500), (97, 264, 3204), (513, 256, 1404), (705, 264, 1092), (96, 1096, 4100), (1600, 136, 2052), (64, 3000, 64)]
 
 
+# those of SIZES that float has no kernel for: few inner indices or columns, or many inner indices for the result's width
+NO_FLOAT = [(1, 8, 4), (31, 24, 36), (7, 1032, 36), (130, 520, 68), (40, 1088, 64), (96, 1096, 4100), (64, 3000, 64)]
+
+
 @pytest.mark.parametrize("dtype", list(CODE))
 @pytest.mark.parametrize("rows,inner,cols", SIZES)
 def test_product(rows, inner, cols, dtype):
@@ -27,15 +32,47 @@ def test_product(rows, inner, cols, dtype):
     out = torch.full((rows + 1, cols), float("nan"), device="cuda", dtype=dtype)   # (a row behind it, to stay as it is)
     xd, wd = x.cuda(), w.cuda()
     p = lambda t: ctypes.c_void_p(t.data_ptr())
-    if not lib.sru_amd_product_wanted(CODE[dtype], rows, inner, cols):
-        assert dtype == torch.float32 and (inner > 512 or inner < 64 or cols < 64)
+    rc = lib.sru_amd_product(CODE[dtype], rows, inner, cols, p(xd), p(wd), p(out), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    if dtype == torch.float32 and (rows, inner, cols) in NO_FLOAT:
+        assert lib.sru_amd_status_string(rc) == lib.sru_amd_status_string(_lib_status("BAD_SHAPE")) and torch.isnan(out).all()
         return
-    assert lib.sru_amd_product(CODE[dtype], rows, inner, cols, p(xd), p(wd), p(out), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert rc == 0
     got = out.cpu()
     assert torch.isnan(got[rows]).all()
     want = x.double() @ w.double()
     # float sums of `inner` terms, then the result's rounding
     bound = inner * 2.0 ** -24 * (x.double().abs() @ w.double().abs()) + HALF_ULP[dtype] * want.abs() + 2.0 ** -24
+    assert ((got[:rows].double() - want).abs() <= bound).all()
+
+
+# (type, rows, inner, cols, rows and columns of the tile in 32, parts of the inner dimension): every kernel, cut off at its edges
+TILES = [(torch.float32, 33, 72, 100, (1, 1, 1)), (torch.float32, 128, 512, 1536, (1, 1, 2)), (torch.float32, 33, 1020, 2052, (1, 1, 2)),
+         (torch.float32, 705, 264, 1092, (1, 2, 1)), (torch.float32, 1601, 136, 2052, (2, 2, 1)),
+         (torch.bfloat16, 31, 24, 36, (1, 1, 1)), (torch.bfloat16, 40, 1088, 68, (1, 1, 2)), (torch.bfloat16, 97, 264, 3204, (1, 2, 1)),
+         (torch.float16, 62, 1544, 7684, (1, 2, 2)), (torch.bfloat16, 62, 1544, 7684, (1, 2, 2)), (torch.bfloat16, 513, 256, 1404, (2, 2, 1)),
+         (torch.float16, 127, 2056, 6100, (2, 2, 2)), (torch.bfloat16, 127, 2056, 6100, (2, 2, 2)),
+         (torch.bfloat16, 199, 1544, 4604, (1, 2, 1))]     # (288 tiles of 64 x 64: two rounds of smaller ones instead)
+
+
+@pytest.mark.parametrize("dtype,rows,inner,cols,tile", TILES)
+def test_every_tile(dtype, rows, inner, cols, tile):
+    from torch.profiler import ProfilerActivity, profile
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(rows)
+    x, w = torch.randn(rows, inner, generator=g).to(dtype), torch.randn(inner, cols, generator=g).to(dtype)
+    out, xd, wd = torch.full((rows + 1, cols), float("nan"), device="cuda", dtype=dtype), x.cuda(), w.cuda()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        assert lib.sru_amd_product(CODE[dtype], rows, inner, cols, p(xd), p(wd), p(out), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+    name = {torch.float32: "float", torch.float16: "sru_amd::half_bits", torch.bfloat16: "sru_amd::bf16_bits"}[dtype]
+    kernels = [e.name for e in seen.events() if "product_tile<" in e.name]
+    assert len(kernels) == 1 and "product_tile<%s, %d, %d, %d>" % (name, *tile) in kernels[0]
+    got = out.cpu()
+    assert torch.isnan(got[rows]).all()
+    want = x.double() @ w.double()
+    bound = inner * 2.0 ** -24 * (x.double().abs() @ w.double().abs()) + HALF_ULP[dtype] * want.abs() + 2.0 ** -24   # (as above)
     assert ((got[:rows].double() - want).abs() <= bound).all()
 
 

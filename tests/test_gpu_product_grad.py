@@ -4,6 +4,7 @@ import ctypes
 
 import pytest
 import torch
+from torch.profiler import ProfilerActivity, profile
 
 from sru_amd import SRUCell, _lib, functional
 
@@ -14,7 +15,8 @@ HALF_ULP = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16
 # (rows, inner, cols): both tiles, whole and cut off at either edge, rows with a remainder of one piece and of none, walks
 # of uneven parts down to four tiles of rows
 SIZES = [(4096, 512, 1536), (8193, 128, 2048), (8255, 136, 2056), (8256, 520, 1000), (8200, 264, 1032), (5000, 1024, 2880), (8196, 2048, 128),
-         (3000, 512, 3072), (8192, 128, 384)]
+         (3000, 512, 3072), (8192, 128, 384), (6000, 1000, 3000), (8196, 456, 6008)]
+WIDE = [(5000, 1024, 2880), (6000, 1000, 3000), (8196, 456, 6008)]    # in tiles of 192 columns
 
 
 @pytest.mark.parametrize("out", [torch.float32, "narrow"])
@@ -30,9 +32,14 @@ def test_gradient(rows, inner, cols, dtype, out):
     assert nbytes > 0 and nbytes % (4 * inner * cols) == 0
     work = torch.full((nbytes // 4 + 64,), float("nan"), device="cuda")
     got = torch.full((inner + 1, cols), float("nan"), device="cuda", dtype=out)
-    rc = lib.sru_amd_product_grad(CODE[dtype], rows, inner, cols, p(xd), p(gd), CODE[out], p(got), p(work), ctypes.c_size_t(nbytes),
-                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        rc = lib.sru_amd_product_grad(CODE[dtype], rows, inner, cols, p(xd), p(gd), CODE[out], p(got), p(work), ctypes.c_size_t(nbytes),
+                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
     assert rc == 0
+    kernels = [e.name for e in seen.events() if "product_grad<" in e.name]
+    assert len(kernels) == 1 and ("_bits, 3>" in kernels[0]) == ((rows, inner, cols) in WIDE)
     assert torch.isnan(got[inner]).all() and torch.isnan(work[nbytes // 4:]).all()
     want = x.double().t() @ g.double()
     # float sums of `rows` terms whose rounding errors are independent (ten deviations), then the result's rounding

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import sru_amd
+from tests.abi import DeviceProblem
 from tests.cases import Case
 from tests.test_gpu_parity import check_against_oracle
 
@@ -60,3 +61,19 @@ def test_padding_is_not_touched_by_what_it_holds(dtype):
     assert torch.equal(last.nan_to_num(nan=7.0), last0.nan_to_num(nan=7.0))
     assert (h[pad] == 0).all()
     assert np.array_equal(last[2].float().numpy(), c0[2].to(last.dtype).float().numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("B", [256, 257])
+def test_column_limit(B, dt):
+    # the last 64 columns that it takes, and a batch row more, which the other kernels take
+    from torch.profiler import ProfilerActivity, profile
+    case = Case(L=130, B=B, d=64, seed=34)
+    check_against_oracle(case, dt, keep_c=False)
+    dp = DeviceProblem(case, dt, checkpointed=True)
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        dp.forward()
+        torch.cuda.synchronize()
+    scans = [e.name for e in seen.events() if "forward_scan" in e.name]
+    assert len(scans) == 1 and ("forward_scan_relay" in scans[0]) == (B == 256)

@@ -104,3 +104,56 @@ def test_where_it_is_taken(dt, L, B, d, kw, taken):
         torch.cuda.synchronize()
     scans = [e.name for e in seen.events() if "backward_scan" in e.name]
     assert len(scans) == 1 and ("backward_scan_team" in scans[0]) == taken, scans
+
+
+# walks of several chunks past those lines: lane pairs on registers and on row tiles, one column per lane
+PAST = [("bf16", dict(L=25, B=641, d=64, pad="right", scale=1.7), {}), ("f16", dict(L=41, B=641, d=64, k=4, act=1), {}),
+        ("bf16", dict(L=33, B=641, d=64, skip=False, pad="random"), {}), ("bf16", dict(L=27, B=330, d=70, dirs=2, mask_c=True), {}),
+        ("bf16", dict(L=25, B=641, d=64, pad="right", scale=1.3), dict(x_f32=True)), ("f16", dict(L=40, B=290, d=70), dict(x_f32=True)),
+        ("bf16", dict(L=67, B=110, d=160), {}), ("f16", dict(L=72, B=110, d=160, k=4, act=1, mask_c=True), {}),
+        ("bf16", dict(L=64, B=220, d=80, dirs=2, skip=False, pad="random"), {}), ("f32", dict(L=41, B=257, d=64, k=4, act=1, pad="right"), {}),
+        ("f32", dict(L=25, B=130, d=64, dirs=2, skip=False, mask_c=True), {})]
+
+
+@pytest.mark.parametrize("dt,cfg,kw", PAST, ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) if isinstance(v, dict) else v)
+def test_the_kernels_past_the_lines(dt, cfg, kw):
+    check_against_oracle(Case(seed=44, **cfg), dt, checkpointed=True, **kw)
+
+
+@pytest.mark.parametrize("L,B,d", [(32, 2, 24), (100, 2, 24), (100, 2, 64), (100, 130, 64)])   # teams of 4, 8, 8, 4; up to 4 rounds
+def test_gradients_beside_factors_beyond_the_float_range(L, B, d):
+    # Every fifth column as in the test above; it has the whole wavefront hand its gradients on step by step. The other
+    # columns have ordinary factors, a gradient of every output and of the last state, and 64-bit results.
+    gen = np.random.default_rng(6)
+    hot = np.arange(d) % 5 == 2
+    u = gen.standard_normal((L, B, d, 3)).astype(np.float32)
+    wc, bias = gen.uniform(-1.2, 1.2, (2, d)).astype(np.float32), (0.5 * gen.standard_normal((2, d))).astype(np.float32)
+    wc[:, hot], bias[:, hot] = 1.0, 0.0
+    c = np.zeros((B, d), np.float32)
+    for t in range(L):
+        h0 = 4e6 * (-1) ** t * (1 + 0.1 * gen.random((B, d)))
+        u[t][:, hot, 0], u[t][:, hot, 1] = h0[:, hot], 2.0 - c[:, hot]
+        g = 1 / (1 + np.exp(-(u[t, ..., 1].astype(np.float64) + wc[0] * c + bias[0])))
+        c = ((c - u[t, ..., 0]) * g + u[t, ..., 0]).astype(np.float32)
+    gh, gl = gen.standard_normal((L, B, d)).astype(np.float32), gen.standard_normal((B, d)).astype(np.float32)
+    gh[1:, :, hot], gl[:, hot] = 0.0, 0.0
+    x = gen.standard_normal((L, B, d)).astype(np.float32)
+    leaf = lambda a, kind: torch.tensor(a).to(kind).requires_grad_()
+    U, X, W, b = (leaf(a, torch.float32).detach().cuda().requires_grad_() for a in (u.reshape(L, B, 3 * d), x, wc.reshape(-1), bias.reshape(-1)))
+    outs = sru_amd.ElementwiseRecurrence.apply(U, X, W, b, None, 0, d, False, True, None, None, None)
+    got = [t.cpu().double() for t in torch.autograd.grad(outs, (U, X, W, b), (torch.tensor(gh).cuda(), torch.tensor(gl).cuda()))]
+    got = got[0].view(L, B, d, 3), got[1], got[2].view(2, d), got[3].view(2, d)
+    assert (got[0][1:, :, hot] == 0).all() and (got[1][1:, :, hot] == 0).all() and all(t.isfinite().all() for t in got)
+
+    cold = torch.tensor(~hot)
+    U, X, W, b = leaf(u[:, :, ~hot], torch.float64), leaf(x[:, :, ~hot], torch.float64), leaf(wc[:, ~hot], torch.float64), leaf(bias[:, ~hot], torch.float64)
+    state, h = torch.zeros(B, int(cold.sum()), dtype=torch.float64), []
+    for t in range(L):
+        g1, g2 = torch.sigmoid(U[t, ..., 1] + W[0] * state + b[0]), torch.sigmoid(U[t, ..., 2] + W[1] * state + b[1])
+        state = (state - U[t, ..., 0]) * g1 + U[t, ..., 0]
+        h.append((state - X[t]) * g2 + X[t])
+    want = torch.autograd.grad((torch.stack(h), state), (U, X, W, b), (torch.tensor(gh[:, :, ~hot]).double(), torch.tensor(gl[:, ~hot]).double()))
+    for a, r in zip((got[0][:, :, cold], got[1][:, :, cold]), want[:2]):
+        assert ((a - r).abs() <= 1e-5 * r.abs().clamp(min=1.0)).all()
+    for a, r in zip((got[2][:, cold], got[3][:, cold]), want[2:]):
+        assert ((a - r).abs() <= 1e-5 * max(1.0, float(r.abs().max()))).all()
