@@ -2,14 +2,14 @@
 // and g (rows, cols), of which a small result is left.
 //
 // What bounds it: the result is small, so the library's tiles of it leave compute units idle or walk all rows one after
-// the other (8192 rows, 512 x 6144: 102 us, 505 TFLOP/s; 256 x 1024: 53 us). Here the rows are split as well, in as many
+// the other (8192 rows, 512 x 6144: 98 us, 526 TFLOP/s; 256 x 1024: 52 us). Here the rows are split as well, in as many
 // parts as fill the chip with one round of workgroups (sru_layer.h), float slices of the result meet in a second
 // launch, and that launch writes the gradient in the type of the parameter: under autocast in float, which
-// took a conversion pass over a gradient rounded to 16 bits. With that pass: 111 -> 71 us, 54 -> 21.5, 2048 x 512 57 -> 33.
-// 16384 rows, 512 x 3072: 153 -> 73. What bounds it now: a tile of rows takes 0.9 us, of which the matrix cores are
+// took a conversion pass over a gradient rounded to 16 bits. With that pass: 103 -> 77 us, 55 -> 21, 2048 x 512 58 -> 33.
+// 16384 rows, 512 x 3072: 148 -> 75. What bounds it now: a tile of rows takes 0.9 us, of which the matrix cores are
 // busy 0.33; LDS, which every operand passes twice, 0.27 (no bank conflicts); the loads as much; they overlap little.
-// Measured against it: a second tile in flight (level), a workgroup order by which an XCD reads all of g (84 -> 71 with
-// this one), 64-bit addresses per lane.
+// Measured against it: a second tile in flight (level), a workgroup order by which an XCD reads all of g (18% slower), 64-bit
+// addresses per lane.
 //
 // Mapping. A workgroup of four wavefronts owns 128 columns of x by 128 or 192 of g and walks its part of the rows 64 at a
 // time: one tile is in LDS as it is in memory, the next in registers on its way there, one barrier a tile. Both operands

@@ -156,16 +156,17 @@ struct GradParams {
 // One round of workgroups, one to each of 256 compute units: a tile of 64 rows takes 0.66 us with 128 columns and
 // 0.88 with 192, the slices are written and read at 3.5 TB/s, and the sum of both is least. Measured (us, library
 // product with conversion / 128 columns / 192, with the best number of parts each, the rule's choice marked *):
-//   8192 rows   512 x 6144   111/83/71*     2048 x 512   57/33*/38    1024 x 3072  89/79/71*    256 x 1024  54/21*/24
-//   4096 rows   512 x 1536   31/24*/26      256 x 3072   32/22*/23    1024 x 3072  49/46/43*
-//   16384 rows  512 x 3072   153/79/73*     1024 x 8192  296/322/328
-//   2048 rows   512 x 3072   24/24/24       2048 x 512   20/19/22
-// More rows and smaller results are the library's worst (32768 rows, 512 x 512 157 -> 36; 16384 rows, 128 x 2048 130 ->
-// 25); where the rows are not split it is level or faster (4096 rows, 768 x 4096 47 / 50).
+//   8192 rows   512 x 6144   103/96/77*     2048 x 512   58/33*/38    1024 x 3072  86/90/73*    256 x 1024  55/21*/24
+//   4096 rows   512 x 1536   32/23*/25      256 x 3072   32/21*/23    1024 x 3072  49/52/46*
+//   16384 rows  512 x 3072   148/92/75*     1024 x 8192  283/314/399
+//   2048 rows   512 x 3072   25/25/26       2048 x 512   21/19/22
+// More rows and smaller results are the library's worst (32768 rows, 512 x 512 155 -> 36; 16384 rows, 128 x 2048 132 ->
+// 25); where the rows are not split it is level or faster (4096 rows, 768 x 4096 51 / 54). Of 120 sizes drawn at random
+// that are taken one was slower (55393 rows, 576 x 3264 286 / 297).
 struct GradPlan { int tile_n, splits; };
 // A call costs its host some 25 us more than torch's: taken from 8192 rows on, where the library loses more than that
-// (8192 rows, 256 x 256 50/16, 128 x 512 71/16; 16384 rows, 256 x 768 96/23), below where the products keep the GPU
-// busier than the host (from 3000 rows and 3e9 multiply-adds; 4096 rows, 256 x 1024 30/18 is left alone). More than 16
+// (8192 rows, 256 x 256 50/17, 128 x 512 70/17; 16384 rows, 256 x 768 95/24), below where the products keep the GPU
+// busier than the host (from 3000 rows and 3e9 multiply-adds; 4096 rows, 256 x 1024 30/17 is left alone). More than 16
 // parts were no faster anywhere.
 constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384;
 inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {

@@ -5,7 +5,7 @@
 // 2048 columns 32.6 us on 64 of the chip's 1024 SIMDs), while the state's own dependence is a
 // multiply-add, exp2, add, reciprocal and a multiply-add. Here one wavefront of a workgroup does only
 // that, for 64 columns, and kRelayHelpers others do the rest: memory, conversions, the output gate.
-// 512 steps of 2048 columns bf16: 33.4 -> 21 us, float 38.7 -> 26; 201 steps of 12160 columns (d = 304) 21.4 -> 12.6.
+// 512 steps of 2048 columns bf16: 33.4 -> 21 us, float 38.7 -> 26; 201 steps of 12160 columns (d = 152 or 304) 21.5 -> 13.2.
 // What bounds it now: a step of the chain, 33 ns of which 27 remain when the helpers do nothing (six dependent
 // instructions, two of them transcendental); a fifth of a chunk is its hand-over (chunks of 8 steps: 40 ns a
 // step; of 32: no faster, for the helpers' registers).

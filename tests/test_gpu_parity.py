@@ -363,8 +363,8 @@ def test_long_right_padded_rows_forward_only_and_training(dt):
 
 
 FLOAT_X = [
-    dict(L=21, B=3, d=64, dirs=2, scale=1.7),                             # lane pairs, wave-uniform
-    dict(L=40, B=4, d=70, dirs=2, pad="right", scale=1.3, mask_c=True),   # lane pairs, wavefronts straddle rows
+    dict(L=21, B=3, d=64, dirs=2, scale=1.7),                             # few columns, whole wavefronts
+    dict(L=40, B=4, d=70, dirs=2, pad="right", scale=1.3, mask_c=True),   # few columns, wavefronts straddle rows
     dict(L=17, B=2, d=6, pad="random"),                                   # less than a wavefront
     dict(L=19, B=64, d=1024, dirs=2, pad="right", scale=1.7),             # two columns per lane (131 072 columns)
     dict(L=12, B=1100, d=70, dirs=2, pad="random", scale=0.8),            # two columns per lane, straddling rows
