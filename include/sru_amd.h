@@ -59,7 +59,7 @@
 extern "C" {
 #endif
 
-#define SRU_AMD_ABI_VERSION 6
+#define SRU_AMD_ABI_VERSION 7
 
 enum sru_amd_dtype {
     SRU_AMD_F32 = 0,
@@ -257,6 +257,27 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
                           const void *weight_c, const void *bias, const void *c_init,
                           const uint8_t *mask_pad, const void *scale_x, void *projected,
                           void *h, void *c_last, void *stream);
+
+/* A stack of such layers, each of the width of its input, in one launch (two with the clearing of the workspace): one time
+ * step, or a sequence in one direction of at most 64 batch rows, through up to SRU_AMD_STACK_MAX_LAYERS layers of one
+ * form (sru/modules.py:617-652, a loop over the layers there). `shape` is that of each layer's recurrence (16-bit streams, k 3,
+ * skip_type 0 or 1, is_custom 0).
+ *
+ * sru_amd_stack_workspace_bytes: 0 where there is no kernel for the stack or the layers one by one are the faster way.
+ *   x            (L, B, D') in shape->dtype
+ *   weight_proj  `layers` pointers to (D', n_proj); NULL iff n_proj is 0
+ *   weight       ... to (n_proj or D', 3 D'), both in shape->dtype, row-major
+ *   weight_c, bias, scale_x   ... as in sru_amd_forward_small; scale_x or any of its pointers may be NULL
+ *   c_init       (layers, B, D') or NULL; c_last (layers, B, D')
+ *   h            (L, B, D'), the last layer's
+ *   workspace    16-byte aligned; contents before and after are undefined
+ * Streams, weights and the workspace are 16-byte aligned. */
+#define SRU_AMD_STACK_MAX_LAYERS 16
+size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers, int64_t n_proj);
+int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t layers, int64_t n_proj, const void *x,
+                          const void *const *weight_proj, const void *const *weight, const void *const *weight_c,
+                          const void *const *bias, const void *const *scale_x, const void *c_init, const uint8_t *mask_pad,
+                          void *h, void *c_last, void *workspace, size_t workspace_bytes, void *stream);
 
 /* A dense product, out (rows, cols) = x (rows, inner) weight (inner, cols), all row-major in `dtype` (float, or 16
  * bits with float sums) and 16-byte aligned: compute_U of a short sequence or a prompt (sru/modules.py:252-274,

@@ -9,7 +9,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsru_amd.so")
-ABI_VERSION = 6
+ABI_VERSION = 7
 STATE_INTERVAL = 8   # SRU_AMD_STATE_INTERVAL
 STATIC_MAX_COLUMNS = 262144   # SRU_AMD_STATIC_MAX_COLUMNS
 NORM_MAX_FEATURES = 4096       # SRU_AMD_NORM_MAX_FEATURES
@@ -50,6 +50,8 @@ SIGNATURES = {
     "sru_amd_backward_static": (ctypes.c_int, [ctypes.POINTER(Shape)] + [_P] * 17),
     "sru_amd_layer_route": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
     "sru_amd_layer_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 13),
+    "sru_amd_stack_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
+    "sru_amd_stack_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 11 + [ctypes.c_size_t, _P]),
     "sru_amd_product_wanted": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3),
     "sru_amd_product": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3 + [_P] * 4),
     "sru_amd_product_grad_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int32] + [ctypes.c_int64] * 3),
@@ -100,7 +102,7 @@ _host = None
 class GeneralHost:
     """Stands for the native host code where that cannot be used: nothing is plain, every call goes the
     general way of functional.py."""
-    scan_forward = scan_backward = product = staticmethod(lambda *args: None)
+    scan_forward = scan_backward = product = stack_forward = staticmethod(lambda *args: None)
     autocast_operand = staticmethod(lambda t: None)
     layer_forward = staticmethod(lambda *args: False)
 

@@ -335,6 +335,131 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// What a cell holds under a name, borrowed; null: nothing.
+struct Cell {
+    PyObject *const attributes, *const parameters, *const buffers;
+    static PyObject *item(PyObject *dict, const char *name) {
+        PyObject *const o = dict ? PyDict_GetItemString(dict, name) : nullptr;
+        return o;
+    }
+    explicit Cell(PyObject *dict) : attributes(dict), parameters(item(dict, "_parameters")), buffers(item(dict, "_buffers")) {}
+    PyObject *attribute(const char *name) const { return item(attributes, name); }
+    bool is(const char *name, PyObject *value) const { return attribute(name) == value; }
+    bool number(const char *name, int64_t &v) const {
+        PyObject *const o = attribute(name);
+        return o && o != Py_None && read(o, v);
+    }
+    bool positive(const char *name) const {   // (or not a number)
+        PyObject *const o = attribute(name);
+        return !o || !PyFloat_Check(o) || PyFloat_AS_DOUBLE(o) != 0.0;
+    }
+    bool empty(const char *name) const {
+        PyObject *const o = attribute(name);
+        return o && PyDict_Check(o) && PyDict_GET_SIZE(o) == 0;
+    }
+    bool tensor(PyObject *dict, const char *name, Arg &a) const {
+        PyObject *const o = item(dict, name);
+        return o && read(o, a);
+    }
+};
+
+// stack_forward(cells, type of a cell, x, c0, mask_pad) -> (h, last states), or None where the layers have to be called one
+// by one: one of them is not of that type, has a step of its own, hooks, a normalisation, a module or dropout, or differs from the others
+// in its form, or there is no kernel for the stack
+PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Arg x, init, pad;
+    if (n != 5 || !PyList_Check(a[0]) || observed() || !read(a[2], x) || !read(a[3], init) || !read(a[4], pad) || !x || !x->is_cuda() || x->dim() != 3 ||
+        !narrow(x->scalar_type()))
+        return none();
+    const int64_t layers = PyList_GET_SIZE(a[0]), length = x->size(0), batch = x->size(1), width = x->size(2);
+    constexpr int kLayers = SRU_AMD_STACK_MAX_LAYERS;
+    if (layers < 1 || layers > kLayers) return none();
+    const at::ScalarType type = x->scalar_type();
+    const c10::Device device = x->device();
+    sru_amd_shape s{};
+    s.length = length;
+    s.batch = batch;
+    s.k = 3;
+    dtype_code(type, s.dtype);
+    s.state_interval = 1;
+    s.x_dtype = SRU_AMD_X_AS_STREAMS;
+    const void *projs[kLayers], *weights[kLayers], *wcs[kLayers], *biases[kLayers], *scales[kLayers];
+    size_t need = 0;
+    int64_t n_proj = 0;
+    uint32_t flags = 0;
+    for (int64_t l = 0; l < layers; ++l) {
+        PyObject *const o = PyList_GET_ITEM(a[0], l);
+        PyObject **const dict = (PyObject *)Py_TYPE(o) == a[1] ? _PyObject_GetDictPtr(o) : nullptr;
+        if (!dict || !*dict) return none();
+        const Cell cell(*dict);
+        for (const char *own : {"forward", "compute_UV", "compute_U", "apply_recurrence", "_whole_layer", "_normalise", "_call_impl", "_compiled_call_impl"})
+            if (cell.attribute(own)) return none();
+        for (const char *hooks : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"})
+            if (!cell.empty(hooks)) return none();
+        PyObject *const native = cell.attribute("native_16bit");
+        if (!cell.is("custom_m", Py_None) || !cell.is("layer_norm", Py_None) || (native && native != Py_True) ||
+            (!cell.is("training", Py_False) && (cell.positive("dropout") || cell.positive("rnn_dropout"))))
+            return none();
+        int64_t d = 0, act = 0, inputs = 0;
+        bool both = false, has_skip = false, rescale = false;
+        if (!cell.number("hidden_size", d) || !cell.number("activation_type", act) || !cell.number("input_size", inputs) || !cell.attribute("bidirectional") ||
+            !cell.attribute("has_skip_term") || !cell.attribute("rescale") || !read(cell.attribute("bidirectional"), both) ||
+            !read(cell.attribute("has_skip_term"), has_skip) || !read(cell.attribute("rescale"), rescale))
+            return none();
+        Arg proj, weight, weight_c, bias, scale;
+        if (!cell.tensor(cell.parameters, "weight", weight) || !cell.tensor(cell.parameters, "weight_c", weight_c) || !cell.tensor(cell.parameters, "bias", bias) ||
+            !(cell.tensor(cell.parameters, "weight_proj", proj) || cell.is("weight_proj", Py_None)) || !weight || !weight_c || !bias)
+            return none();
+        if (rescale && !cell.tensor(cell.buffers, "scale_x", scale)) return none();
+        const int64_t project = proj ? (proj->dim() == 2 ? proj->size(1) : -1) : 0;
+        if (l == 0) {
+            s.hidden = d;
+            s.dirs = both ? 2 : 1;
+            s.activation_type = (int32_t)act;
+            s.skip_type = has_skip ? 1 : 0;
+            n_proj = project;
+            if (d < 1 || d * s.dirs != width || (act != 0 && act != 1)) return none();
+            need = sru_amd_stack_workspace_bytes(&s, layers, n_proj);
+            if (need == 0) return none();
+        }
+        const int64_t inner = n_proj ? n_proj : width;
+        uint32_t small16 = 0;
+        if (d != s.hidden || (both ? 2 : 1) != s.dirs || act != s.activation_type || has_skip != (s.skip_type == 1) || project != n_proj || inputs != width ||
+            weight->scalar_type() != type || weight->dim() != 2 || weight->size(0) != inner || weight->size(1) != 3 * width || !plain(*weight.t, device, inner * 3 * width, 16) ||
+            (proj && (proj->scalar_type() != type || proj->size(0) != width || !plain(*proj.t, device, width * n_proj, 16))) || weight_c->dim() != 1 ||
+            !small(weight_c, device, 2 * width, type, true, SRU_AMD_SMALL_WEIGHT_C, small16) ||
+            !small(bias, device, 2 * width, type, true, SRU_AMD_SMALL_BIAS, small16) || !small(scale, device, 1, type, true, SRU_AMD_SMALL_SCALE, small16))
+            return none();
+        if (!scale) small16 |= flags & SRU_AMD_SMALL_SCALE;
+        if (l == 0) flags = small16;
+        if (small16 != flags) return none();
+        projs[l] = proj.ptr();
+        weights[l] = weight.ptr();
+        wcs[l] = weight_c.ptr();
+        biases[l] = bias.ptr();
+        scales[l] = s.skip_type == 1 ? scale.ptr() : nullptr;
+    }
+    if (!plain(*x.t, device, length * batch * width, 16) || (init && (init->dim() != 3 || init->size(0) != layers)) ||
+        !small(init, device, layers * batch * width, type, true, SRU_AMD_SMALL_INIT, flags) || !plain_pad(pad, device, length, batch))
+        return none();
+    at::Tensor h, last;
+    int rc;
+    {
+        const Unlocked unlocked;
+        const c10::DeviceGuard guard(device);
+        const auto options = x->options();
+        h = at::empty({length, batch, width}, options);
+        last = at::empty({layers, batch, width}, options);
+        const at::Tensor workspace = at::empty({(int64_t)need / 4}, options.dtype(at::kFloat));
+        rc = sru_amd_stack_forward(&s, flags | SRU_AMD_SMALL_LAST, layers, n_proj, x.ptr(), projs, weights, wcs, biases, scales, init.ptr(),
+                                   static_cast<const uint8_t *>(pad.ptr()), h.data_ptr(), last.data_ptr(), workspace.data_ptr(), need, stream_of(device));
+    }
+    if (rc != SRU_AMD_OK) return none();
+    return Py_BuildValue("(NN)", wrap(h), wrap(last));
+    END_HANDLE_TH_ERRORS
+}
+
 // product(x, weight) -> x weight in float, by the kernel where that is the faster one, else None
 PyObject *float_product(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -383,6 +508,7 @@ PyMethodDef methods[] = {
     {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},
     {"scan_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_backward)), METH_FASTCALL, nullptr},
     {"layer_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_forward)), METH_FASTCALL, nullptr},
+    {"stack_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(stack_forward)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Calls of the recurrence in the plain case.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -346,6 +346,45 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
     return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
 }
 
+size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers, int64_t n_proj) {
+    if (check_shape(shape) != SRU_AMD_OK || n_proj < 0) return 0;
+    const sru_amd_shape &s = *shape;
+    const int64_t Dp = s.hidden * s.dirs;
+    if (elem_size(s.dtype) != 2 || s.is_custom || x_is_float_beside_16bit(s) || s.k != 3 || s.length != 1 || !stack_sizes_ok(layers, s.batch, Dp, n_proj)) return 0;
+    return stack_workspace(layers, s.batch, Dp, n_proj);
+}
+
+int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t layers, int64_t n_proj, const void *x,
+                          const void *const *weight_proj, const void *const *weight, const void *const *weight_c,
+                          const void *const *bias, const void *const *scale_x, const void *c_init, const uint8_t *mask_pad,
+                          void *h, void *c_last, void *workspace, size_t workspace_bytes, void *stream) {
+    if (const int rc = check_shape(shape)) return rc;
+    const sru_amd_shape &s = *shape;
+    const size_t need = sru_amd_stack_workspace_bytes(shape, layers, n_proj);
+    if (need == 0) return SRU_AMD_ERR_BAD_SHAPE;
+    if (const int rc = check_small(s, small16)) return rc;
+    if (!x || !weight || !weight_c || !bias || !h || !c_last || (n_proj > 0 && !weight_proj)) return SRU_AMD_ERR_NULL_POINTER;
+    if (!workspace || !aligned(workspace, 16) || workspace_bytes < need) return SRU_AMD_ERR_WORKSPACE;
+    auto small_align = [&](uint32_t bit) { return (small16 & bit) ? (size_t)2 : (size_t)4; };
+    StackParams p{};
+    for (int64_t l = 0; l < layers; ++l) {
+        StackLayer &to = p.layer[l];
+        to = {weight[l], n_proj ? weight_proj[l] : nullptr, weight_c[l], bias[l], s.skip_type == 1 && scale_x ? scale_x[l] : nullptr};
+        if (!to.weight || !to.wc || !to.bias || (n_proj > 0 && !to.weight_proj)) return SRU_AMD_ERR_NULL_POINTER;
+        if (!aligned(to.weight, 16) || !aligned(to.weight_proj, 16) || !aligned(to.wc, small_align(SRU_AMD_SMALL_WEIGHT_C)) ||
+            !aligned(to.bias, small_align(SRU_AMD_SMALL_BIAS)) || !aligned(to.scale_x, small_align(SRU_AMD_SMALL_SCALE)))
+            return SRU_AMD_ERR_MISALIGNED;
+    }
+    if (!aligned(x, 16) || !aligned(h, 16) || !aligned(c_init, small_align(SRU_AMD_SMALL_INIT)) || !aligned(c_last, small_align(SRU_AMD_SMALL_LAST)))
+        return SRU_AMD_ERR_MISALIGNED;
+    p.x = x; p.c0 = c_init; p.pad = mask_pad; p.h = h; p.c_last = c_last;
+    p.layers = (int32_t)layers; p.rows = (int32_t)s.batch; p.Dp = (int32_t)(s.hidden * s.dirs); p.n_proj = (int32_t)n_proj;
+    p.outputs_at = stack_outputs_at(layers, s.batch, n_proj);
+    p.act = s.activation_type; p.skip = s.skip_type == 1; p.small16 = small16;
+    const hipError_t err = launch_layer_stack(p, workspace, need, s.dtype == SRU_AMD_F16, static_cast<hipStream_t>(stream));
+    return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
+}
+
 int sru_amd_product_wanted(int32_t dtype, int64_t rows, int64_t inner, int64_t cols) {
     return (dtype == SRU_AMD_F32 || dtype == SRU_AMD_F16 || dtype == SRU_AMD_BF16) && product_wanted((int)elem_size(dtype), rows, inner, cols);
 }

@@ -94,6 +94,42 @@ inline bool rows_sizes_ok(int64_t L, int64_t B, int64_t d, int64_t dirs, int64_t
 }
 hipError_t launch_layer_rows(const RowsParams &p, bool half, int k, hipStream_t st);
 
+// One time step of a stack of layers of one width in one launch (layer_stack.hip).
+constexpr int kStackMaxLayers = 16;   // their pointers are kernel arguments
+constexpr size_t kStackHeader = 256;  // bytes of the workspace in front of what pieces hand over
+struct StackLayer {
+    const void *weight, *weight_proj, *wc, *bias, *scale_x;
+};
+struct StackParams {
+    StackLayer layer[kStackMaxLayers];
+    const void *x, *c0;       // (rows, Dp); (layers, rows, Dp) or null
+    const uint8_t *pad;
+    void *h, *c_last;
+    uint32_t *ticket;
+    char *exchange;           // projected rows of every layer, outputs of every layer but the last
+    int64_t outputs_at;
+    int32_t layers, rows, Dp, n_proj, pieces, act, skip;
+    uint32_t small16;
+};
+// Where the step kernels take each of the layers, of which there have to be two. Layer by layer / in one launch, bf16, us a pass,
+// launched one by one and in a graph (8 layers unless another number is given):
+//                          1 row                  16 rows                 64 rows
+//   64                  81/24   30/25          82/23   30/29           81/53   55/60
+//   1024                86/32   57/38          86/38   64/45          111/87  115/92
+//   2048                85/60   89/68          95/72   99/78          162/134 167/139
+//   2048 -> 512        112/43   96/49         107/61  109/68          189/145 193/151
+//   3072               189/139 193/149        211/165 216/173         233/267 233/272 (past the step kernels' sizes)
+//   two of 64           30/18   18/21          28/16   16/17           27/15   21/22
+//   two of 2048         27/20   29/27          28/22   32/30           45/38   49/45
+inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
+    return layers >= 2 && layers <= kStackMaxLayers && n_proj < Dp && step_sizes_ok(rows, Dp, Dp, n_proj);
+}
+inline int64_t stack_outputs_at(int64_t layers, int64_t rows, int64_t n_proj) { return layers * rows * n_proj * 2; }
+inline size_t stack_workspace(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
+    return kStackHeader + (size_t)(stack_outputs_at(layers, rows, n_proj) + (layers - 1) * rows * Dp * 2);
+}
+hipError_t launch_layer_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st);
+
 // A product by itself (product.hip): x (rows, inner) times weight (inner, cols), all in one type.
 struct ProductParams {
     const void *x, *weight;

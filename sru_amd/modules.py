@@ -19,6 +19,7 @@ import torch.nn as nn
 from torch import Tensor
 from torch.nn.utils.rnn import PackedSequence, pad_packed_sequence, pack_padded_sequence
 
+from . import _lib
 from .functional import dense, layer_forward
 from .norm import layer_norm as fused_layer_norm, supported as fused_layer_norm_supported
 from .ops import elementwise_recurrence_gpu
@@ -262,6 +263,12 @@ class SRUCell(nn.Module):
 # The steps that `layer_forward` stands for, as this file defines them: a subclass, an instance or an
 # assignment to the class may put others in their place, which are then called.
 _COMPUTE_UV, _COMPUTE_U, _APPLY_RECURRENCE = SRUCell.compute_UV, SRUCell.compute_U, SRUCell.apply_recurrence
+# ... and what a stack's one call stands for: whole cells, as torch calls them.
+_CELL_METHODS = tuple((name, getattr(SRUCell, name)) for name in ("__call__", "forward", "compute_UV", "compute_U", "apply_recurrence",
+                                                                  "_whole_layer", "_normalise"))
+_LAYER_FORWARD = layer_forward
+_GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks,
+                 torch.nn.modules.module._global_backward_hooks, torch.nn.modules.module._global_backward_pre_hooks)
 
 
 class SRU(nn.Module):
@@ -336,11 +343,15 @@ class SRU(nn.Module):
             states = list(c0.unbind(0))
 
         x = input if self.input_to_hidden is None else self.input_to_hidden(input)
-        finals = []
-        for layer, state in zip(self.rnn_lst, states):
-            x, c = layer(x, state, mask_pad=mask_pad)
-            finals.append(c)
-        c_stack = torch.stack(finals)
+        done = self._whole_stack(x, c0, mask_pad)
+        if done is not None:
+            x, c_stack = done
+        else:
+            finals = []
+            for layer, state in zip(self.rnn_lst, states):
+                x, c = layer(x, state, mask_pad=mask_pad)
+                finals.append(c)
+            c_stack = torch.stack(finals)
         if self.nn_rnn_compatible_return:
             # (layers, batch, dirs*hidden) -> (layers*dirs, batch, hidden), as nn.RNN returns it
             b = input.size(1)
@@ -350,6 +361,17 @@ class SRU(nn.Module):
         if packed:
             x = pack_padded_sequence(x, lengths, enforce_sorted=False)
         return x, c_stack
+
+    def _whole_stack(self, x: Tensor, c0: Optional[Tensor], mask_pad: Optional[Tensor]) -> Optional[Tuple[Tensor, Tensor]]:
+        """All layers in one call without gradients: (output, last states), or None where they are called one by one, as they
+        are wherever one of them could tell the difference (see `SRUCell._whole_layer`; hooks, a method put in place of a
+        cell's own, a module of another type in its place)."""
+        if (torch.is_grad_enabled() or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not Tensor or torch.compiler.is_compiling()
+                or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or layer_forward is not _LAYER_FORWARD
+                or type(self.rnn_lst) is not nn.ModuleList or any(getattr(SRUCell, name) is not own for name, own in _CELL_METHODS)
+                or any(_GLOBAL_HOOKS)):
+            return None
+        return _lib.host().stack_forward(list(self.rnn_lst._modules.values()), SRUCell, x, c0, mask_pad)
 
     def reset_parameters(self):
         for layer in self.rnn_lst:
