@@ -102,7 +102,7 @@ _host = None
 class GeneralHost:
     """Stands for the native host code where that cannot be used: nothing is plain, every call goes the
     general way of functional.py."""
-    scan_forward = scan_backward = product = stack_forward = staticmethod(lambda *args: None)
+    scan_forward = scan_backward = product = stack_forward = recurrence = layer = staticmethod(lambda *args: None)
     autocast_operand = staticmethod(lambda t: None)
     layer_forward = staticmethod(lambda *args: False)
 

@@ -6,7 +6,7 @@
 //
 // Why: a forward and backward pass of the recurrence cost the host 145-175 us in Python, more than the
 // kernels of most sizes take. 128 x 32 x 1024 f32 with padding, 53 us of kernels: 159 us a pass then,
-// 90-94 us through here (the rest is torch's own autograd); one token through ten layers of 2048: 221
+// 90-94 us through here (with Python's autograd around it); one token through ten layers of 2048: 221
 // and 133 us.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -19,7 +19,10 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/PyInterpreter.h>
+#include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
 
 #include "sru_amd.h"
 
@@ -96,6 +99,17 @@ struct Call {
     const c10::Device device() const { return u->device(); }
 };
 
+// the first twelve arguments of a recurrence's forward call
+bool read_scan(PyObject *const *a, Call &c) {
+    if (!read(a[0], c.u) || !read(a[1], c.x) || !read(a[2], c.weight_c) || !read(a[3], c.bias) || !read(a[4], c.init) || !read(a[5], c.act) ||
+        !read(a[6], c.d) || !read(a[9], c.scale) || !read(a[10], c.mask_c) || !read(a[11], c.pad) || !read(a[7], c.bidirectional) ||
+        !read(a[8], c.has_skip) || !c.x || c.x->dim() != 3)
+        return false;
+    c.length = c.x->size(0);
+    c.batch = c.x->size(1);
+    return true;
+}
+
 bool dtype_code(at::ScalarType t, int32_t &code) {
     code = t == at::kFloat ? SRU_AMD_F32 : t == at::kHalf ? SRU_AMD_F16 : SRU_AMD_BF16;
     return t == at::kFloat || narrow(t);
@@ -165,34 +179,62 @@ PyObject *wrap(const at::Tensor &t) {
     return THPVariable_Wrap(t);
 }
 
+// The recurrence of a prepared call: h, last state and, to be differentiated, the checkpoints.
+int run_forward(Call &c, bool train, at::Tensor &h, at::Tensor &last, at::Tensor &kept) {
+    if (narrow(c.u->scalar_type())) c.small16 |= SRU_AMD_SMALL_LAST;
+    const auto options = c.u->options();
+    h = at::empty({c.length, c.batch, c.width()}, options);
+    last = at::empty({c.batch, c.width()}, options);
+    if (train)
+        kept = at::empty({(int64_t)sru_amd_state_bytes(&c.shape) / (4 * c.batch * c.width()), c.batch, c.width()}, options.dtype(at::kFloat));
+    return sru_amd_forward_small(&c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(), c.mask_c.ptr(),
+                                 static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), h.data_ptr(), train ? kept.data_ptr() : nullptr,
+                                 last.data_ptr(), stream_of(c.device()));
+}
+
+// What a call's gradients need besides it, in the plain case.
+bool prepare_backward(Call &c, const Arg &kept, const Arg &grad_h, const Arg &grad_last) {
+    if (!kept || !grad_h || !prepare(c, true, false)) return false;
+    const int64_t columns = c.batch * c.width();
+    return kept->scalar_type() == at::kFloat && plain(*kept.t, c.device(), (int64_t)sru_amd_state_bytes(&c.shape) / 4, 4) &&
+           grad_h->scalar_type() == c.u->scalar_type() && plain(*grad_h.t, c.device(), c.length * columns, 4) &&
+           small(grad_last, c.device(), columns, c.u->scalar_type(), true, SRU_AMD_SMALL_LAST, c.small16);
+}
+
+constexpr int kGradients = 5;   // of u, x, weight_c, bias and init
+int run_backward(const Call &c, const Arg &kept, const Arg &grad_h, const Arg &grad_last, at::Tensor (&grads)[kGradients]) {
+    const int64_t width = c.width(), columns = c.batch * width;
+    const auto floats = c.u->options().dtype(at::kFloat);
+    grads[0] = at::empty(c.u->sizes(), c.u->options());
+    if (c.x) grads[1] = at::empty(c.x->sizes(), c.x->options());
+    grads[2] = at::empty({2 * width}, floats);
+    grads[3] = at::empty(c.bias->sizes(), floats);
+    const int64_t need = (int64_t)sru_amd_backward_workspace_bytes(&c.shape);
+    // (the gradient of an initial state that was not given is written behind the workspace)
+    const at::Tensor workspace = at::empty({need / 4 + (c.init ? 0 : columns)}, floats);
+    if (c.init) grads[4] = at::empty(c.init->sizes(), floats);
+    float *const init_out = c.init ? grads[4].data_ptr<float>() : workspace.data_ptr<float>() + need / 4;
+    return sru_amd_backward_small(
+        &c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(), c.mask_c.ptr(),
+        static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), kept.ptr(), grad_h.ptr(), grad_last.ptr(), grads[0].data_ptr(),
+        c.x ? grads[1].data_ptr() : nullptr, grads[2].data_ptr(), grads[3].data_ptr(), init_out, workspace.data_ptr(), (size_t)need,
+        stream_of(c.device()));
+}
+
 // scan_forward(u, x, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_c, mask_pad, train)
 //   -> (h, last, checkpoints or None, whether x and scale are read)
 PyObject *scan_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Call c;
-    if (observed() || n != 13 || !read(a[0], c.u) || !read(a[1], c.x) || !read(a[2], c.weight_c) || !read(a[3], c.bias) || !read(a[4], c.init) ||
-        !read(a[5], c.act) || !read(a[6], c.d) || !read(a[9], c.scale) || !read(a[10], c.mask_c) || !read(a[11], c.pad) ||
-        !read(a[7], c.bidirectional) || !read(a[8], c.has_skip))
-        return none();
+    if (observed() || n != 13 || !read_scan(a, c)) return none();
     const bool train = a[12] == Py_True;
-    if (!c.x || c.x->dim() != 3) return none();
-    c.length = c.x->size(0);
-    c.batch = c.x->size(1);
     if (!prepare(c, train, !train)) return none();
-    if (narrow(c.u->scalar_type())) c.small16 |= SRU_AMD_SMALL_LAST;
     at::Tensor h, last, kept;
     int rc;
     {
         const Unlocked unlocked;
         const c10::DeviceGuard guard(c.device());
-        const auto options = c.u->options();
-        h = at::empty({c.length, c.batch, c.width()}, options);
-        last = at::empty({c.batch, c.width()}, options);
-        if (train)
-            kept = at::empty({(int64_t)sru_amd_state_bytes(&c.shape) / (4 * c.batch * c.width()), c.batch, c.width()}, options.dtype(at::kFloat));
-        rc = sru_amd_forward_small(&c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(), c.mask_c.ptr(),
-                                   static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), h.data_ptr(), train ? kept.data_ptr() : nullptr,
-                                   last.data_ptr(), stream_of(c.device()));
+        rc = run_forward(c, train, h, last, kept);
     }
     if (rc != SRU_AMD_OK) return none();
     return Py_BuildValue("(NNNO)", wrap(h), wrap(last), wrap(kept), c.shape.skip_type == 1 ? Py_True : Py_False);
@@ -210,40 +252,27 @@ PyObject *scan_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         !read(a[10], grad_last) || !read(a[11], c.act) || !read(a[12], c.d) || !read(a[15], c.length) || !read(a[16], c.batch) ||
         !read(a[13], c.bidirectional) || !read(a[14], c.has_skip))
         return none();
-    if (!kept || !grad_h || !prepare(c, true, false)) return none();
-    const c10::Device device = c.device();
-    const int64_t width = c.width(), columns = c.batch * width;
-    const at::ScalarType type = c.u->scalar_type();
-    if (kept->scalar_type() != at::kFloat || !plain(*kept.t, device, (int64_t)sru_amd_state_bytes(&c.shape) / 4, 4) ||
-        grad_h->scalar_type() != type || !plain(*grad_h.t, device, c.length * columns, 4) ||
-        !small(grad_last, device, columns, type, true, SRU_AMD_SMALL_LAST, c.small16))
-        return none();
-    at::Tensor grad_u, grad_x, grad_wc, grad_bias, grad_init;
+    if (!prepare_backward(c, kept, grad_h, grad_last)) return none();
+    at::Tensor grads[kGradients];
     int rc;
     {
         const Unlocked unlocked;
-        const c10::DeviceGuard guard(device);
-        const auto floats = c.u->options().dtype(at::kFloat);
-        grad_u = at::empty(c.u->sizes(), c.u->options());
-        if (c.x) grad_x = at::empty(c.x->sizes(), c.x->options());
-        grad_wc = at::empty({2 * width}, floats);
-        grad_bias = at::empty(c.bias->sizes(), floats);
-        const int64_t need = (int64_t)sru_amd_backward_workspace_bytes(&c.shape);
-        // (the gradient of an initial state that was not given is written behind the workspace)
-        const at::Tensor workspace = at::empty({need / 4 + (c.init ? 0 : columns)}, floats);
-        if (c.init) grad_init = at::empty(c.init->sizes(), floats);
-        float *const init_out = c.init ? grad_init.data_ptr<float>() : workspace.data_ptr<float>() + need / 4;
-        rc = sru_amd_backward_small(
-            &c.shape, c.small16, c.u.ptr(), c.x.ptr(), c.weight_c.ptr(), c.bias.ptr(), c.init.ptr(), c.mask_c.ptr(),
-            static_cast<const uint8_t *>(c.pad.ptr()), c.scale.ptr(), kept.ptr(), grad_h.ptr(), grad_last.ptr(), grad_u.data_ptr(),
-            c.x ? grad_x.data_ptr() : nullptr, grad_wc.data_ptr(), grad_bias.data_ptr(), init_out, workspace.data_ptr(), (size_t)need,
-            stream_of(device));
+        const c10::DeviceGuard guard(c.device());
+        rc = run_backward(c, kept, grad_h, grad_last, grads);
     }
     if (rc != SRU_AMD_OK) return none();
-    return Py_BuildValue("(NNNNN)", wrap(grad_u), wrap(grad_x), wrap(grad_wc), wrap(grad_bias), wrap(grad_init));
+    return Py_BuildValue("(NNNNN)", wrap(grads[0]), wrap(grads[1]), wrap(grads[2]), wrap(grads[3]), wrap(grads[4]));
     END_HANDLE_TH_ERRORS
 }
 
+// out = x weight, by a kernel where that is the faster one (the device is set)
+void product_into(at::Tensor &out, const at::Tensor &x, const at::Tensor &weight, int32_t dtype) {
+    const int64_t rows = x.size(0), inner = x.size(1), cols = weight.size(1);
+    if (sru_amd_product_wanted(dtype, rows, inner, cols) && aligned(x, 16) && aligned(weight, 16) && weight.is_contiguous() && x.is_contiguous() &&
+        sru_amd_product(dtype, rows, inner, cols, x.data_ptr(), weight.data_ptr(), out.data_ptr(), stream_of(x.device())) == SRU_AMD_OK)
+        return;
+    at::mm_out(out, x, weight);
+}
 // x weight, with `own` by a kernel where that is the faster one (the device is set)
 at::Tensor product(const at::Tensor &x, const at::Tensor &weight, int32_t dtype, bool own) {
     const int64_t rows = x.size(0), inner = x.size(1), cols = weight.size(1);
@@ -252,6 +281,308 @@ at::Tensor product(const at::Tensor &x, const at::Tensor &weight, int32_t dtype,
         if (sru_amd_product(dtype, rows, inner, cols, x.data_ptr(), weight.data_ptr(), out.data_ptr(), stream_of(x.device())) == SRU_AMD_OK) return out;
     }
     return at::mm(x, weight);
+}
+
+// ---------------------------------------------------------------- autograd
+// The graph's own nodes in the plain case. Python's autograd Functions cost some 25 us of host time a pass more for the
+// recurrence and 60 for a layer: two float layers of 256, 32 steps of 32 rows, 320 -> 163-220 us a training step with 105 us of
+// kernels; the recurrence alone, 128 x 32 x 1024 float padded, 96 -> 76 us with 53. A layer that knows both of its parts also adds the
+// skip term's gradient in the product that makes the rest of it: 512 x 16 rows, ten layers of 2048 under autocast 4246 -> 4091 us.
+
+using torch::autograd::SavedVariable;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+
+bool usable(const at::Tensor &t) {   // (what came back from a hook or from another node)
+    return !t.defined() || (t.layout() == at::kStrided && t.has_storage() && !t.key_set().has(c10::DispatchKey::Python));
+}
+
+// Tensors and flags of a recurrence between its forward and backward pass.
+struct Kept {
+    enum { U, X, WeightC, Bias, Init, Scale, MaskC, Pad, States, kCount };
+    SavedVariable saved[kCount];
+    int64_t act = 0, d = 0, length = 0, batch = 0;
+    bool bidirectional = false, has_skip = false;
+
+    void keep(const Call &c, const at::Tensor &states) {
+        const auto save = [](const Arg &a) { return a ? SavedVariable(*a.t, false) : SavedVariable(); };
+        const Arg of_states{&states};
+        int i = 0;
+        for (const Arg *a : {&c.u, &c.x, &c.weight_c, &c.bias, &c.init, &c.scale, &c.mask_c, &c.pad, &of_states}) saved[i++] = save(*a);
+        act = c.act;
+        d = c.d;
+        length = c.length;
+        batch = c.batch;
+        bidirectional = c.bidirectional;
+        has_skip = c.has_skip;
+    }
+    void release() {
+        for (SavedVariable &v : saved) v.reset_data();
+    }
+};
+
+// functional._scan_gradients(saved tensors, call, grad_h, grad_last): the general way, and what is wrong with a call
+void general_gradients(const Kept &k, const variable_list &saved, const at::Tensor &grad_h, const at::Tensor &grad_last, at::Tensor (&grads)[kGradients]) {
+    struct Locked {
+        const PyGILState_STATE state = PyGILState_Ensure();
+        ~Locked() { PyGILState_Release(state); }
+    } locked;
+    const auto raise = [] {
+        python_error error;
+        error.persist();
+        throw error;
+    };
+    PyObject *tensors = PyTuple_New((Py_ssize_t)saved.size());
+    for (size_t i = 0; tensors && i < saved.size(); ++i) PyTuple_SET_ITEM(tensors, (Py_ssize_t)i, wrap(saved[i]));
+    PyObject *const module = tensors ? PyImport_ImportModule("sru_amd.functional") : nullptr;
+    PyObject *const out = module ? PyObject_CallMethod(module, "_scan_gradients", "N(LLOOLL)NN", tensors, (long long)k.act, (long long)k.d,
+                                                       k.bidirectional ? Py_True : Py_False, k.has_skip ? Py_True : Py_False, (long long)k.length,
+                                                       (long long)k.batch, wrap(grad_h), wrap(grad_last))
+                                 : nullptr;
+    Py_XDECREF(module);
+    if (!out) raise();
+    for (int i = 0; i < kGradients; ++i) {
+        PyObject *const o = PyTuple_GET_ITEM(out, i);
+        if (o != Py_None) grads[i] = THPVariable_Unpack(o);
+    }
+    Py_DECREF(out);
+}
+
+void gradients_of(const Kept &k, const std::shared_ptr<torch::autograd::Node> &node, const at::Tensor &grad_h, const at::Tensor &grad_last,
+                  at::Tensor (&grads)[kGradients]) {
+    variable_list t;
+    for (const SavedVariable &v : k.saved) t.push_back(v.unpack(node));
+    bool as_usual = !observed() && usable(grad_h) && usable(grad_last);
+    for (const at::Tensor &v : t) as_usual = as_usual && usable(v);
+    if (as_usual) {
+        const auto arg = [&](const at::Tensor &v) { return Arg{v.defined() ? &v : nullptr}; };
+        Call c;
+        c.u = arg(t[Kept::U]);
+        c.x = arg(t[Kept::X]);
+        c.weight_c = arg(t[Kept::WeightC]);
+        c.bias = arg(t[Kept::Bias]);
+        c.init = arg(t[Kept::Init]);
+        c.scale = arg(t[Kept::Scale]);
+        c.mask_c = arg(t[Kept::MaskC]);
+        c.pad = arg(t[Kept::Pad]);
+        c.act = k.act;
+        c.d = k.d;
+        c.length = k.length;
+        c.batch = k.batch;
+        c.bidirectional = k.bidirectional;
+        c.has_skip = k.has_skip;
+        const Arg states = arg(t[Kept::States]), gh = arg(grad_h), gl = arg(grad_last);
+        if (prepare_backward(c, states, gh, gl)) {
+            const c10::DeviceGuard guard(c.device());
+            if (run_backward(c, states, gh, gl, grads) == SRU_AMD_OK) return;
+        }
+    }
+    general_gradients(k, t, grad_h, grad_last, grads);
+}
+
+struct RecurrenceNode : torch::autograd::Node {
+    Kept kept;
+    std::string name() const override { return "ElementwiseRecurrenceBackward"; }
+    void release_variables() override {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        kept.release();
+    }
+    variable_list apply(variable_list &&out) override {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        at::Tensor grads[kGradients];
+        gradients_of(kept, shared_from_this(), out[0], out[1], grads);
+        return variable_list(grads, grads + kGradients);
+    }
+};
+
+template <typename N> std::shared_ptr<N> new_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }
+bool wants(const Arg &a) { return a && a->requires_grad(); }
+Variable variable(const Arg &a) { return a ? *a.t : Variable(); }
+
+// recurrence(u, x, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_c, mask_pad) -> (h, last), in the graph
+// where gradients are recorded, or None: not the plain case
+PyObject *recurrence(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Call c;
+    if (observed() || n != 12 || !read_scan(a, c)) return none();
+    const Call given = c;
+    if (!prepare(c, true, false)) return none();
+    at::Tensor h, last, states;
+    int rc;
+    {
+        const Unlocked unlocked;
+        const c10::DeviceGuard guard(c.device());
+        rc = run_forward(c, true, h, last, states);
+    }
+    if (rc != SRU_AMD_OK) return none();
+    if (at::GradMode::is_enabled() && (wants(given.u) || wants(given.x) || wants(given.weight_c) || wants(given.bias) || wants(given.init))) {
+        const auto node = new_node<RecurrenceNode>();
+        node->set_next_edges(torch::autograd::collect_next_edges(variable(given.u), variable(given.x), variable(given.weight_c), variable(given.bias),
+                                                                 variable(given.init)));
+        node->kept.keep(c, states);
+        torch::autograd::create_gradient_edge(h, node);
+        torch::autograd::create_gradient_edge(last, node);
+    }
+    return Py_BuildValue("(NN)", wrap(h), wrap(last));
+    END_HANDLE_TH_ERRORS
+}
+
+// x^T grad in `dtype`
+at::Tensor weight_gradient(const at::Tensor &x, const at::Tensor &grad, at::ScalarType dtype) {
+    int32_t code = 0, out_code = 0;
+    const int64_t rows = x.size(0), inner = x.size(1), cols = grad.size(1);
+    if (!at::GradMode::is_enabled() && narrow(x.scalar_type()) && x.scalar_type() == grad.scalar_type() && dtype_code(x.scalar_type(), code) &&
+        dtype_code(dtype, out_code) && plain(x, grad.device(), rows * inner, 16) && plain(grad, grad.device(), rows * cols, 16)) {
+        const int64_t need = (int64_t)sru_amd_product_grad_workspace_bytes(code, rows, inner, cols);
+        if (need > 0) {
+            at::Tensor out = at::empty({inner, cols}, x.options().dtype(dtype));
+            const at::Tensor workspace = at::empty({need / 4}, x.options().dtype(at::kFloat));
+            if (sru_amd_product_grad(code, rows, inner, cols, x.data_ptr(), grad.data_ptr(), out_code, out.data_ptr(), workspace.data_ptr(),
+                                     (size_t)need, stream_of(x.device())) == SRU_AMD_OK)
+                return out;
+        }
+    }
+    return at::mm(x.t(), grad).to(dtype);
+}
+
+// A layer: the dense products and the recurrence behind them. The input's gradient is the skip term's plus the product's,
+// which the product adds to it where both are of one type.
+struct LayerNode : torch::autograd::Node {
+    enum { Input, Residual, WeightProj, Weight, WeightC, Bias, Init };
+    Kept kept;
+    SavedVariable operand, projected, weight_proj, weight;   // as the products read them
+    at::ScalarType input_type = at::kFloat, proj_type = at::kFloat, weight_type = at::kFloat;   // as they were given
+    bool one_input = false, has_proj = false;                // the skip term reads the layer's input
+    std::string name() const override { return "SRULayerBackward"; }
+    void release_variables() override {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        kept.release();
+        for (SavedVariable *v : {&operand, &projected, &weight_proj, &weight}) v->reset_data();
+    }
+    variable_list apply(variable_list &&out) override {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        const c10::impl::ExcludeDispatchKeyGuard as_they_are(c10::autocast_dispatch_keyset);
+        const auto self = shared_from_this();
+        at::Tensor grads[kGradients];
+        gradients_of(kept, self, out[0], out[1], grads);
+        const c10::DeviceGuard guard(grads[0].device());
+        variable_list result(7);
+        result[WeightC] = grads[2];
+        result[Bias] = grads[3];
+        result[Init] = grads[4];
+        const int64_t rows = kept.length * kept.batch;
+        at::Tensor grad = grads[0].view({rows, -1});
+        const bool input = task_should_compute_output(Input), of_proj = has_proj && task_should_compute_output(WeightProj);
+        const auto flat = [&](const SavedVariable &v) {
+            const at::Tensor t = v.unpack(self);
+            return t.reshape({rows, t.size(-1)});
+        };
+        if (task_should_compute_output(Weight)) {   // (to be differentiated again: as a function of what was projected)
+            const at::Tensor x = !has_proj ? flat(operand) : at::GradMode::is_enabled() ? at::mm(flat(operand), weight_proj.unpack(self)) : flat(projected);
+            result[Weight] = weight_gradient(x, grad, weight_type);
+        }
+        if (has_proj && (input || of_proj)) {
+            grad = at::mm(grad, weight.unpack(self).t());
+            if (of_proj) result[WeightProj] = weight_gradient(flat(operand), grad, proj_type);
+        }
+        if (!one_input) result[Residual] = grads[1];
+        if (!input) return result;
+        const at::Tensor back = (has_proj ? weight_proj : weight).unpack(self).t();
+        at::Tensor skip = one_input ? grads[1] : at::Tensor();
+        const auto whole = [&](const at::Tensor &t) { return t.view({kept.length, kept.batch, back.size(1)}); };
+        if (!skip.defined()) {
+            result[Input] = whole(at::mm(grad, back)).to(input_type);
+        } else if (at::GradMode::is_enabled()) {
+            result[Input] = skip + whole(at::mm(grad, back)).to(input_type);
+        } else if (skip.scalar_type() == grad.scalar_type()) {
+            skip.view({rows, back.size(1)}).addmm_(grad, back);
+            result[Input] = skip;
+        } else {
+            result[Input] = skip.add_(whole(at::mm(grad, back)));
+        }
+        return result;
+    }
+};
+
+// layer(input, residual, weight_proj, weight, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_c, mask_pad)
+//   -> (h, last) in the graph, or None: not the plain case, or no gradients are recorded
+PyObject *layer(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    Call c;
+    Arg input, weight_proj, weight;
+    if (observed() || !at::GradMode::is_enabled() || n != 14 || !read(a[0], input) || !read(a[1], c.x) || !read(a[2], weight_proj) || !read(a[3], weight) ||
+        !read(a[4], c.weight_c) || !read(a[5], c.bias) || !read(a[6], c.init) || !read(a[7], c.act) || !read(a[8], c.d) || !read(a[9], c.bidirectional) ||
+        !read(a[10], c.has_skip) || !read(a[11], c.scale) || !read(a[12], c.mask_c) || !read(a[13], c.pad) || !input || !weight || !c.weight_c ||
+        !c.bias || !c.x || c.x->dim() != 3 || input->dim() != 3 || !input->is_cuda() || input->size(0) != c.x->size(0) || input->size(1) != c.x->size(1))
+        return none();
+    if (!(wants(input) || wants(c.x) || wants(weight_proj) || wants(weight) || wants(c.weight_c) || wants(c.bias) || wants(c.init))) return none();
+    const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+    const at::ScalarType type = autocast ? at::autocast::get_autocast_dtype(at::kCUDA) : input->scalar_type();
+    int32_t code = 0;
+    if (!dtype_code(type, code) || (autocast && !narrow(type))) return none();
+    const c10::Device device = input->device();
+    c.length = input->size(0);
+    c.batch = input->size(1);
+    const int64_t rows = c.length * c.batch, in = input->size(2);
+    if (rows < 1 || in < 1 || !input->is_contiguous() || !aligned(*input.t, 16) || input->is_conj() || input->is_neg()) return none();
+    int64_t inner = in;
+    for (const Arg *w : {&weight_proj, &weight}) {
+        if (!*w) continue;
+        if ((*w)->dim() != 2 || (*w)->size(0) != inner || !plain(*w->t, device, (*w)->numel(), 16)) return none();
+        inner = (*w)->size(1);
+    }
+    for (const Arg *t : {&input, &weight_proj, &weight})
+        if (*t && (*t)->scalar_type() != type && !(autocast && (*t)->scalar_type() == at::kFloat)) return none();
+    if (autocast && narrow(c.x->scalar_type()) && c.x->scalar_type() != type) return none();
+    const Call given = c;
+    at::Tensor operand = *input.t, proj_operand = variable(weight_proj), weight_operand = *weight.t, projected, u, h, last, states;
+    int rc;
+    {
+        const Unlocked unlocked;
+        const c10::DeviceGuard guard(device);
+        u = at::empty({c.length, c.batch, inner}, input->options().dtype(type).requires_grad(false));
+        c.u.t = &u;
+        if (prepare(c, true, false)) {
+            if (autocast) {   // (with gradients recorded: these are torch's own conversions, a parameter's made once in a region)
+                operand = at::autocast::cached_cast(type, operand, at::kCUDA);
+                if (weight_proj) proj_operand = at::autocast::cached_cast(type, proj_operand, at::kCUDA);
+                weight_operand = at::autocast::cached_cast(type, weight_operand, at::kCUDA);
+            }
+            const at::AutoDispatchBelowADInplaceOrView below;
+            const c10::impl::ExcludeDispatchKeyGuard as_they_are(c10::autocast_dispatch_keyset);
+            at::Tensor x = operand.view({rows, in}), result = u.view({rows, inner});
+            if (weight_proj) {
+                projected = at::empty({rows, weight_proj->size(1)}, u.options());
+                product_into(projected, x, proj_operand, code);
+                x = projected;
+            }
+            product_into(result, x, weight_operand, code);
+            rc = run_forward(c, true, h, last, states);
+        } else {
+            rc = -1;
+        }
+    }
+    if (rc != SRU_AMD_OK) return none();
+    const auto node = new_node<LayerNode>();
+    const bool one_input = given.x.t->is_same(*input.t);
+    node->set_next_edges(torch::autograd::collect_next_edges(*input.t, one_input || !c.x ? Variable() : *given.x.t, variable(weight_proj), *weight.t,
+                                                             *given.weight_c.t, *given.bias.t, variable(given.init)));
+    node->kept.keep(c, states);
+    node->one_input = one_input;
+    node->has_proj = (bool)weight_proj;
+    node->input_type = input->scalar_type();
+    node->weight_type = weight->scalar_type();
+    if (weight_proj) node->proj_type = weight_proj->scalar_type();
+    // (of the products' operands those that some gradient needs)
+    const bool first = wants(input) || wants(weight_proj);
+    if (weight_proj || wants(weight)) node->operand = SavedVariable(operand, false);
+    if (weight_proj && wants(weight)) node->projected = SavedVariable(projected, false);
+    if (weight_proj ? first : wants(input)) node->weight = SavedVariable(weight_operand, false);
+    if (weight_proj) node->weight_proj = SavedVariable(proj_operand, false);
+    torch::autograd::create_gradient_edge(h, node);
+    torch::autograd::create_gradient_edge(last, node);
+    return Py_BuildValue("(NN)", wrap(h), wrap(last));
+    END_HANDLE_TH_ERRORS
 }
 
 // layer_forward(x, residual, weight_proj, weight, weight_c, bias, init, act, d, bidirectional, has_skip, scale, mask_pad)
@@ -508,6 +839,8 @@ PyMethodDef methods[] = {
     {"scan_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_forward)), METH_FASTCALL, nullptr},
     {"scan_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(scan_backward)), METH_FASTCALL, nullptr},
     {"layer_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_forward)), METH_FASTCALL, nullptr},
+    {"recurrence", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(recurrence)), METH_FASTCALL, nullptr},
+    {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer)), METH_FASTCALL, nullptr},
     {"stack_forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(stack_forward)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Calls of the recurrence in the plain case.", -1, methods, nullptr, nullptr, nullptr, nullptr};

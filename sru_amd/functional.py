@@ -345,10 +345,15 @@ def _grad_workspace(dtype, rows, inner, cols):
     return _lib.load().sru_amd_product_grad_workspace_bytes(_DTYPES[dtype], rows, inner, cols)
 
 
+def _transformed() -> bool:
+    """Whether torch's calls are traced, compiled or transformed."""
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _observed() -> bool:
     """Whether something records, transforms or compiles torch's calls: then a product is one of them."""
-    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or _lib.host().observed()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0)
+    return _transformed() or _lib.host().observed()
 
 
 def _weight_gradient(x: Tensor, grad: Tensor, dtype: torch.dtype) -> Tensor:
@@ -441,6 +446,14 @@ def dense(x: Tensor, weight: Tensor) -> Tensor:
     return x.mm(weight) if out is None else out     # (in one place: a trace is compared with its repetition line by line)
 
 
+_STEPS = _weight_gradient, _grad_workspace
+
+
+def replaced() -> bool:
+    """Whether another function stands for a step of a layer with gradients, which then has to be called."""
+    return (_weight_gradient, _grad_workspace) != _STEPS or ElementwiseRecurrence.apply != _APPLY
+
+
 class ElementwiseRecurrence(Function):
     """Drop-in for sru/cuda_functional.py:156-261.
 
@@ -483,61 +496,92 @@ class ElementwiseRecurrence(Function):
 
     @staticmethod
     def backward(ctx, grad_h, grad_last):
-        pb = ctx.problem
         saved = list(ctx.saved_tensors)
-        if pb is None:
-            if grad_h is not None:
-                done = _lib.host().scan_backward(*saved, grad_h, grad_last, *ctx.call)
-                if done is not None:
-                    return done + (None,) * 7
-            # (a gradient that is missing, strided or of another dtype, or tensors that a saved-tensor
-            # hook gave back differently)
-            u, x, weight_c, bias, init, scale_x, mask_c, mask_pad, c = saved
-            activation_type, d_out, bidirectional, has_skip_term, length, batch = ctx.call
-            pb = _problem_cached(u.dtype, 3, length, batch, u.numel(), u.size(-1), 0, d_out, bool(bidirectional),
-                                 bool(has_skip_term), int(activation_type), True, x is not None and x.dtype == torch.float32, True)
-            (u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_), _ = _prepare_inputs(
-                pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
-            c = c.contiguous()
-            x_like = u if x is None else x     # (no gradient goes to an x that the skip term does not read)
-            in_dtypes = (u.dtype, x_like.dtype, weight_c.dtype, bias.dtype, None if init is None else init.dtype)
-            in_shapes = (u.shape, x_like.shape, weight_c.shape, bias.shape, None if init is None else init.shape)
-        else:
-            c = saved.pop()
-            it = iter(saved)
-            u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_ = [next(it) if p else None for p in ctx.present]
-            in_dtypes, in_shapes = ctx.in_dtypes, ctx.in_shapes
-        dev = u_.device
-        if grad_h is None:     # only last_hidden was used downstream
-            gh = torch.zeros(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
-        else:
-            gh = _aligned(grad_h if grad_h.dtype == pb.dtype else grad_h.to(pb.dtype), 4)
-        # (None: the kernels start from a zero state gradient; 16 bits are read as they are)
-        narrow_last = grad_last is not None and grad_last.dtype == pb.dtype and pb.dtype in _NARROW and _plain(grad_last)
-        gl = grad_last.contiguous() if narrow_last else _small(grad_last, pb.small_dtype)
-        grad_u = torch.empty_like(u_)
-        grad_x = torch.empty_like(x_) if pb.skip_type == 1 else None
-        grad_wc = torch.empty_like(wc_) if pb.is_custom else \
-            torch.empty(2 * pb.Dp, dtype=pb.small_dtype, device=dev)
-        # grad_bias (2, D') and grad_init (B, D') share one allocation
-        small = torch.empty((2 + pb.batch) * pb.Dp, dtype=pb.small_dtype, device=dev)
-        grad_bias, grad_init = small[:2 * pb.Dp], small[2 * pb.Dp:]
-        ws_bytes = pb.workspace_bytes
-        workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=dev)
-        with _on_device(dev) as stream:
-            rc = _lib.load().sru_amd_backward_small(
-                ctypes.byref(pb.shape), _lib.SMALL_LAST if narrow_last else 0, _ptr(u_), _ptr(x_), _ptr(wc_), _ptr(bias_), _ptr(init_),
-                _ptr(mask_c_), _ptr(pad_), _ptr(scale_), _ptr(c), _ptr(gh), _ptr(gl),
-                _ptr(grad_u), _ptr(grad_x), _ptr(grad_wc), _ptr(grad_bias), _ptr(grad_init),
-                _ptr(workspace), ctypes.c_size_t(ws_bytes), stream)
-        _lib.check(rc, "sru_amd_backward_small")
-        u_dt, x_dt, wc_dt, bias_dt, init_dt = in_dtypes
-        u_sh, x_sh, wc_sh, bias_sh, init_sh = in_shapes
-        grad_u = grad_u.view(u_sh).to(u_dt)
-        if grad_x is not None:
-            grad_x = grad_x.view(x_sh).to(x_dt)
-        grad_wc = grad_wc.view(wc_sh).to(wc_dt)
-        grad_bias = grad_bias.view(bias_sh).to(bias_dt)
-        grad_init = None if init_sh is None else grad_init.view(init_sh).to(init_dt)
-        return grad_u, grad_x, grad_wc, grad_bias, grad_init, \
-            None, None, None, None, None, None, None
+        if ctx.problem is None:
+            return _scan_gradients(saved, ctx.call, grad_h, grad_last) + (None,) * 7
+        c = saved.pop()
+        it = iter(saved)
+        prepared = [next(it) if p else None for p in ctx.present]
+        return _prepared_gradients(ctx.problem, *prepared, c, ctx.in_dtypes, ctx.in_shapes, grad_h, grad_last) + (None,) * 7
+
+
+_General = ElementwiseRecurrence
+
+
+class ElementwiseRecurrence(_General):
+    __doc__ = _General.__doc__
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is not ElementwiseRecurrence or cls.forward is not _FORWARD or cls.backward is not _BACKWARD:
+            return super().apply(*args, **kwargs)
+        if not torch.compiler.is_compiling() and not kwargs and 10 <= len(args) <= 12:
+            done = _recurrence(*args)
+            if done is not None:
+                return done
+        return _General.apply(*args, **kwargs)    # (a class that torch.compile knows how to follow)
+
+
+_FORWARD, _BACKWARD, _APPLY = ElementwiseRecurrence.forward, ElementwiseRecurrence.backward, ElementwiseRecurrence.apply
+
+
+def _recurrence(u, x, weight_c, bias, init, activation_type, d_out, bidirectional, has_skip_term, scale_x, mask_c=None, mask_pad=None):
+    """The Function's call in the plain case, as a node of the native host code; None otherwise."""
+    native = getattr(_lib.host(), "recurrence", None)
+    return None if native is None or _transformed() else native(u, x, weight_c, bias, init, activation_type, d_out, bidirectional, has_skip_term, scale_x,
+                                              mask_c, mask_pad)
+
+
+def _scan_gradients(saved, call, grad_h, grad_last):
+    """Gradients of u, x, weight_c, bias and init from the tensors of a plain forward call."""
+    if grad_h is not None:
+        done = _lib.host().scan_backward(*saved, grad_h, grad_last, *call)
+        if done is not None:
+            return done
+    # (a gradient that is missing, strided or of another dtype, or tensors that a saved-tensor
+    # hook gave back differently)
+    u, x, weight_c, bias, init, scale_x, mask_c, mask_pad, c = saved
+    activation_type, d_out, bidirectional, has_skip_term, length, batch = call
+    pb = _problem_cached(u.dtype, 3, length, batch, u.numel(), u.size(-1), 0, d_out, bool(bidirectional),
+                         bool(has_skip_term), int(activation_type), True, x is not None and x.dtype == torch.float32, True)
+    prepared, _ = _prepare_inputs(pb, u, x, weight_c, bias, init, scale_x, mask_c, mask_pad)
+    x_like = u if x is None else x     # (no gradient goes to an x that the skip term does not read)
+    in_dtypes = (u.dtype, x_like.dtype, weight_c.dtype, bias.dtype, None if init is None else init.dtype)
+    in_shapes = (u.shape, x_like.shape, weight_c.shape, bias.shape, None if init is None else init.shape)
+    return _prepared_gradients(pb, *prepared, c.contiguous(), in_dtypes, in_shapes, grad_h, grad_last)
+
+
+def _prepared_gradients(pb, u_, x_, wc_, bias_, init_, scale_, mask_c_, pad_, c, in_dtypes, in_shapes, grad_h, grad_last):
+    dev = u_.device
+    if grad_h is None:     # only last_hidden was used downstream
+        gh = torch.zeros(pb.length, pb.batch, pb.Dp, dtype=pb.dtype, device=dev)
+    else:
+        gh = _aligned(grad_h if grad_h.dtype == pb.dtype else grad_h.to(pb.dtype), 4)
+    # (None: the kernels start from a zero state gradient; 16 bits are read as they are)
+    narrow_last = grad_last is not None and grad_last.dtype == pb.dtype and pb.dtype in _NARROW and _plain(grad_last)
+    gl = grad_last.contiguous() if narrow_last else _small(grad_last, pb.small_dtype)
+    grad_u = torch.empty_like(u_)
+    grad_x = torch.empty_like(x_) if pb.skip_type == 1 else None
+    grad_wc = torch.empty_like(wc_) if pb.is_custom else \
+        torch.empty(2 * pb.Dp, dtype=pb.small_dtype, device=dev)
+    # grad_bias (2, D') and grad_init (B, D') share one allocation
+    small = torch.empty((2 + pb.batch) * pb.Dp, dtype=pb.small_dtype, device=dev)
+    grad_bias, grad_init = small[:2 * pb.Dp], small[2 * pb.Dp:]
+    ws_bytes = pb.workspace_bytes
+    workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=dev)
+    with _on_device(dev) as stream:
+        rc = _lib.load().sru_amd_backward_small(
+            ctypes.byref(pb.shape), _lib.SMALL_LAST if narrow_last else 0, _ptr(u_), _ptr(x_), _ptr(wc_), _ptr(bias_), _ptr(init_),
+            _ptr(mask_c_), _ptr(pad_), _ptr(scale_), _ptr(c), _ptr(gh), _ptr(gl),
+            _ptr(grad_u), _ptr(grad_x), _ptr(grad_wc), _ptr(grad_bias), _ptr(grad_init),
+            _ptr(workspace), ctypes.c_size_t(ws_bytes), stream)
+    _lib.check(rc, "sru_amd_backward_small")
+    u_dt, x_dt, wc_dt, bias_dt, init_dt = in_dtypes
+    u_sh, x_sh, wc_sh, bias_sh, init_sh = in_shapes
+    grad_u = grad_u.view(u_sh).to(u_dt)
+    if grad_x is not None:
+        grad_x = grad_x.view(x_sh).to(x_dt)
+    grad_wc = grad_wc.view(wc_sh).to(wc_dt)
+    grad_bias = grad_bias.view(bias_sh).to(bias_dt)
+    grad_init = None if init_sh is None else grad_init.view(init_sh).to(init_dt)
+    return grad_u, grad_x, grad_wc, grad_bias, grad_init

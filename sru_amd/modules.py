@@ -19,7 +19,7 @@ import torch.nn as nn
 from torch import Tensor
 from torch.nn.utils.rnn import PackedSequence, pad_packed_sequence, pack_padded_sequence
 
-from . import _lib
+from . import _lib, functional
 from .functional import dense, layer_forward
 from .norm import layer_norm as fused_layer_norm, supported as fused_layer_norm_supported
 from .ops import elementwise_recurrence_gpu
@@ -153,11 +153,28 @@ class SRUCell(nn.Module):
                     h = self._normalise(h, feeds_projection=False)
                 return h, c
 
-        U, V = self.compute_UV(input, c0, mask_pad)
-        h, c = self.apply_recurrence(U, V, residual, c0, scale_val, mask_c, mask_pad)
+        done = self._native_layer(input, residual, c0, scale_val, mask_c, mask_pad) if torch.is_grad_enabled() else None
+        if done is not None:
+            h, c = done
+        else:
+            U, V = self.compute_UV(input, c0, mask_pad)
+            h, c = self.apply_recurrence(U, V, residual, c0, scale_val, mask_c, mask_pad)
         if self.layer_norm is not None and self.normalize_after:
             h = self._normalise(h, feeds_projection=False)
         return h, c
+
+    def _native_layer(self, input: Tensor, residual: Tensor, c0: Optional[Tensor], scale_val: Optional[Tensor], mask_c: Optional[Tensor],
+                      mask_pad: Optional[Tensor]) -> Optional[Tuple[Tensor, Tensor]]:
+        """compute_UV and apply_recurrence with gradients, as one node of the graph, where the layer projects with its own
+        weights, no step is overridden or replaced, and nothing watches, transforms or compiles torch's calls."""
+        if (torch.compiler.is_compiling() or self.custom_m is not None or not getattr(self, "native_16bit", True) or input.size(-1) != self.input_size
+                or getattr(self.compute_UV, "__func__", None) is not _COMPUTE_UV or getattr(self.compute_U, "__func__", None) is not _COMPUTE_U
+                or getattr(self.apply_recurrence, "__func__", None) is not _APPLY_RECURRENCE
+                or dense is not _DENSE or elementwise_recurrence_gpu is not _RECURRENCE_GPU or functional.replaced()):
+            return None
+        native = getattr(_lib.host(), "layer", None)
+        return None if native is None or functional._transformed() else native(input, residual, self.weight_proj, self.weight, self.weight_c, self.bias, c0, self.activation_type,
+                                                  self.hidden_size, self.bidirectional, self.has_skip_term, scale_val, mask_c, mask_pad)
 
     def _whole_layer(self, input: Tensor, residual: Tensor) -> bool:
         """Whether `layer_forward` may stand for compute_UV and apply_recurrence: nothing is
@@ -266,7 +283,7 @@ _COMPUTE_UV, _COMPUTE_U, _APPLY_RECURRENCE = SRUCell.compute_UV, SRUCell.compute
 # ... and what a stack's one call stands for: whole cells, as torch calls them.
 _CELL_METHODS = tuple((name, getattr(SRUCell, name)) for name in ("__call__", "forward", "compute_UV", "compute_U", "apply_recurrence",
                                                                   "_whole_layer", "_normalise"))
-_LAYER_FORWARD = layer_forward
+_LAYER_FORWARD, _DENSE, _RECURRENCE_GPU = layer_forward, dense, elementwise_recurrence_gpu
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks,
                  torch.nn.modules.module._global_backward_hooks, torch.nn.modules.module._global_backward_pre_hooks)
 
