@@ -259,8 +259,8 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
                           void *h, void *c_last, void *stream);
 
 /* A stack of such layers, each of the width of its input, in one launch (two with the clearing of the workspace): one time
- * step, or a sequence in one direction of at most 64 batch rows, through up to SRU_AMD_STACK_MAX_LAYERS layers of one
- * form (sru/modules.py:617-652, a loop over the layers there). `shape` is that of each layer's recurrence (16-bit streams, k 3,
+ * step of up to 64 rows, or a sequence of one or two batch rows in one direction, through up to SRU_AMD_STACK_MAX_LAYERS layers of
+ * one form (sru/modules.py:617-652, a loop over the layers there). `shape` is that of each layer's recurrence (16-bit streams, k 3,
  * skip_type 0 or 1, is_custom 0).
  *
  * sru_amd_stack_workspace_bytes: 0 where there is no kernel for the stack or the layers one by one are the faster way.

@@ -10,7 +10,7 @@ ROOT = os.path.dirname(HERE)
 SOURCES = [os.path.join(HERE, "csrc", n)
            for n in ("sru_amd.hip", "sru_norm.hip", "scan_f32_fwd.hip", "scan_f32_bwd.hip", "scan_f16_fwd.hip",
                      "scan_f16_bwd.hip", "scan_bf16_fwd.hip", "scan_bf16_bwd.hip", "scan_f64.hip", "layer_step.hip",
-                     "layer_rows.hip", "layer_stack.hip", "product.hip", "product_grad.hip")]
+                     "layer_rows.hip", "layer_stack.hip", "prompt_stack.hip", "product.hip", "product_grad.hip")]
 OUTPUT = os.path.join(HERE, "libsru_amd.so")
 OBJ_DIR = os.path.join(HERE, "csrc", "build")
 HOST_MODULE = os.path.join(HERE, "_host.so")

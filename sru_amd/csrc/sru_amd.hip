@@ -349,9 +349,8 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
 size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers, int64_t n_proj) {
     if (check_shape(shape) != SRU_AMD_OK || n_proj < 0) return 0;
     const sru_amd_shape &s = *shape;
-    const int64_t Dp = s.hidden * s.dirs;
-    if (elem_size(s.dtype) != 2 || s.is_custom || x_is_float_beside_16bit(s) || s.k != 3 || s.length != 1 || !stack_sizes_ok(layers, s.batch, Dp, n_proj)) return 0;
-    return stack_workspace(layers, s.batch, Dp, n_proj);
+    if (elem_size(s.dtype) != 2 || s.is_custom || x_is_float_beside_16bit(s) || s.k != 3 || (s.length > 1 && s.dirs != 1)) return 0;
+    return stack_plan(layers, s.length, s.batch, s.hidden * s.dirs, n_proj).bytes;
 }
 
 int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t layers, int64_t n_proj, const void *x,
@@ -378,10 +377,11 @@ int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
     if (!aligned(x, 16) || !aligned(h, 16) || !aligned(c_init, small_align(SRU_AMD_SMALL_INIT)) || !aligned(c_last, small_align(SRU_AMD_SMALL_LAST)))
         return SRU_AMD_ERR_MISALIGNED;
     p.x = x; p.c0 = c_init; p.pad = mask_pad; p.h = h; p.c_last = c_last;
-    p.layers = (int32_t)layers; p.rows = (int32_t)s.batch; p.Dp = (int32_t)(s.hidden * s.dirs); p.n_proj = (int32_t)n_proj;
-    p.outputs_at = stack_outputs_at(layers, s.batch, n_proj);
+    p.layers = (int32_t)layers; p.rows = (int32_t)(s.length * s.batch); p.Dp = (int32_t)(s.hidden * s.dirs); p.n_proj = (int32_t)n_proj;
+    const StackPlan plan = stack_plan(layers, s.length, s.batch, p.Dp, n_proj);
+    p.batch = (int32_t)s.batch; p.steps = plan.steps; p.chunks = plan.chunks; p.outputs_at = plan.outputs_at; p.states_at = plan.states_at;
     p.act = s.activation_type; p.skip = s.skip_type == 1; p.small16 = small16;
-    const hipError_t err = launch_layer_stack(p, workspace, need, s.dtype == SRU_AMD_F16, static_cast<hipStream_t>(stream));
+    const hipError_t err = (s.length == 1 ? launch_layer_stack : launch_prompt_stack)(p, workspace, need, s.dtype == SRU_AMD_F16, static_cast<hipStream_t>(stream));
     return err == hipSuccess ? SRU_AMD_OK : SRU_AMD_ERR_LAUNCH;
 }
 

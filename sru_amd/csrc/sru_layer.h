@@ -106,10 +106,11 @@ struct StackParams {
     const uint8_t *pad;
     void *h, *c_last;
     uint32_t *ticket;
-    char *exchange;           // projected rows of every layer, outputs of every layer but the last
-    int64_t outputs_at;
+    char *exchange;           // projected rows of every layer, outputs of every layer but the last, states between chunks
+    int64_t outputs_at, states_at;
     int32_t layers, rows, Dp, n_proj, pieces, act, skip;
     uint32_t small16;
+    int32_t batch, steps, chunks;   // of a sequence: rows is length * batch
 };
 // Where the step kernels take each of the layers, of which there have to be two. Layer by layer / in one launch, bf16, us a pass,
 // launched one by one and in a graph (8 layers unless another number is given):
@@ -124,10 +125,45 @@ struct StackParams {
 inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
     return layers >= 2 && layers <= kStackMaxLayers && n_proj < Dp && step_sizes_ok(rows, Dp, Dp, n_proj);
 }
-inline int64_t stack_outputs_at(int64_t layers, int64_t rows, int64_t n_proj) { return layers * rows * n_proj * 2; }
-inline size_t stack_workspace(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
-    return kStackHeader + (size_t)(stack_outputs_at(layers, rows, n_proj) + (layers - 1) * rows * Dp * 2);
+// A sequence of one or two batch rows through such a stack (prompt_stack.hip): time steps in a chunk, 0 where the layers one
+// by one are as fast or nearly so.
+//
+// What it saves is the walk that follows the walk of the layer before, per layer; what it costs is products in pieces of 64 rows
+// and less, 300-400 TFLOP/s in all. So: few rows, inner sizes that pass through LDS at once (more of them where the walk is
+// long), and enough layers. Chunks of 32 rows where the chunks are few or their pieces small: they are handed on sooner.
+// Layer by layer / chunks of 64 rows / 32, bf16, us a pass, launched one by one (in a graph the gain is 0-10% less):
+//   one row   512 x 2048 -> 512, 10 layers 418/332/401    1024 of the same 645/553/712     128 of the same 229/164/171
+//             370 x 256, 10 layers 207/120/94     491 x 1024, 6 layers 215/175/221  230 x 512 -> 128, 4 layers 79/67/60
+//             386 x 2048, 4 layers 167/212/299    194 x 1024, 4 layers 81/81/80     175 x 640, 2 layers 35/43/40
+//   two rows  512 x 512, 4 layers 119/90/114      462 x 128, 6 layers 139/84/82     512 x 2048 -> 512, 10 layers 475/519/692
+//   four      806 x 512, 8 layers 382/404/554     512 x 1024 -> 256, 6 layers 249/523/740
+constexpr int kStackRows = 64;        // rows of a chunk at the most
+inline int prompt_steps(int64_t layers, int64_t length, int64_t batch, int64_t Dp, int64_t n_proj) {
+    const int64_t inner = n_proj ? n_proj : Dp;
+    if (layers < 3 || layers > kStackMaxLayers || length < 64 || length > 4096 || batch > 2 || Dp % 32 != 0 || n_proj % 32 != 0 || n_proj >= Dp || Dp > 2048 ||
+        inner > (length >= 256 ? 1024 : 512) || (batch == 2 && (n_proj || Dp > 512)))
+        return 0;
+    const int64_t rows = length * batch <= 256 || Dp <= 256 ? kStackRows / 2 : kStackRows;
+    return (int)(rows / batch);
 }
+struct StackPlan {
+    int steps, chunks;
+    int64_t outputs_at, states_at;
+    size_t bytes;
+};
+inline StackPlan stack_plan(int64_t layers, int64_t length, int64_t batch, int64_t Dp, int64_t n_proj) {
+    StackPlan plan{};
+    plan.steps = length == 1 ? (int)stack_sizes_ok(layers, batch, Dp, n_proj) : prompt_steps(layers, length, batch, Dp, n_proj);
+    if (plan.steps == 0) return plan;
+    const int64_t rows = length * batch;
+    plan.chunks = (int)((length + plan.steps - 1) / plan.steps);
+    plan.outputs_at = layers * rows * n_proj * 2;
+    plan.states_at = plan.outputs_at + (layers - 1) * rows * Dp * 2;
+    plan.bytes = kStackHeader + (size_t)(plan.states_at + layers * (plan.chunks - 1) * batch * Dp * 4);
+    return plan;
+}
+hipError_t clear_exchange(StackParams &p, void *workspace, size_t bytes, hipStream_t st);   // and sets where it is
+hipError_t launch_prompt_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st);
 hipError_t launch_layer_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st);
 
 // A product by itself (product.hip): x (rows, inner) times weight (inner, cols), all in one type.

@@ -1,5 +1,5 @@
-"""One time step of a whole stack in one launch (sru_amd_stack_forward) against the same layers called one by one, which
-test_gpu_layer_forward.py holds against float64."""
+"""Whole stacks in one launch (sru_amd_stack_forward), one time step or a short sequence, against the same layers called one by
+one, which test_gpu_layer_forward.py holds against float64."""
 import threading
 
 import pytest
@@ -63,6 +63,46 @@ def test_one_step(d, kw, batch, dtype):
     check(model, x, c0.float())
 
 
+# sequences: chunks of 32 rows and of 64, a last chunk of few steps, a second half of rows that is not there, a last group of
+# 32 cells, one row and two, inner sizes below, at and past what passes through LDS at once
+SEQUENCES = [(64, 1, 32, {}), (65, 1, 96, dict(projection_size=32)), (100, 2, 64, dict(use_tanh=True)), (257, 1, 288, {}), (300, 1, 544, dict(projection_size=96)),
+             (289, 1, 512, dict(has_skip_term=False)), (290, 1, 544, {}), (129, 2, 480, {}), (130, 1, 1024, dict(projection_size=512)),
+             (513, 1, 2048, dict(projection_size=512)), (300, 1, 1024, dict(projection_size=992))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("length,batch,d,kw", SEQUENCES)
+def test_sequences(length, batch, d, kw, dtype):
+    model = make(d, dtype, **kw)
+    x = torch.randn(length, batch, d, device="cuda").to(dtype)
+    c0 = torch.randn(3, batch, d, device="cuda").to(dtype)
+    pad = torch.rand(length, batch, device="cuda") < 0.3
+    pad[-3:] = True
+    with torch.no_grad():
+        for state, mask in ((None, None), (c0, pad), (c0.float(), None)):
+            assert model._whole_stack(x, state, mask) is not None
+            got, want = model(x, state, mask_pad=mask), one_by_one(model, x, state, mask_pad=mask)
+            wide = model.float()(x.float(), None if state is None else state.float(), mask_pad=mask)
+            model.to(dtype)
+            for a, b, exact in zip(got, want, wide):
+                # U stays in float here and is rounded on the way to the recurrence there: no further from the result in
+                # float throughout, of which both are a few roundings of 16 bits per layer away
+                exact, norm = exact.double(), exact.double().norm()
+                assert float((a.double() - exact).norm() / norm) <= 1.05 * float((b.double() - exact).norm() / norm)
+                assert float((a.double() - b.double()).norm() / norm) <= 4 * EPS[dtype]
+                if mask is not None and a.shape[0] == length:
+                    assert not bool(a[mask].any())
+
+
+@pytest.mark.parametrize("length,batch,d,kw,taken", [(64, 1, 64, {}, True), (63, 1, 64, {}, False), (64, 3, 64, {}, False), (64, 1, 48, {}, False),
+                                                    (64, 1, 544, {}, False), (256, 1, 544, {}, True), (256, 1, 1056, {}, False),
+                                                    (64, 2, 64, dict(projection_size=32), False), (64, 1, 64, dict(bidirectional=True), False)])
+def test_sequences_that_are_taken(length, batch, d, kw, taken):
+    model = make(d, torch.bfloat16, **kw)
+    with torch.no_grad():
+        assert (model._whole_stack(torch.zeros(length, batch, model.output_size, device="cuda", dtype=torch.bfloat16), None, None) is not None) == taken
+
+
 @pytest.mark.parametrize("layers,taken", [(1, False), (2, True), (16, True), (17, False)])
 def test_numbers_of_layers(layers, taken):
     model = make(256, torch.bfloat16, layers)
@@ -92,8 +132,8 @@ def test_nans_and_the_pattern_that_stands_for_nothing():
 
 
 def test_streams_and_threads():
-    models = [make(512, torch.bfloat16, 8, projection_size=128), make(320, torch.float16, 6)]
-    inputs = [torch.randn(1, 16, m.output_size, device="cuda").to(m.rnn_lst[0].weight.dtype) for m in models]
+    models = [make(512, torch.bfloat16, 8, projection_size=128), make(320, torch.float16, 6), make(256, torch.bfloat16, 5)]
+    inputs = [torch.randn(length, batch, m.output_size, device="cuda").to(m.rnn_lst[0].weight.dtype) for m, length, batch in zip(models, (1, 1, 150), (16, 16, 1))]
     with torch.no_grad():
         want = [m(x) for m, x in zip(models, inputs)]
     torch.cuda.synchronize()
@@ -103,11 +143,11 @@ def test_streams_and_threads():
         stream = torch.cuda.Stream()
         with torch.no_grad(), torch.cuda.stream(stream):
             for _ in range(50):
-                h, c = models[i % 2](inputs[i % 2])
-                if not (torch.equal(h, want[i % 2][0]) and torch.equal(c, want[i % 2][1])):
+                h, c = models[i % 3](inputs[i % 3])
+                if not (torch.equal(h, want[i % 3][0]) and torch.equal(c, want[i % 3][1])):
                     wrong.append(i)
 
-    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
     for t in threads:
         t.start()
     for t in threads:
@@ -116,9 +156,10 @@ def test_streams_and_threads():
     assert not wrong
 
 
-def test_recorded_and_replayed():
+@pytest.mark.parametrize("length,batch", [(1, 16), (130, 1)])
+def test_recorded_and_replayed(length, batch):
     model = make(256, torch.bfloat16, 4, projection_size=64)
-    x = torch.randn(1, 16, 256, device="cuda").to(torch.bfloat16)
+    x = torch.randn(length, batch, 256, device="cuda").to(torch.bfloat16)
     with torch.no_grad():
         model(x)
         torch.cuda.synchronize()
@@ -126,7 +167,7 @@ def test_recorded_and_replayed():
         with torch.cuda.graph(graph):
             h, c = model(x)
         for _ in range(5):
-            x.copy_(torch.randn(1, 16, 256, device="cuda"))
+            x.copy_(torch.randn(length, batch, 256, device="cuda"))
             graph.replay()
             want_h, want_c = model(x.clone())
             assert torch.equal(h, want_h) and torch.equal(c, want_c)
