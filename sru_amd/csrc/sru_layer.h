@@ -225,22 +225,24 @@ struct GradParams {
 // The tile of the workgroups (128 columns of x by tile_n of g) and the number of parts of the rows; 0: the library's
 // product is not slower, or a size is not a whole number of 16-byte pieces.
 //
-// One round of workgroups, one to each of 256 compute units: a tile of 64 rows takes 0.66 us with 128 columns and
-// 0.88 with 192, the slices are written and read at 3.5 TB/s, and the sum of both is least. Measured (us, library
-// product with conversion / 128 columns / 192, with the best number of parts each, the rule's choice marked *):
-//   8192 rows   512 x 6144   103/96/77*     2048 x 512   58/33*/38    1024 x 3072  86/90/73*    256 x 1024  55/21*/24
-//   4096 rows   512 x 1536   32/23*/25      256 x 3072   32/21*/23    1024 x 3072  49/52/46*
-//   16384 rows  512 x 3072   148/92/75*     1024 x 8192  283/314/399
-//   2048 rows   512 x 3072   25/25/26       2048 x 512   21/19/22
-// More rows and smaller results are the library's worst (32768 rows, 512 x 512 155 -> 36; 16384 rows, 128 x 2048 132 ->
-// 25); where the rows are not split it is level or faster (4096 rows, 768 x 4096 51 / 54). Of 120 sizes drawn at random
-// that are taken one was slower (55393 rows, 576 x 3264 286 / 297).
+// At most one round of workgroups, one to each of 256 compute units: a pair of tiles of 64 rows takes 1.12 us with 128
+// columns and 1.52 with 192, the slices are written and read at 2.5 TB/s, and the sum of both is least. Measured (us,
+// library product with conversion / 128 columns / 192, with the best number of parts each, the rule's choice marked *):
+//   8192 rows   512 x 6144   92/77/65*      2048 x 512   56/30*/33    1024 x 3072  83/73/63*    256 x 1024  54/20*/23
+//   4096 rows   512 x 1536   30/22*/24      256 x 3008   34/20*/22    1024 x 3072  49/43/40*
+//   16384 rows  512 x 3072   125/72/63*     10195 rows, 1152 x 976  89/40*/43
+// More rows and smaller results are the library's worst (38185 rows, 568 x 688 240 -> 51).
+// 67 sizes drawn at random that are split take 0.40 of the library's time, the worst 0.82. Rows that are not split take
+// one launch where the gradient is float. With 192 columns they take 0.75 of its time over 28 sizes (9682 rows, 1024 x
+// 4384 188 -> 112; 3782 rows, 1552 x 2480 58 -> 52), but from 25000 rows on, where the library's larger tiles settle in,
+// five sizes lie between 0.78 and 1.17 (32951 rows, 1016 x 4544 340 -> 396) and are left to it, as is what 128 columns
+// would be better for (0.73 to 0.89). Beyond one round it is faster (16384 rows, 2048 x 6144 362 / 453).
 struct GradPlan { int tile_n, splits; };
 // A call costs its host some 25 us more than torch's: taken from 8192 rows on, where the library loses more than that
 // (8192 rows, 256 x 256 50/17, 128 x 512 70/17; 16384 rows, 256 x 768 95/24), below where the products keep the GPU
 // busier than the host (from 3000 rows and 3e9 multiply-adds; 4096 rows, 256 x 1024 30/17 is left alone). More than 16
 // parts were no faster anywhere.
-constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384;
+constexpr int64_t kGradMinRows = 3000, kGradManyRows = 8192, kGradMinWork = 3000000000, kGradMinResult = 128 * 384, kGradWholeRows = 24576;
 inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {
     if (rows < kGradMinRows || rows > (1 << 24) || inner > (1 << 16) || cols > (1 << 16) || inner < 128 || cols < 128 || inner % 8 != 0 || cols % 8 != 0 || inner * cols < kGradMinResult ||
         (rows < kGradManyRows && rows * inner * cols < kGradMinWork) || rows * inner >= (1 << 30) || rows * cols >= (1 << 30))   // (31-bit byte offsets)
@@ -249,15 +251,15 @@ inline GradPlan product_grad_plan(int64_t rows, int64_t inner, int64_t cols) {
     int64_t least = 0;
     for (const int tile_n : {128, 192}) {
         const int64_t tiles = (inner + 127) / 128 * ((cols + tile_n - 1) / tile_n);
-        for (int64_t splits = 1; splits == 1 || (splits <= 16 && tiles * splits <= 256 && splits * 256 <= rows); ++splits) {
-            const int64_t walk = ((rows + 63) / 64 + splits - 1) / splits * ((tiles * splits + 255) / 256) * (tile_n == 128 ? 660 : 880);   // ns
-            const int64_t cost = walk + splits * inner * cols * 8 / 3500;
+        for (int64_t splits = 1; splits <= 16 && tiles * splits <= 256 && splits * 256 <= rows; ++splits) {
+            const int64_t pairs = ((rows + 63) / 64 + 2 * splits - 1) / (2 * splits);
+            const int64_t cost = pairs * (tile_n == 128 ? 1120 : 1520) + splits * inner * cols * 8 / 2500;   // ns
             if (best.splits == 0 || cost < least) best = GradPlan{tile_n, (int)splits}, least = cost;
         }
     }
-    return best.splits < 2 ? GradPlan{0, 0} : best;   // (no two parts of a result beyond 128 tiles of 128 x 192 fit a round)
+    return best.splits == 1 && (best.tile_n == 128 || rows > kGradWholeRows) ? GradPlan{0, 0} : best;
 }
 // p.out: room for the slices; out: the result in out_dtype (float or the 16 bits of x and g)
-hipError_t launch_product_grad(const GradParams &p, const GradPlan &plan, bool half, int32_t out_dtype, void *out, hipStream_t st);
+hipError_t launch_product_grad(GradParams p, const GradPlan &plan, bool half, int32_t out_dtype, void *out, hipStream_t st);
 
 }  // namespace sru_amd

@@ -201,3 +201,21 @@ def test_a_default_device_changes_nothing():
         assert type(functional.dense(x, w).grad_fn).__name__ == "_ProductBackward"
         with torch.no_grad():
             assert functional._short_product(*floats) is not None
+
+
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,inner,cols", [(3001, 1416, 2984), (4096, 1032, 3648), (8225, 520, 9216)])
+def test_rows_in_one_part(rows, inner, cols, out):
+    """Tiles that fill the chip by themselves: an odd and an even number of tiles of rows, cut-off tiles at every edge; a
+    float result is written by the product itself."""
+    gen = torch.Generator().manual_seed(rows)
+    x, g = (torch.randn(rows, n, generator=gen).bfloat16().cuda() for n in (inner, cols))
+    assert functional._grad_workspace(x.dtype, rows, inner, cols) == 4 * inner * cols
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        got = functional._weight_gradient(x, g, out)
+        torch.cuda.synchronize()
+    assert any("product_grad<" in e.name for e in seen.events())
+    assert any("add_slices<" in e.name for e in seen.events()) == (out != torch.float32)
+    want, spread = x.double().t() @ g.double(), (x.double().square().t() @ g.double().square()).sqrt()
+    # (as above: independent rounding errors of `rows` float sums, then the result's rounding)
+    assert ((got.double() - want).abs() <= 10 * rows ** 0.5 * 2.0 ** -24 * spread + HALF_ULP[out] * want.abs()).all()
