@@ -3,15 +3,21 @@
 //
 // What bounds it: layer after layer, a prompt of 512 steps through ten layers of 2048 features (projection 512) was ten serial
 // walks of 21 us on 32 of 256 compute units, each behind two short products, 23 us: 427 us. Here a layer starts on the first steps
-// when the layer before has done these: 332 us. 128 steps 229 -> 164, 1024 645 -> 553; 370 steps, ten layers of 256, 207 -> 94.
+// when the layer before has done these: 286 us. 128 steps 229 -> 144, 1024 640 -> 496; 370 steps, ten layers of 256, 207 -> 93.
 // What bounds it now: of the way from a layer to the next, 16 us for 64 steps, 3.7 are the projection, 7.4 the walking piece (3.0 of
-// them the walk itself, 2.8 the product), the rest handing over; and once there are many chunks on their way, workgroups
-// that wait in a compute unit's only place.
+// them the walk itself, 2.8 the product), the rest handing over; and once there are many chunks on their way, 25 us for each
+// of them, workgroups that wait in a compute unit's only place.
 //
 // Pieces. A chunk is a number of time steps of all batch rows, 64 rows at the most. Per layer and chunk there are n_proj / 32
 // pieces that project 32 columns each (sru_stack.h), and Dp / 64 that make U for 64 cells, float and never in memory, and walk
-// the chunk's steps. They are numbered along the diagonals of (layer, chunk), projections first, so that a piece only
-// reads what pieces of smaller numbers write; how they are drawn and how they hand results over is layer_stack.hip's.
+// the chunk's steps. A piece only reads what pieces of smaller numbers write; how they are drawn and how they hand results over
+// is layer_stack.hip's.
+//
+// Their order. From a layer to the next it is three times as far as from a chunk to the next, which waits for a walk alone, so a
+// layer's projection of a chunk is numbered with what is `stride` chunks further on in the layer before, and its walk `delay`
+// chunks behind it: drawn about when it can begin, a piece holds its place for less waiting. (Along the diagonals of layer and
+// chunk, a stride of one, the same prompt took 332 us, 1024 steps 560, 2048 of six layers of 512 268 -> 177; two chunks and one
+// behind 334 and 554, three and two 356 and 600, four and one 317 and 488. Chunks of 32 rows best at four and two.)
 //
 // A walking piece: 512 inner indices of all rows pass through LDS at a time (the next ones on their way in registers); of these two
 // groups of four wavefronts take one half each, and a wavefront 16 cells with their three streams, weights from memory
@@ -323,24 +329,25 @@ __global__ void __launch_bounds__(kStackThreads) prompt_stack(const StackParams 
     if (threadIdx.x == 0) control = StackControl{draw_piece(p), kPatience};
     __syncthreads();
     int number = __builtin_amdgcn_readfirstlane(control.next);
-    int diagonal = 0, before = 0;   // pieces of smaller diagonals
+    int slot = 0, before = 0;   // pieces of earlier slots
     while (number < p.pieces) {
         int drawn = 0;
         if (threadIdx.x == 0) drawn = draw_piece(p);
         // (projecting pieces are of 32 rows: registers for all that they read)
         const int n_project = again(p.n_proj) / kCells * (TILES / 2), n_walk = (again(p.Dp) + kWalkCells - 1) / kWalkCells, chunks = again(p.chunks), layers = again(p.layers);
-        int l0, pairs;
-        for (;;) {   // (ends: `number` is that of a piece of some diagonal)
-            l0 = max(0, diagonal - chunks + 1);
-            pairs = min(diagonal, layers - 1) - l0 + 1;
-            if (number < before + pairs * (n_project + n_walk)) break;
-            before += pairs * (n_project + n_walk);
-            ++diagonal;
+        const int stride = again(p.stride), delay = again(p.delay);
+        int first, pairs, first_walk, walks;   // of the slot: the lowest layer and the number of them, for either kind
+        for (;;) {   // (ends: `number` is that of a piece of some slot)
+            first = max(0, (slot - chunks + stride) / stride), first_walk = max(0, (slot - delay - chunks + stride) / stride);
+            pairs = max(0, min(slot / stride, layers - 1) - first + 1), walks = slot < delay ? 0 : max(0, min((slot - delay) / stride, layers - 1) - first_walk + 1);
+            if (number < before + pairs * n_project + walks * n_walk) break;
+            before += pairs * n_project + walks * n_walk;
+            ++slot;
         }
         int i = number - before;
         const bool project = i < pairs * n_project;
         if (!project) i -= pairs * n_project;
-        const int each = project ? n_project : n_walk, l = l0 + i / each, chunk = diagonal - l;
+        const int each = project ? n_project : n_walk, l = (project ? first : first_walk) + i / each, chunk = slot - (project ? 0 : delay) - l * stride;
         const int rows = again(p.steps) * again(p.batch), row0 = chunk * rows, R = min(rows, again(p.rows) - row0);
         if (project) {
             const int columns = i % each / (TILES / 2), from = TILES == 2 ? 0 : i % 2 * 32;
@@ -363,6 +370,8 @@ template <typename T> const void *kernel_of(int tiles, bool one) {
 hipError_t launch_prompt_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st) {
     const int tiles = p.steps * p.batch <= 32 ? 2 : 4;
     p.pieces = p.layers * p.chunks * (p.n_proj / kCells * (tiles / 2) + (p.Dp + kWalkCells - 1) / kWalkCells);
+    p.stride = tiles == 2 ? 4 : 3;
+    p.delay = p.n_proj ? p.stride - 2 : 0;
     const hipError_t e = clear_exchange(p, workspace, bytes, st);
     if (e != hipSuccess) return e;
     void *args[] = {&p};

@@ -111,6 +111,7 @@ struct StackParams {
     int32_t layers, rows, Dp, n_proj, pieces, act, skip;
     uint32_t small16;
     int32_t batch, steps, chunks;   // of a sequence: rows is length * batch
+    int32_t stride, delay;          // and its order of pieces (prompt_stack.hip)
 };
 // Where the step kernels take each of the layers, of which there have to be two. Layer by layer / in one launch, bf16, us a pass,
 // launched one by one and in a graph (8 layers unless another number is given):
@@ -125,26 +126,36 @@ struct StackParams {
 inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
     return layers >= 2 && layers <= kStackMaxLayers && n_proj < Dp && step_sizes_ok(rows, Dp, Dp, n_proj);
 }
-// A sequence of one or two batch rows through such a stack (prompt_stack.hip): time steps in a chunk, 0 where the layers one
+// A sequence of a few batch rows through such a stack (prompt_stack.hip): time steps in a chunk, 0 where the layers one
 // by one are as fast or nearly so.
 //
 // What it saves is the walk that follows the walk of the layer before, per layer; what it costs is products in pieces of 64 rows
-// and less, 300-400 TFLOP/s in all. So: few rows, inner sizes that pass through LDS at once (more of them where the walk is
-// long), and enough layers. Chunks of 32 rows where the chunks are few or their pieces small: they are handed on sooner.
-// Layer by layer / chunks of 64 rows / 32, bf16, us a pass, launched one by one (in a graph the gain is 0-10% less):
-//   one row   512 x 2048 -> 512, 10 layers 418/332/401    1024 of the same 645/553/712     128 of the same 229/164/171
-//             370 x 256, 10 layers 207/120/94     491 x 1024, 6 layers 215/175/221  230 x 512 -> 128, 4 layers 79/67/60
-//             386 x 2048, 4 layers 167/212/299    194 x 1024, 4 layers 81/81/80     175 x 640, 2 layers 35/43/40
-//   two rows  512 x 512, 4 layers 119/90/114      462 x 128, 6 layers 139/84/82     512 x 2048 -> 512, 10 layers 475/519/692
-//   four      806 x 512, 8 layers 382/404/554     512 x 1024 -> 256, 6 layers 249/523/740
+// and less. Both are estimated, in ns. Layer by layer: per layer 10 us (15 with a projection), 31 ns a step, and the product at
+// 380 TFLOP/s. In chunks: the way through the layers, which the first chunk goes alone, then per chunk the walk, and the pieces of
+// all layers on 256 compute units. Fitted to 260 measured points (three to ten layers of 64 to 2048, one to four rows, 32 to 1024
+// steps); taken where chunks of 64 rows or of 32, the better of them, are expected to take 0.93
+// of the time. At 196 of these points they took 0.73 of it, the worst 1.06 (78 x 3 rows, 3 layers of 64, 36 -> 38 us). Inner sizes beyond one pass through LDS take longer than that where the walk is short.
+// Layer by layer / chunks of 64 rows / 32, bf16, us a pass in a graph:
+//   one row   512 x 2048 -> 512, 10 layers 424/286/320    1024 of the same 640/496/628   128 of the same 229/163/144
+//             370 x 256, 10 layers 207/119/93     491 x 1024, 6 layers 215/139/133  230 x 512 -> 128, 4 layers 79/67/58
+//             936 x 2048 -> 512, 10 layers 606/457/589    54 x 2048 -> 512, 8 layers 171/131/112
+//   two rows  512 x 512, 4 layers 119/77/82       175 x 1280 -> 320, 10 layers 247/237/171
+//   three     276 x 384, 6 layers 122/86/89       104 x 2048 -> 512, 8 layers 211/171/192
+//   four      143 x 384 -> 96, 10 layers 171/139/139      346 x 2048 -> 512, 10 layers 510/605/814
 constexpr int kStackRows = 64;        // rows of a chunk at the most
 inline int prompt_steps(int64_t layers, int64_t length, int64_t batch, int64_t Dp, int64_t n_proj) {
-    const int64_t inner = n_proj ? n_proj : Dp;
-    if (layers < 3 || layers > kStackMaxLayers || length < 64 || length > 4096 || batch > 2 || Dp % 32 != 0 || n_proj % 32 != 0 || n_proj >= Dp || Dp > 2048 ||
-        inner > (length >= 256 ? 1024 : 512) || (batch == 2 && (n_proj || Dp > 512)))
+    const int64_t inner = n_proj ? n_proj : Dp, weights = n_proj ? 4 * Dp * n_proj : 3 * Dp * Dp;
+    if (layers < 3 || layers > kStackMaxLayers || length < 32 || length > 4096 || batch > 4 || Dp % 32 != 0 || n_proj % 32 != 0 || n_proj >= Dp || Dp > 2048 ||
+        inner > (length >= 256 ? 1024 : 512))
         return 0;
-    const int64_t rows = length * batch <= 256 || Dp <= 256 ? kStackRows / 2 : kStackRows;
-    return (int)(rows / batch);
+    const int64_t one_by_one = layers * (n_proj ? 15500 : 10300) + layers * length * 31 + layers * length * batch * weights / 190000;
+    const auto in_chunks = [&](int64_t rows) {
+        const int64_t chunks = (length + rows / batch - 1) / (rows / batch), walks = (Dp + 63) / 64, projections = n_proj / 32 * (rows / 32);
+        const int64_t way = (rows == 64 ? 8800 + inner * 53 / 10 : 6900 + inner * 37 / 10) + (n_proj ? 2500 : 0);
+        return layers * way + chunks * ((rows == 64 ? 2400 : 1550) + layers * (walks * inner * 29 + projections * 38000) / 1000);
+    };
+    const int64_t wide = in_chunks(kStackRows), narrow = in_chunks(kStackRows / 2);
+    return (wide < narrow ? wide : narrow) * 100 > one_by_one * 93 ? 0 : (int)((wide < narrow ? kStackRows : kStackRows / 2) / batch);
 }
 struct StackPlan {
     int steps, chunks;

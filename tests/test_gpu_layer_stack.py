@@ -63,19 +63,22 @@ def test_one_step(d, kw, batch, dtype):
     check(model, x, c0.float())
 
 
-# sequences: chunks of 32 rows and of 64, a last chunk of few steps, a second half of rows that is not there, a last group of
-# 32 cells, one row and two, inner sizes below, at and past what passes through LDS at once
-SEQUENCES = [(64, 1, 32, {}), (65, 1, 96, dict(projection_size=32)), (100, 2, 64, dict(use_tanh=True)), (257, 1, 288, {}), (300, 1, 544, dict(projection_size=96)),
-             (289, 1, 512, dict(has_skip_term=False)), (290, 1, 544, {}), (129, 2, 480, {}), (130, 1, 1024, dict(projection_size=512)),
-             (513, 1, 2048, dict(projection_size=512)), (300, 1, 1024, dict(projection_size=992))]
-
+# sequences: chunks of 32 rows and of 64, one chunk and fewer of them than lie between two layers, a last chunk of few steps, a
+# second half of rows that is not there, a last group of 32 cells, one row to four, rows that do not divide a chunk, inner
+# sizes below, at and past what passes through LDS at once, the fewest layers and the most (of some width: sixteen layers of 32
+# cells make a single rounding grow until the two errors compared below differ by chance, 0.5 to 10 over 16 inputs, 0.95 on average)
+SEQUENCES = [(32, 1, 64, {}), (64, 1, 32, {}), (64, 1, 256, dict(layers=16)), (65, 1, 96, dict(projection_size=32)), (100, 2, 64, dict(use_tanh=True)), (257, 1, 288, {}),
+             (300, 1, 544, dict(projection_size=96)), (289, 1, 512, dict(has_skip_term=False)), (290, 1, 544, {}), (129, 2, 480, dict(layers=6)),
+             (130, 4, 128, dict(layers=5, projection_size=32)), (200, 3, 256, dict(layers=6, projection_size=64)), (64, 3, 64, {}),
+             (100, 1, 2048, dict(layers=10, projection_size=512)), (513, 1, 2048, dict(layers=6, projection_size=512)),
+             (700, 1, 1280, dict(layers=10, projection_size=544)), (500, 3, 320, dict(layers=10)), (491, 1, 1024, dict(layers=6))]
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("length,batch,d,kw", SEQUENCES)
 def test_sequences(length, batch, d, kw, dtype):
     model = make(d, dtype, **kw)
     x = torch.randn(length, batch, d, device="cuda").to(dtype)
-    c0 = torch.randn(3, batch, d, device="cuda").to(dtype)
+    c0 = torch.randn(len(model.rnn_lst), batch, d, device="cuda").to(dtype)
     pad = torch.rand(length, batch, device="cuda") < 0.3
     pad[-3:] = True
     with torch.no_grad():
@@ -86,17 +89,19 @@ def test_sequences(length, batch, d, kw, dtype):
             model.to(dtype)
             for a, b, exact in zip(got, want, wide):
                 # U stays in float here and is rounded on the way to the recurrence there: no further from the result in
-                # float throughout, of which both are a few roundings of 16 bits per layer away
+                # float throughout, of which both are a few roundings of 16 bits per layer away (the norm of N independent
+                # errors varies by 1 / sqrt(2 N); the state carries one over some four steps, so of two norms' ratio
+                # three deviations are 6 / sqrt(numel))
                 exact, norm = exact.double(), exact.double().norm()
-                assert float((a.double() - exact).norm() / norm) <= 1.05 * float((b.double() - exact).norm() / norm)
+                assert float((a.double() - exact).norm() / norm) <= (1.05 + 6 / a.numel() ** 0.5) * float((b.double() - exact).norm() / norm)
                 assert float((a.double() - b.double()).norm() / norm) <= 4 * EPS[dtype]
                 if mask is not None and a.shape[0] == length:
                     assert not bool(a[mask].any())
 
 
-@pytest.mark.parametrize("length,batch,d,kw,taken", [(64, 1, 64, {}, True), (63, 1, 64, {}, False), (64, 3, 64, {}, False), (64, 1, 48, {}, False),
+@pytest.mark.parametrize("length,batch,d,kw,taken", [(32, 1, 64, {}, True), (31, 1, 64, {}, False), (64, 4, 64, {}, True), (64, 5, 64, {}, False), (64, 1, 48, {}, False),
                                                     (64, 1, 544, {}, False), (256, 1, 544, {}, True), (256, 1, 1056, {}, False),
-                                                    (64, 2, 64, dict(projection_size=32), False), (64, 1, 64, dict(bidirectional=True), False)])
+                                                    (130, 4, 128, dict(projection_size=32), False), (64, 1, 64, dict(bidirectional=True), False)])
 def test_sequences_that_are_taken(length, batch, d, kw, taken):
     model = make(d, torch.bfloat16, **kw)
     with torch.no_grad():
