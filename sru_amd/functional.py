@@ -352,8 +352,10 @@ def _transformed() -> bool:
 
 
 def _observed() -> bool:
-    """Whether something records, transforms or compiles torch's calls: then a product is one of them."""
-    return _transformed() or _lib.host().observed()
+    """Whether something records, transforms or compiles torch's calls: then a product is one of them. (In one piece with
+    what `_transformed` asks: without gradients the smallest stacks wait for every call of Python's.)"""
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or _lib.host().observed()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0)
 
 
 def _weight_gradient(x: Tensor, grad: Tensor, dtype: torch.dtype) -> Tensor:
