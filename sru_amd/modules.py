@@ -360,7 +360,7 @@ class SRU(nn.Module):
             states = list(c0.unbind(0))
 
         x = input if self.input_to_hidden is None else self.input_to_hidden(input)
-        done = None if x.dtype is torch.float32 or torch.is_grad_enabled() else self._whole_stack(x, c0, mask_pad)
+        done = None if x.dtype is torch.float32 else self._whole_stack(x, c0, mask_pad)
         if done is not None:
             x, c_stack = done
         else:
@@ -383,7 +383,7 @@ class SRU(nn.Module):
         """All layers in one call without gradients: (output, last states), or None where they are called one by one, as they
         are wherever one of them could tell the difference (see `SRUCell._whole_layer`; hooks, a method put in place of a
         cell's own, a module of another type in its place)."""
-        if (x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not Tensor or torch.compiler.is_compiling()
+        if (torch.is_grad_enabled() or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not Tensor or torch.compiler.is_compiling()
                 or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or layer_forward is not _LAYER_FORWARD
                 or type(self.rnn_lst) is not nn.ModuleList or any(getattr(SRUCell, name) is not own for name, own in _CELL_METHODS)
                 or any(_GLOBAL_HOOKS)):
