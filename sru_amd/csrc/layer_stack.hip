@@ -4,7 +4,7 @@
 // What bounds it: the step kernels (layer_step.hip) took ten layers of 2048 features (projection 512, 16 rows) 20 launches that
 // wait for each other, 5.4 and 7.9 us each, of which the weights' way from memory is a quarter. Here a workgroup takes
 // pieces of work in the order in which they depend on each other and has a piece's weights on their way before what
-// the piece reads exists: 134 -> 73 us a pass, 50 with one row (134), 184 with 64 (236); 2048 features without a projection 131 -> 89;
+// the piece reads exists: 134 -> 69 us a pass, 49 with one row (134), 174 with 64 (236); 2048 features without a projection, 8 layers, 95 -> 65;
 // six layers of 512 features 63 -> 21. Recorded in a graph 109 -> 67 (8 layers), two layers without a projection level.
 // What bounds it now, per layer and 16 rows, 6.2 us: handing 64 KB of outputs and 16 KB of projected rows over, 1.5 and 1.0 us;
 // from the arrival to the store 1.2 us each, of which the matrix instructions are a tenth and the partial sums' way through LDS half.
@@ -71,12 +71,25 @@ hipError_t clear_exchange(StackParams &p, void *workspace, size_t bytes, hipStre
     return hipLaunchKernel(reinterpret_cast<const void *>(fill_not_yet), dim3((unsigned)min((n + 255) / 256, (int64_t)2048)), dim3(256), args, 0, st);
 }
 
+// Workgroups: those of the layer at work and as many again that wait for it with their weights there already. More of them
+// only ask the memory for results that are far off: with 256 (or all pieces, if fewer) / this many, us a pass:
+//   2048 -> 512, 10 layers, 16 rows 71.3/69.4, 64 rows 177.3/174.5, one 48.4/48.9    1024 -> 256, 8 layers 47.4/43.1
+//   1536 -> 384, 8 layers 46.1/42.8    2048, 8 layers 69.7/65.1, one row 58.7/55.1   1280, 40 rows 65.9/63.0
+// Without a projection in between, a layer of few pieces is over before the weights of the next but one have arrived: as many
+// again, up to 128 in all (1024, 8 layers 36.3, 34.2 with two layers' and 30.9 with three; 512, 10 layers 33.6, 33.4, 31.0).
+// Below 48 there is nothing to gain (128, 16 layers 33.4 with 64, 35.7 with 12).
+static int stack_workgroups(const StackParams &p) {
+    const int each = p.n_proj / kCells + p.Dp / kCells;
+    const int ahead = p.n_proj ? 2 * each : min(3 * each, max(2 * each, 128));
+    return min(p.pieces, min(256, max(48, ahead)));
+}
+
 hipError_t launch_layer_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st) {
     p.pieces = p.layers * (p.n_proj / kCells + p.Dp / kCells);
     const hipError_t e = clear_exchange(p, workspace, bytes, st);
     if (e != hipSuccess) return e;
     void *args[] = {&p};
-    return hipLaunchKernel(half ? kernel_of<half_bits>(p.rows) : kernel_of<bf16_bits>(p.rows), dim3((unsigned)min(p.pieces, 256)), dim3(kStackThreads), args, 0, st);
+    return hipLaunchKernel(half ? kernel_of<half_bits>(p.rows) : kernel_of<bf16_bits>(p.rows), dim3((unsigned)stack_workgroups(p)), dim3(kStackThreads), args, 0, st);
 }
 
 }  // namespace sru_amd

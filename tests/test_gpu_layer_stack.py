@@ -63,6 +63,15 @@ def test_one_step(d, kw, batch, dtype):
     check(model, x, c0.float())
 
 
+# more pieces than workgroups: the least number of them, three layers' worth, 128, two layers' with a projection, all the chip
+@pytest.mark.parametrize("d,layers,kw", [(128, 16, {}), (576, 6, {}), (1600, 4, {}), (1024, 5, dict(projection_size=256)), (2048, 5, dict(projection_size=512)),
+                                         (2048, 4, dict(projection_size=1792))])
+def test_pieces_beyond_the_workgroups(d, layers, kw):
+    model = make(d, torch.bfloat16, layers, **kw)
+    for batch in (1, 20):
+        check(model, torch.randn(1, batch, d, device="cuda").to(torch.bfloat16))
+
+
 # sequences: chunks of 32 rows and of 64, one chunk and fewer of them than lie between two layers, a last chunk of few steps, a
 # second half of rows that is not there, a last group of 32 cells, one row to four, rows that do not divide a chunk, inner
 # sizes below, at and past what passes through LDS at once, the fewest layers and the most (of some width: sixteen layers of 32
