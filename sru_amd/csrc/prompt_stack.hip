@@ -334,26 +334,16 @@ __global__ void __launch_bounds__(kStackThreads) prompt_stack(const StackParams 
         int drawn = 0;
         if (threadIdx.x == 0) drawn = draw_piece(p);
         // (projecting pieces are of 32 rows: registers for all that they read)
-        const int n_project = again(p.n_proj) / kCells * (TILES / 2), n_walk = (again(p.Dp) + kWalkCells - 1) / kWalkCells, chunks = again(p.chunks), layers = again(p.layers);
-        const int stride = again(p.stride), delay = again(p.delay);
-        int first, pairs, first_walk, walks;   // of the slot: the lowest layer and the number of them, for either kind
-        for (;;) {   // (ends: `number` is that of a piece of some slot)
-            first = max(0, (slot - chunks + stride) / stride), first_walk = max(0, (slot - delay - chunks + stride) / stride);
-            pairs = max(0, min(slot / stride, layers - 1) - first + 1), walks = slot < delay ? 0 : max(0, min((slot - delay) / stride, layers - 1) - first_walk + 1);
-            if (number < before + pairs * n_project + walks * n_walk) break;
-            before += pairs * n_project + walks * n_walk;
-            ++slot;
-        }
-        int i = number - before;
-        const bool project = i < pairs * n_project;
-        if (!project) i -= pairs * n_project;
-        const int each = project ? n_project : n_walk, l = (project ? first : first_walk) + i / each, chunk = slot - (project ? 0 : delay) - l * stride;
-        const int rows = again(p.steps) * again(p.batch), row0 = chunk * rows, R = min(rows, again(p.rows) - row0);
-        if (project) {
-            const int columns = i % each / (TILES / 2), from = TILES == 2 ? 0 : i % 2 * 32;
-            if (from < R) piece<T, 2, 2, 8, true, true>(p, lds.parts, control, l, columns, row0 + from, min(R - from, 32));
+        const PromptOrder order = {again(p.layers), again(p.chunks), again(p.stride), again(p.delay),
+                                   again(p.n_proj) / kCells * (TILES / 2), again(p.projecting_last), (again(p.Dp) + kWalkCells - 1) / kWalkCells};
+        const PromptPiece at = prompt_piece(order, number, slot, before);
+        const int rows = again(p.steps) * again(p.batch), row0 = at.chunk * rows, R = min(rows, again(p.rows) - row0);
+        if (at.project) {
+            const int halves = min(TILES / 2, (R + 31) / 32), from = at.index % halves * 32;
+            piece<T, 2, 2, 8, true, true>(p, lds.parts, control, at.layer, at.index / halves, row0 + from, min(R - from, 32));
         } else
-            walk_piece<T, TILES, ONE_PHASE>(p, lds, control, l, chunk, i % each, row0, R);
+            walk_piece<T, TILES, ONE_PHASE>(p, lds, control, at.layer, at.chunk, at.index, row0, R);
+        // (every wavefront has read `number`: either kind of piece has a barrier, and there are no empty ones)
         if (threadIdx.x == 0) control.next = drawn;
         __syncthreads();
         number = __builtin_amdgcn_readfirstlane(control.next);
@@ -369,9 +359,11 @@ template <typename T> const void *kernel_of(int tiles, bool one) {
 
 hipError_t launch_prompt_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st) {
     const int tiles = p.steps * p.batch <= 32 ? 2 : 4;
-    p.pieces = p.layers * p.chunks * (p.n_proj / kCells * (tiles / 2) + (p.Dp + kWalkCells - 1) / kWalkCells);
-    p.stride = tiles == 2 ? 4 : 3;
-    p.delay = p.n_proj ? p.stride - 2 : 0;
+    const PromptOrder order = prompt_order(p);
+    p.pieces = prompt_pieces(order);
+    p.stride = order.stride;
+    p.delay = order.delay;
+    p.projecting_last = order.projecting_last;
     const hipError_t e = clear_exchange(p, workspace, bytes, st);
     if (e != hipSuccess) return e;
     void *args[] = {&p};

@@ -111,7 +111,8 @@ struct StackParams {
     int32_t layers, rows, Dp, n_proj, pieces, act, skip;
     uint32_t small16;
     int32_t batch, steps, chunks;   // of a sequence: rows is length * batch
-    int32_t stride, delay;          // and its order of pieces (prompt_stack.hip)
+    int32_t stride, delay;          // and its order of pieces (PromptOrder)
+    int32_t projecting_last;
 };
 // Where the step kernels take each of the layers, of which there have to be two. Layer by layer / in one launch, bf16, us a pass,
 // launched one by one and in a graph (8 layers unless another number is given; 256 workgroups, fewer and up to 0.88 of the time since):
@@ -172,6 +173,51 @@ inline StackPlan stack_plan(int64_t layers, int64_t length, int64_t batch, int64
     plan.states_at = plan.outputs_at + (layers - 1) * rows * Dp * 2;
     plan.bytes = kStackHeader + (size_t)(plan.states_at + layers * (plan.chunks - 1) * batch * Dp * 4);
     return plan;
+}
+// The order in which a prompt's pieces are numbered. A slot has the projecting pieces of one chunk of every `stride`-th
+// layer and then the walking ones `delay` chunks behind; of a slot's layers only the lowest can be at the last chunk, which
+// has fewer projecting pieces where it has fewer rows. There is no piece without rows: whoever runs one passes a barrier in it.
+struct PromptOrder {
+    int layers, chunks, stride, delay;
+    int projecting, projecting_last, walking;   // pieces of a chunk, and of the last one
+};
+struct PromptPiece {
+    int layer, chunk, index;   // index: among the chunk's pieces of its kind
+    bool project;
+};
+inline PromptOrder prompt_order(const StackParams &p) {
+    const int halves = p.steps * p.batch <= 32 ? 1 : 2, columns = p.n_proj / 32;   // (projecting pieces have 32 rows, chunks two halves)
+    const int last = p.rows - (p.chunks - 1) * p.steps * p.batch;
+    const int stride = halves == 1 ? 4 : 3;
+    return {p.layers, p.chunks, stride, p.n_proj ? stride - 2 : 0, columns * halves, columns * ((last + 31) / 32), (p.Dp + 63) / 64};
+}
+inline int prompt_pieces(const PromptOrder &o) {
+    return o.layers * ((o.chunks - 1) * o.projecting + o.projecting_last + o.chunks * o.walking);
+}
+// Piece `number`, which has to be one; slot and before (the number of pieces in slots in front of it) start from zero and are those of
+// the last piece asked for, of a smaller number.
+__host__ __device__ inline PromptPiece prompt_piece(const PromptOrder &o, int number, int &slot, int &before) {
+    const auto less = [](int a, int b) { return a < b ? a : b; };
+    const auto more = [](int a, int b) { return a < b ? b : a; };
+    for (;;) {   // (ends: `number` is that of a piece of some slot)
+        const int first = more(0, (slot - o.chunks + o.stride) / o.stride), first_walk = more(0, (slot - o.delay - o.chunks + o.stride) / o.stride);
+        const int layers = more(0, less(slot / o.stride, o.layers - 1) - first + 1);
+        const int walks = slot < o.delay ? 0 : more(0, less((slot - o.delay) / o.stride, o.layers - 1) - first_walk + 1);
+        const int absent = layers > 0 && slot - first * o.stride == o.chunks - 1 ? o.projecting - o.projecting_last : 0;
+        const int projects = layers * o.projecting - absent;
+        int i = number - before;
+        if (i < projects) {
+            if (i >= o.projecting - absent) i += absent;
+            return {first + i / o.projecting, slot - (first + i / o.projecting) * o.stride, i % o.projecting, true};
+        }
+        i -= projects;
+        if (i < walks * o.walking) {
+            const int layer = first_walk + i / o.walking;
+            return {layer, slot - o.delay - layer * o.stride, i % o.walking, false};
+        }
+        before += projects + walks * o.walking;
+        ++slot;
+    }
 }
 hipError_t clear_exchange(StackParams &p, void *workspace, size_t bytes, hipStream_t st);   // and sets where it is
 hipError_t launch_prompt_stack(StackParams p, void *workspace, size_t bytes, bool half, hipStream_t st);
