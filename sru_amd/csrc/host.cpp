@@ -163,7 +163,8 @@ bool prepare(Call &c, bool checkpointed, bool may_narrow) {
 void *stream_of(const c10::Device &device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
 
 // Other Python threads run while this one allocates, multiplies and launches, each of which may wait (for
-// memory, for room in a queue), as they do in torch's own calls. The tensors are held by the caller's arguments.
+// memory, for room in a queue), as they do in torch's own calls. The tensors are held by the caller's arguments; a call
+// that is given the objects which have them (stack_forward) holds their memory itself.
 class Unlocked {
     PyThreadState *const state = PyEval_SaveThread();
 
@@ -716,6 +717,8 @@ PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     s.state_interval = 1;
     s.x_dtype = SRU_AMD_X_AS_STREAMS;
     const void *projs[kLayers], *weights[kLayers], *wcs[kLayers], *biases[kLayers], *scales[kLayers];
+    // Another thread may give a cell another parameter, or a parameter other memory, while this one is unlocked.
+    c10::Storage held[kLayers][5];
     size_t need = 0;
     int64_t n_proj = 0;
     uint32_t flags = 0;
@@ -770,6 +773,9 @@ PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         wcs[l] = weight_c.ptr();
         biases[l] = bias.ptr();
         scales[l] = s.skip_type == 1 ? scale.ptr() : nullptr;
+        c10::Storage *hold = held[l];
+        for (const Arg *t : {&proj, &weight, &weight_c, &bias, &scale})
+            if (*t) *hold++ = (*t)->storage();
     }
     if (!plain(*x.t, device, length * batch * width, 16) || (init && (init->dim() != 3 || init->size(0) != layers)) ||
         !small(init, device, layers * batch * width, type, true, SRU_AMD_SMALL_INIT, flags) || !plain_pad(pad, device, length, batch))

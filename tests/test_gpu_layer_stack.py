@@ -170,6 +170,49 @@ def test_streams_and_threads():
     assert not wrong
 
 
+@pytest.mark.parametrize("replace", ["parameter", "memory"])
+@pytest.mark.parametrize("length", [1, 130])
+def test_weights_replaced_by_another_thread(length, replace):
+    """A call reads the weights that it found: they are equal ones here, and what is freed meanwhile becomes NaNs (all on one
+    stream, in the order of the calls)."""
+    model = make(256, torch.bfloat16, 8, projection_size=64)
+    x = torch.randn(length, 1, 256, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        assert model._whole_stack(x, None, None) is not None
+        want = model(x)
+    done, failed, rounds = threading.Event(), [], 0
+
+    def work():
+        try:
+            while not done.is_set():
+                for cell in model.rnn_lst:
+                    for name in ("weight", "weight_proj", "weight_c", "bias"):
+                        old = getattr(cell, name)
+                        size, new = old.shape, old.detach().clone()
+                        if replace == "memory":
+                            old.data = new
+                        else:
+                            setattr(cell, name, torch.nn.Parameter(new))
+                        del old, new
+                        torch.full(size, float("nan"), device="cuda", dtype=torch.bfloat16)
+        except BaseException as e:
+            failed.append(e)
+
+    thread = threading.Thread(target=work)
+    thread.start()
+    try:
+        with torch.no_grad():
+            for rounds in range(1, 301):
+                got = model(x)
+                if not all(torch.equal(a, b) for a, b in zip(got, want)):
+                    failed.append(rounds)
+                    break
+    finally:
+        done.set()
+        thread.join()
+    assert not failed and rounds == 300
+
+
 @pytest.mark.parametrize("length,batch", [(1, 16), (130, 1)])
 def test_recorded_and_replayed(length, batch):
     model = make(256, torch.bfloat16, 4, projection_size=64)
