@@ -382,10 +382,10 @@ class SRU(nn.Module):
     def _whole_stack(self, x: Tensor, c0: Optional[Tensor], mask_pad: Optional[Tensor]) -> Optional[Tuple[Tensor, Tensor]]:
         """All layers in one call without gradients: (output, last states), or None where they are called one by one, as they
         are wherever one of them could tell the difference (see `SRUCell._whole_layer`; hooks, a method put in place of a
-        cell's own, a module of another type in its place)."""
+        cell's own, a module of another type in its place) or not all of them are to run (a changed `num_layers`)."""
         if (torch.is_grad_enabled() or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not Tensor or torch.compiler.is_compiling()
                 or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or layer_forward is not _LAYER_FORWARD
-                or type(self.rnn_lst) is not nn.ModuleList or any(getattr(SRUCell, name) is not own for name, own in _CELL_METHODS)
+                or type(self.rnn_lst) is not nn.ModuleList or len(self.rnn_lst._modules) != self.num_layers or any(getattr(SRUCell, name) is not own for name, own in _CELL_METHODS)
                 or any(_GLOBAL_HOOKS)):
             return None
         return _lib.host().stack_forward(list(self.rnn_lst._modules.values()), SRUCell, x, c0, mask_pad)

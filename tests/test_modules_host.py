@@ -207,6 +207,23 @@ def test_a_step_put_in_place_of_the_layers_own_is_called(where, step, monkeypatc
         cell(x)
 
 
+@pytest.mark.parametrize("change", [None, lambda m: setattr(m, "num_layers", 2), lambda m: m.rnn_lst.append(SRUCell(8, 8))])
+def test_a_stack_in_one_call_has_as_many_layers_as_run_one_by_one(change, monkeypatch):
+    from sru_amd import _lib
+    model = SRU(8, 8, num_layers=3).bfloat16()
+    if change is not None:
+        change(model)
+    x = torch.zeros(2, 2, 8).bfloat16()
+    called = []
+    monkeypatch.setattr(_lib, "host", lambda: type("Host", (), {"stack_forward": staticmethod(lambda cells, *a: ("h", len(cells)))}))
+    for cell in model.rnn_lst:
+        monkeypatch.setattr(cell, "forward", lambda x, state, mask_pad=None: (called.append(1) or x, x[0]))
+    with torch.no_grad():
+        assert model._whole_stack(x, None, None) == (("h", 3) if change is None else None)
+        model(x)
+    assert len(called) == {None: 0}.get(change, model.num_layers)
+
+
 def test_native_calls_stand_aside_under_modes():
     """Under a mode that sees every call the native host code leaves the call to Python."""
     from torch.overrides import TorchFunctionMode
