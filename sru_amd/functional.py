@@ -453,7 +453,8 @@ _STEPS = _weight_gradient, _grad_workspace
 
 def replaced() -> bool:
     """Whether another function stands for a step of a layer with gradients, which then has to be called."""
-    return (_weight_gradient, _grad_workspace) != _STEPS or ElementwiseRecurrence.apply != _APPLY
+    return ((_weight_gradient, _grad_workspace) != _STEPS or ElementwiseRecurrence.apply != _APPLY
+            or ElementwiseRecurrence.forward is not _FORWARD or ElementwiseRecurrence.backward is not _BACKWARD)
 
 
 class ElementwiseRecurrence(Function):

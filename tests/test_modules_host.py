@@ -207,6 +207,18 @@ def test_a_step_put_in_place_of_the_layers_own_is_called(where, step, monkeypatc
         cell(x)
 
 
+@pytest.mark.parametrize("step", ["forward", "backward", "apply"])
+def test_a_step_put_in_place_of_the_recurrences_own_is_called(step, monkeypatch):
+    """A layer's node of native code stands for the Function as this package defines it."""
+    from sru_amd import ElementwiseRecurrence, _lib
+    cell, x = SRUCell(8, 8), torch.zeros(2, 2, 8)
+    node = (torch.ones(2, 2, 8), torch.ones(2, 8))
+    monkeypatch.setattr(_lib, "host", lambda: type("Host", (), {"layer": staticmethod(lambda *a: node)}))
+    assert cell._native_layer(x, x, None, cell.scale_x, None, None) is node
+    monkeypatch.setattr(ElementwiseRecurrence, step, staticmethod(_own_step))
+    assert cell._native_layer(x, x, None, cell.scale_x, None, None) is None
+
+
 @pytest.mark.parametrize("change", [None, lambda m: setattr(m, "num_layers", 2), lambda m: m.rnn_lst.append(SRUCell(8, 8))])
 def test_a_stack_in_one_call_has_as_many_layers_as_run_one_by_one(change, monkeypatch):
     from sru_amd import _lib
