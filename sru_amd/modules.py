@@ -281,8 +281,8 @@ class SRUCell(nn.Module):
 # assignment to the class may put others in their place, which are then called.
 _COMPUTE_UV, _COMPUTE_U, _APPLY_RECURRENCE = SRUCell.compute_UV, SRUCell.compute_U, SRUCell.apply_recurrence
 # ... and what a stack's one call stands for: whole cells, as torch calls them.
-_CELL_METHODS = tuple((name, getattr(SRUCell, name)) for name in ("__call__", "forward", "compute_UV", "compute_U", "apply_recurrence",
-                                                                  "_whole_layer", "_normalise"))
+_CELL_METHODS = tuple((name, getattr(SRUCell, name)) for name in ("__call__", "_call_impl", "forward", "compute_UV", "compute_U",
+                                                                  "apply_recurrence", "_whole_layer", "_normalise"))
 _LAYER_FORWARD, _DENSE, _RECURRENCE_GPU = layer_forward, dense, elementwise_recurrence_gpu
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks,
                  torch.nn.modules.module._global_backward_hooks, torch.nn.modules.module._global_backward_pre_hooks)

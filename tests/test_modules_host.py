@@ -219,6 +219,18 @@ def test_a_step_put_in_place_of_the_recurrences_own_is_called(step, monkeypatch)
     assert cell._native_layer(x, x, None, cell.scale_x, None, None) is None
 
 
+@pytest.mark.parametrize("name", ["__call__", "_call_impl", "forward", "compute_U", "apply_recurrence"])
+def test_a_stack_in_one_call_stands_for_cells_as_torch_calls_them(name, monkeypatch):
+    from sru_amd import _lib
+    model, x = SRU(8, 8).bfloat16(), torch.zeros(2, 2, 8).bfloat16()
+    monkeypatch.setattr(_lib, "host", lambda: type("Host", (), {"stack_forward": staticmethod(lambda *a: "whole")}))
+    with torch.no_grad():
+        assert model._whole_stack(x, None, None) == "whole"
+        own = getattr(SRUCell, name)
+        monkeypatch.setattr(torch.nn.Module if name.startswith("_") else SRUCell, name, lambda self, *a, **kw: own(self, *a, **kw))
+        assert model._whole_stack(x, None, None) is None
+
+
 @pytest.mark.parametrize("change", [None, lambda m: setattr(m, "num_layers", 2), lambda m: m.rnn_lst.append(SRUCell(8, 8))])
 def test_a_stack_in_one_call_has_as_many_layers_as_run_one_by_one(change, monkeypatch):
     from sru_amd import _lib
