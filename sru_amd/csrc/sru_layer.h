@@ -131,11 +131,19 @@ inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_p
 // by one are as fast or nearly so.
 //
 // What it saves is the walk that follows the walk of the layer before, per layer; what it costs is products in pieces of 64 rows
-// and less. Both are estimated, in ns. Layer by layer: per layer 10 us (15 with a projection), 31 ns a step, and the product at
-// 380 TFLOP/s. In chunks: the way through the layers, which the first chunk goes alone, then per chunk the walk, and the pieces of
-// all layers on 256 compute units. Fitted to 260 measured points (three to ten layers of 64 to 2048, one to four rows, 32 to 1024
-// steps); taken where chunks of 64 rows or of 32, the better of them, are expected to take 0.93
-// of the time. At 196 of these points they took 0.73 of it, the worst 1.06 (78 x 3 rows, 3 layers of 64, 36 -> 38 us). Inner sizes beyond one pass through LDS take longer than that where the walk is short.
+// and less, and words that every layer hands over. Both ways are estimated, in ns. Layer by layer: launches, 33 ns a step, and
+// products that read their weights and go at 2 PFLOP/s in the end, with the streams of the recurrence. In chunks: the way through
+// the layers, which the first chunk goes alone, then what follows each other from chunk to chunk (the walk's steps; more where
+// projections lie between and chunks are on their way in all layers), and the pieces of all layers on 256 compute units.
+//
+// Both are fitted to 10 892 points drawn at random, each measured in a graph layer by layer, in chunks of 64 rows and of 32 (three to
+// sixteen layers of 32 to 2048, projections up to 3/4, one to four rows, 32 to 4096 steps): standard deviations 4.6, 7.3 and 6.1%.
+// (An estimate fitted to 260 points of up to 1024 steps was up to 2.0 times slower than the layers one by one beyond them: 3550 x 3,
+// 13 layers of 2048 -> 512, 2959 -> 6021 us.) Where the better of the chunks is expected to take 0.93 of the time it takes 0.66 of it, over
+// 8 270 points; 0.9% of these take longer, 0.4% by more than 5%, the worst 1.27 (644 x 3, 13 layers of 1792 -> 448, 730 us layer by layer).
+// Launched one by one, a layer costs its host 12.4 us, 16 with a projection, of which 12 and 14 are counted on, and the launches here
+// take 7 us less than in a graph: three layers of 64, 32 steps, 47 us and 26, where a graph takes 34 and 33. Of 2 930 points of up to 600 steps
+// that are taken 4 are slower launched so, the worst 1.14. (3 803 further points that are taken, in a graph: 0.67, 3% slower, the worst 1.13.)
 // Layer by layer / chunks of 64 rows / 32, bf16, us a pass in a graph:
 //   one row   512 x 2048 -> 512, 10 layers 424/286/320    1024 of the same 640/496/628   128 of the same 229/163/144
 //             370 x 256, 10 layers 207/119/93     491 x 1024, 6 layers 215/139/133  230 x 512 -> 128, 4 layers 79/67/58
@@ -144,20 +152,30 @@ inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_p
 //   three     276 x 384, 6 layers 122/86/89       104 x 2048 -> 512, 8 layers 211/171/192
 //   four      143 x 384 -> 96, 10 layers 171/139/139      346 x 2048 -> 512, 10 layers 510/605/814
 constexpr int kStackRows = 64;        // rows of a chunk at the most
+struct ChunkCost {
+    int launch, layer, layer_projects, layer_step, chunk, chunk_waits, step, walk, walk_more, project;   // walk_more: past what LDS holds at once
+};
 inline int prompt_steps(int64_t layers, int64_t length, int64_t batch, int64_t Dp, int64_t n_proj) {
     const int64_t inner = n_proj ? n_proj : Dp, weights = n_proj ? 4 * Dp * n_proj : 3 * Dp * Dp;
     if (layers < 3 || layers > kStackMaxLayers || length < 32 || length > 4096 || batch > 4 || Dp % 32 != 0 || n_proj % 32 != 0 || n_proj >= Dp || Dp > 2048 ||
         inner > (length >= 256 ? 1024 : 512))
         return 0;
-    const int64_t one_by_one = layers * (n_proj ? 15500 : 10300) + layers * length * 31 + layers * length * batch * weights / 190000;
-    const auto in_chunks = [&](int64_t rows) {
-        const int64_t chunks = (length + rows / batch - 1) / (rows / batch), walks = (Dp + 63) / 64, projections = n_proj / 32 * (rows / 32);
-        const int64_t way = (rows == 64 ? 8800 + inner * 53 / 10 : 6900 + inner * 37 / 10) + (n_proj ? 2500 : 0);
-        return layers * way + chunks * ((rows == 64 ? 2400 : 1550) + layers * (walks * inner * 29 + projections * 38000) / 1000);
+    const int64_t one_by_one = 8600 + layers * (6300 + (n_proj ? 3000 : 0) + 33 * length + weights / 300 + length * batch * (weights + 6300 * Dp) / 1000000);
+    const auto in_chunks = [&](int64_t rows, int64_t stride, const ChunkCost &c) {
+        const int64_t steps = rows / batch, chunks = (length + steps - 1) / steps, walks = (Dp + 63) / 64, projections = n_proj / 32 * (rows / 32);
+        const int64_t waiting = n_proj && chunks > layers * stride ? chunks - layers * stride : 0;
+        return c.launch + layers * (c.layer + (n_proj ? c.layer_projects : 0) + c.layer_step * steps) + chunks * c.chunk + waiting * c.chunk_waits + length * c.step +
+               chunks * layers * (walks * (c.walk + (inner > 512 ? c.walk_more : 0)) + projections * c.project);
     };
-    const int64_t wide = in_chunks(kStackRows), narrow = in_chunks(kStackRows / 2);
-    return (wide < narrow ? wide : narrow) * 100 > one_by_one * 93 ? 0 : (int)((wide < narrow ? kStackRows : kStackRows / 2) / batch);
+    const int64_t wide = in_chunks(kStackRows, 3, ChunkCost{12000, 6570, 1800, 31, 745, 1120, 34, 31, 29, 26});
+    const int64_t narrow = in_chunks(kStackRows / 2, 4, ChunkCost{14000, 4450, 1680, 37, 650, 390, 31, 21, 27, 32});
+    const int64_t best = wide < narrow ? wide : narrow, launched = 10000 + layers * (n_proj ? 14000 : 12000);
+    return best * 100 > (one_by_one < launched ? launched : one_by_one) * 93 ? 0 : (int)((wide < narrow ? kStackRows : kStackRows / 2) / batch);
 }
+// A workspace holds what every layer hands over, over the whole sequence, and is filled and written once and read once each pass: where it
+// no longer fits beside the weights in the last-level cache the pieces wait for memory (10 layers of 2048 -> 512 reach this
+// at 4270 rows). Layer by layer two layers' worth are held.
+constexpr size_t kStackMaxBytes = (size_t)192 << 20;
 struct StackPlan {
     int steps, chunks;
     int64_t outputs_at, states_at;
@@ -172,7 +190,7 @@ inline StackPlan stack_plan(int64_t layers, int64_t length, int64_t batch, int64
     plan.outputs_at = layers * rows * n_proj * 2;
     plan.states_at = plan.outputs_at + (layers - 1) * rows * Dp * 2;
     plan.bytes = kStackHeader + (size_t)(plan.states_at + layers * (plan.chunks - 1) * batch * Dp * 4);
-    return plan;
+    return plan.bytes > kStackMaxBytes ? StackPlan{} : plan;
 }
 // The order in which a prompt's pieces are numbered. A slot has the projecting pieces of one chunk of every `stride`-th
 // layer and then the walking ones `delay` chunks behind; of a slot's layers only the lowest can be at the last chunk, which

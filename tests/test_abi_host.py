@@ -288,3 +288,17 @@ def test_every_product_kernel_in_the_library_can_be_chosen():
     tiles = {(1, 1, 1), (1, 1, 2), (1, 2, 1), (2, 2, 1)}
     for name, chosen in ((b"f", tiles), (b"NS_9bf16_bitsE", tiles | {(1, 2, 2), (2, 2, 2)}), (b"NS_9half_bitsE", tiles | {(1, 2, 2), (2, 2, 2)})):
         assert {tuple(map(int, b[1:])) for b in built if b[0] == name} == chosen
+
+
+# Prompts through stacks, us in a graph layer by layer / in chunks of 64 rows / of 32
+@pytest.mark.parametrize("length,batch,width,n_proj,layers,taken", [
+    (512, 1, 2048, 512, 10, True), (1024, 1, 2048, 512, 10, True),           # 424/286/320, 640/496/628
+    (3357, 3, 64, 0, 16, True), (1720, 3, 768, 96, 16, True),                # 1947/495, 1365/1005
+    (3550, 3, 2048, 512, 13, False), (3644, 4, 2048, 256, 10, False),        # 2959/6021, 2327/4635
+    (998, 4, 2048, 256, 13, False), (1000, 4, 1024, 0, 3, False),            # 997/1659, 208/341
+    (996, 3, 768, 0, 3, False), (3996, 4, 1024, 0, 3, False),                # 178/242, 688/1217
+    (4096, 4, 2048, 256, 16, False), (4096, 3, 1024, 0, 16, False)])         # workspaces of 1.3 GB and 0.4
+def test_prompts_go_by_what_was_measured(length, batch, width, n_proj, layers, taken):
+    shape = _lib.Shape(length, batch, width, 1, 3, 0, 1, 0, _lib.BF16, 1, _lib.X_AS_STREAMS)
+    nbytes = _lib.load().sru_amd_stack_workspace_bytes(ctypes.byref(shape), layers, n_proj)
+    assert (nbytes > 0) == taken and nbytes <= 192 << 20
