@@ -697,7 +697,7 @@ struct Cell {
 
 // stack_forward(cells, type of a cell, x, c0, mask_pad) -> (h, last states), or None where the layers have to be called one
 // by one: one of them is not of that type, has a step of its own, hooks, a normalisation, a module or dropout, or differs from the others
-// in its form, or there is no kernel for the stack
+// in its form, or there is no kernel for the stack or no room for its workspace
 PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Arg x, init, pad;
@@ -786,11 +786,15 @@ PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const Unlocked unlocked;
         const c10::DeviceGuard guard(device);
         const auto options = x->options();
-        h = at::empty({length, batch, width}, options);
-        last = at::empty({layers, batch, width}, options);
-        const at::Tensor workspace = at::empty({(int64_t)need / 4}, options.dtype(at::kFloat));
-        rc = sru_amd_stack_forward(&s, flags | SRU_AMD_SMALL_LAST, layers, n_proj, x.ptr(), projs, weights, wcs, biases, scales, init.ptr(),
-                                   static_cast<const uint8_t *>(pad.ptr()), h.data_ptr(), last.data_ptr(), workspace.data_ptr(), need, stream_of(device));
+        try {
+            h = at::empty({length, batch, width}, options);
+            last = at::empty({layers, batch, width}, options);
+            const at::Tensor workspace = at::empty({(int64_t)need / 4}, options.dtype(at::kFloat));
+            rc = sru_amd_stack_forward(&s, flags | SRU_AMD_SMALL_LAST, layers, n_proj, x.ptr(), projs, weights, wcs, biases, scales, init.ptr(),
+                                       static_cast<const uint8_t *>(pad.ptr()), h.data_ptr(), last.data_ptr(), workspace.data_ptr(), need, stream_of(device));
+        } catch (const c10::OutOfMemoryError &) {   // (layer by layer there is less at a time)
+            rc = SRU_AMD_ERR_WORKSPACE;
+        }
     }
     if (rc != SRU_AMD_OK) return none();
     return Py_BuildValue("(NN)", wrap(h), wrap(last));

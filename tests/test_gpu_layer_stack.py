@@ -170,6 +170,30 @@ def test_streams_and_threads():
     assert not wrong
 
 
+def test_no_room_for_the_workspace():
+    """Where the allocator refuses it, the layers are called one by one, which hold less at a time."""
+    model = make(2048, torch.bfloat16, 10, projection_size=512)
+    x = torch.randn(1024, 1, 2048, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        want = one_by_one(model, x)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_reserved()
+        one_by_one(model, x)
+        growth = torch.cuda.max_memory_reserved() - before
+        torch.cuda.empty_cache()
+        room = 1024 * (10 * 512 + 9 * 2048) * 2     # of the workspace, at the least
+        assert growth < room
+        torch.cuda.set_per_process_memory_fraction((before + growth + (2 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+        try:
+            got = model(x)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert model._whole_stack(x, None, None) is not None
+
+
 @pytest.mark.parametrize("replace", ["parameter", "memory"])
 @pytest.mark.parametrize("length", [1, 130])
 def test_weights_replaced_by_another_thread(length, replace):
