@@ -59,7 +59,7 @@
 extern "C" {
 #endif
 
-#define SRU_AMD_ABI_VERSION 7
+#define SRU_AMD_ABI_VERSION 8
 
 enum sru_amd_dtype {
     SRU_AMD_F32 = 0,
@@ -264,6 +264,7 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
  * skip_type 0 or 1, is_custom 0).
  *
  * sru_amd_stack_workspace_bytes: 0 where there is no kernel for the stack or the layers one by one are the faster way.
+ * sru_amd_stack_wanted_in_graph: whether the one launch is the faster way in a recorded graph too, where a launch costs its host nothing.
  *   x            (L, B, D') in shape->dtype
  *   weight_proj  `layers` pointers to (D', n_proj); NULL iff n_proj is 0
  *   weight       ... to (n_proj or D', 3 D'), both in shape->dtype, row-major
@@ -274,6 +275,7 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
  * Streams, weights and the workspace are 16-byte aligned. */
 #define SRU_AMD_STACK_MAX_LAYERS 16
 size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers, int64_t n_proj);
+int sru_amd_stack_wanted_in_graph(const sru_amd_shape *shape, int64_t layers, int64_t n_proj);
 int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t layers, int64_t n_proj, const void *x,
                           const void *const *weight_proj, const void *const *weight, const void *const *weight_c,
                           const void *const *bias, const void *const *scale_x, const void *c_init, const uint8_t *mask_pad,

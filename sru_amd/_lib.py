@@ -9,7 +9,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsru_amd.so")
-ABI_VERSION = 7
+ABI_VERSION = 8
 STATE_INTERVAL = 8   # SRU_AMD_STATE_INTERVAL
 STATIC_MAX_COLUMNS = 262144   # SRU_AMD_STATIC_MAX_COLUMNS
 NORM_MAX_FEATURES = 4096       # SRU_AMD_NORM_MAX_FEATURES
@@ -51,6 +51,7 @@ SIGNATURES = {
     "sru_amd_layer_route": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
     "sru_amd_layer_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 13),
     "sru_amd_stack_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
+    "sru_amd_stack_wanted_in_graph": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_int64, ctypes.c_int64]),
     "sru_amd_stack_forward": (ctypes.c_int, [ctypes.POINTER(Shape), ctypes.c_uint32, ctypes.c_int64, ctypes.c_int64] + [_P] * 11 + [ctypes.c_size_t, _P]),
     "sru_amd_product_wanted": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3),
     "sru_amd_product": (ctypes.c_int, [ctypes.c_int32] + [ctypes.c_int64] * 3 + [_P] * 4),

@@ -667,6 +667,14 @@ PyObject *layer_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// Whether what is launched now goes into a graph.
+bool recorded(const c10::Device &device) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(device.index()).stream(), &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // (another stream is, and this is the one that all wait for)
+    return false;
+}
+
 // What a cell holds under a name, borrowed; null: nothing.
 struct Cell {
     PyObject *const attributes, *const parameters, *const buffers;
@@ -697,7 +705,7 @@ struct Cell {
 
 // stack_forward(cells, type of a cell, x, c0, mask_pad) -> (h, last states), or None where the layers have to be called one
 // by one: one of them is not of that type, has a step of its own, hooks, a normalisation, a module or dropout, or differs from the others
-// in its form, or there is no kernel for the stack or no room for its workspace
+// in its form, or there is no kernel for the stack (or, in a graph, a slower one) or no room for its workspace
 PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     Arg x, init, pad;
@@ -755,7 +763,7 @@ PyObject *stack_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
             n_proj = project;
             if (d < 1 || d * s.dirs != width || (act != 0 && act != 1)) return none();
             need = sru_amd_stack_workspace_bytes(&s, layers, n_proj);
-            if (need == 0) return none();
+            if (need == 0 || (!sru_amd_stack_wanted_in_graph(&s, layers, n_proj) && recorded(device))) return none();
         }
         const int64_t inner = n_proj ? n_proj : width;
         uint32_t small16 = 0;

@@ -353,6 +353,11 @@ size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers,
     return stack_plan(layers, s.length, s.batch, s.hidden * s.dirs, n_proj).bytes;
 }
 
+int sru_amd_stack_wanted_in_graph(const sru_amd_shape *shape, int64_t layers, int64_t n_proj) {
+    if (sru_amd_stack_workspace_bytes(shape, layers, n_proj) == 0) return 0;
+    return shape->length > 1 || stack_wanted_in_graph(layers, shape->batch, shape->hidden * shape->dirs, n_proj);
+}
+
 int sru_amd_stack_forward(const sru_amd_shape *shape, uint32_t small16, int64_t layers, int64_t n_proj, const void *x,
                           const void *const *weight_proj, const void *const *weight, const void *const *weight_c,
                           const void *const *bias, const void *const *scale_x, const void *c_init, const uint8_t *mask_pad,

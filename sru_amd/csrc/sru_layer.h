@@ -127,6 +127,14 @@ struct StackParams {
 inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
     return layers >= 2 && layers <= kStackMaxLayers && n_proj < Dp && step_sizes_ok(rows, Dp, Dp, n_proj);
 }
+// ... and whether it is the faster way in a graph as well, where a launch costs its host nothing. Without projections few narrow layers are over
+// before the fill in front of them has paid off: a launch saves 0.6 us a layer and 1.6 more for 1000 features, less 10 ns a row, and the fill
+// costs 2.5, fitted to 762 sizes in a graph (2 to 16 layers of 32 to 2048, 1 to 64 rows). The 566 on this side take 0.83 of the time, the
+// worst 1.10 (32, six layers, 16 rows 22.1 / 24.3); of the 196 others 140 took longer, up to 1.19 (32, three layers, 48 rows 21.2 / 25.3). Launched one by
+// one all of them gain (37.0 / 17.8), as do all with projections in a graph.
+inline bool stack_wanted_in_graph(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
+    return n_proj > 0 || layers * (610 + 8 * Dp / 5 - 10 * rows) >= 2800;
+}
 // A sequence of a few batch rows through such a stack (prompt_stack.hip): time steps in a chunk, 0 where the layers one
 // by one are as fast or nearly so.
 //

@@ -302,3 +302,16 @@ def test_prompts_go_by_what_was_measured(length, batch, width, n_proj, layers, t
     shape = _lib.Shape(length, batch, width, 1, 3, 0, 1, 0, _lib.BF16, 1, _lib.X_AS_STREAMS)
     nbytes = _lib.load().sru_amd_stack_workspace_bytes(ctypes.byref(shape), layers, n_proj)
     assert (nbytes > 0) == taken and nbytes <= 192 << 20
+
+
+# One step through stacks, us in a graph layer by layer / in one launch, which is the faster way for all of these launched one by one
+@pytest.mark.parametrize("rows,width,n_proj,layers,wanted", [
+    (48, 32, 0, 3, 0), (64, 64, 0, 8, 0), (16, 64, 0, 2, 0),          # 21.2/25.3, 51.4/53.5, 18.2/17.6
+    (64, 2048, 0, 2, 1), (1, 1024, 0, 2, 1), (16, 256, 0, 8, 1),      # 46.0/44.4, 18.4/18.4
+    (48, 64, 32, 3, 1)])
+def test_one_step_in_a_graph(rows, width, n_proj, layers, wanted):
+    shape = _lib.Shape(1, rows, width, 1, 3, 0, 1, 0, _lib.BF16, 1, _lib.X_AS_STREAMS)
+    lib = _lib.load()
+    assert lib.sru_amd_stack_workspace_bytes(ctypes.byref(shape), layers, n_proj) > 0
+    assert lib.sru_amd_stack_wanted_in_graph(ctypes.byref(shape), layers, n_proj) == wanted
+    assert lib.sru_amd_stack_wanted_in_graph(ctypes.byref(shape), 17, n_proj) == 0 and lib.sru_amd_stack_wanted_in_graph(None, layers, n_proj) == 0

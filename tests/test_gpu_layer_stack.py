@@ -255,6 +255,27 @@ def test_recorded_and_replayed(length, batch):
             torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("d,layers,rows,taken", [(64, 2, 16, False), (32, 3, 48, False), (256, 8, 16, True)])
+def test_one_step_in_a_graph_where_launches_cost_the_host_nothing(d, layers, rows, taken):
+    model = make(d, torch.bfloat16, layers)
+    x = torch.randn(1, rows, d, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        assert model._whole_stack(x, None, None) is not None
+        one_by_one(model, x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            assert (model._whole_stack(x, None, None) is not None) == taken
+            h, c = model(x)
+        for _ in range(3):
+            x.copy_(torch.randn(1, rows, d, device="cuda"))
+            graph.replay()
+            for want in (one_by_one(model, x), model(x)):   # (the same sums, up to a contraction: see check)
+                for a, b in zip((h, c), want):
+                    assert float(((a.double() - b.double()).abs() / b.double().abs().clamp(min=1.0)).max()) <= 2 * EPS[torch.bfloat16] * layers
+            torch.cuda.synchronize()
+
+
 def test_layers_that_could_tell_are_called():
     x = torch.randn(1, 4, 64, device="cuda").to(torch.bfloat16)
     whole = lambda m: m._whole_stack(x, None, None) is not None
