@@ -281,8 +281,12 @@ class SRUCell(nn.Module):
 # assignment to the class may put others in their place, which are then called.
 _COMPUTE_UV, _COMPUTE_U, _APPLY_RECURRENCE = SRUCell.compute_UV, SRUCell.compute_U, SRUCell.apply_recurrence
 # ... and what a stack's one call stands for: whole cells, as torch calls them.
-_CELL_METHODS = tuple((name, getattr(SRUCell, name)) for name in ("__call__", "_call_impl", "forward", "compute_UV", "compute_U",
-                                                                  "apply_recurrence", "_whole_layer", "_normalise"))
+def _cell_methods():
+    return (SRUCell.__call__, SRUCell._call_impl, SRUCell.forward, SRUCell.compute_UV, SRUCell.compute_U, SRUCell.apply_recurrence, SRUCell._whole_layer,
+            SRUCell._normalise)
+
+
+_CELL_METHODS = _cell_methods()
 _LAYER_FORWARD, _DENSE, _RECURRENCE_GPU = layer_forward, dense, elementwise_recurrence_gpu
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks,
                  torch.nn.modules.module._global_backward_hooks, torch.nn.modules.module._global_backward_pre_hooks)
@@ -383,12 +387,15 @@ class SRU(nn.Module):
         """All layers in one call without gradients: (output, last states), or None where they are called one by one, as they
         are wherever one of them could tell the difference (see `SRUCell._whole_layer`; hooks, a method put in place of a
         cell's own, a module of another type in its place) or not all of them are to run (a changed `num_layers`)."""
-        if (torch.is_grad_enabled() or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not Tensor or torch.compiler.is_compiling()
-                or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or layer_forward is not _LAYER_FORWARD
-                or type(self.rnn_lst) is not nn.ModuleList or len(self.rnn_lst._modules) != self.num_layers or any(getattr(SRUCell, name) is not own for name, own in _CELL_METHODS)
-                or any(_GLOBAL_HOOKS)):
+        # (what rules most calls out first, and the list of layers looked up once: a stack that is not taken pays for being asked)
+        if (self.num_layers < 2 or torch.is_grad_enabled() or x.dtype not in (torch.float16, torch.bfloat16) or torch.compiler.is_compiling()
+                or type(x) is not Tensor or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or layer_forward is not _LAYER_FORWARD):
             return None
-        return _lib.host().stack_forward(list(self.rnn_lst._modules.values()), SRUCell, x, c0, mask_pad)
+        layers = self._modules.get("rnn_lst")
+        if (type(layers) is not nn.ModuleList or len(layers._modules) != self.num_layers or any(_GLOBAL_HOOKS)
+                or _cell_methods() != _CELL_METHODS):
+            return None
+        return _lib.host().stack_forward(list(layers._modules.values()), SRUCell, x, c0, mask_pad)
 
     def reset_parameters(self):
         for layer in self.rnn_lst:
