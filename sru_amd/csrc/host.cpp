@@ -428,11 +428,11 @@ PyObject *recurrence(PyObject *, PyObject *const *a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// x^T grad in `dtype`
+// x^T grad in `dtype` (under a mode that sees every call, or of what a hook made something else of, a call of torch's)
 at::Tensor weight_gradient(const at::Tensor &x, const at::Tensor &grad, at::ScalarType dtype) {
     int32_t code = 0, out_code = 0;
     const int64_t rows = x.size(0), inner = x.size(1), cols = grad.size(1);
-    if (!at::GradMode::is_enabled() && narrow(x.scalar_type()) && x.scalar_type() == grad.scalar_type() && dtype_code(x.scalar_type(), code) &&
+    if (!at::GradMode::is_enabled() && !observed() && usable(x) && usable(grad) && narrow(x.scalar_type()) && x.scalar_type() == grad.scalar_type() && dtype_code(x.scalar_type(), code) &&
         dtype_code(dtype, out_code) && plain(x, grad.device(), rows * inner, 16) && plain(grad, grad.device(), rows * cols, 16)) {
         const int64_t need = (int64_t)sru_amd_product_grad_workspace_bytes(code, rows, inner, cols);
         if (need > 0) {

@@ -94,6 +94,29 @@ def test_graph_properties():
     assert float((again - full[0]).abs().max()) <= 1e-5 * float(full[0].abs().max())
 
 
+def test_a_backward_pass_that_a_mode_watches_shows_its_products():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Products(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen += func in (torch.ops.aten.mm.default, torch.ops.aten.addmm_.default)
+            return func(*args, **(kwargs or {}))
+
+    cell, x = SRUCell(512, 512, n_proj=128).cuda(), torch.randn(256, 32, 512, device="cuda").bfloat16().requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        h, _ = cell(x)
+    assert h.grad_fn.name() == "SRULayerBackward" and functional._grad_workspace(torch.bfloat16, 8192, 512, 128) > 0
+    probe, leaves = torch.randn_like(h), (x, cell.weight, cell.weight_proj)
+    want = torch.autograd.grad(h, leaves, probe, retain_graph=True)
+    with Products() as products:
+        got = torch.autograd.grad(h, leaves, probe)
+    assert products.seen == 4     # of two weights, of what was projected and of the input
+    for a, b in zip(got, want):   # (a weight's is rounded to 16 bits on the way here)
+        assert a.dtype == b.dtype and float((a.float() - b.float()).abs().max()) <= 2.0 ** -7 * float(b.float().abs().max())
+
+
 @pytest.mark.parametrize("kw", [{}, dict(n_proj=32)])
 def test_what_is_differentiable_twice_stays_so(kw, monkeypatch):
     """The dense products are, the recurrence's gradients are constants."""
