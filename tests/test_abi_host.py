@@ -315,3 +315,44 @@ def test_one_step_in_a_graph(rows, width, n_proj, layers, wanted):
     assert lib.sru_amd_stack_workspace_bytes(ctypes.byref(shape), layers, n_proj) > 0
     assert lib.sru_amd_stack_wanted_in_graph(ctypes.byref(shape), layers, n_proj) == wanted
     assert lib.sru_amd_stack_wanted_in_graph(ctypes.byref(shape), 17, n_proj) == 0 and lib.sru_amd_stack_wanted_in_graph(None, layers, n_proj) == 0
+
+
+def test_a_stacks_call_checks_its_arguments_before_launching():
+    lib = _lib.load()
+    layers, width, n_proj = 3, 64, 32
+    shape = _lib.Shape(1, 4, width, 1, 3, 0, 1, 0, _lib.BF16, 1, _lib.X_AS_STREAMS)
+    need = lib.sru_amd_stack_workspace_bytes(ctypes.byref(shape), layers, n_proj)
+    pointers = lambda *at: (ctypes.c_void_p * layers)(*(at or [0x1000] * layers))
+    # x, weight_proj, weight, weight_c, bias, scale_x, c_init, mask_pad, h, c_last, workspace, its bytes
+    fine = dict(x=FAKE, weight_proj=pointers(), weight=pointers(), weight_c=pointers(), bias=pointers(), scale_x=pointers(), c_init=FAKE, mask_pad=FAKE,
+                h=FAKE, c_last=FAKE, workspace=FAKE, nbytes=need)
+
+    def call(shape=shape, small16=0, layers=layers, n_proj=n_proj, **kw):
+        a = dict(fine, **kw)
+        return lib.sru_amd_stack_forward(ctypes.byref(shape) if shape else None, small16, layers, n_proj, *list(a.values())[:-1], a["nbytes"], None)
+
+    code = _lib_status
+    assert call(shape=None) == code("NULL_POINTER") and call(workspace=None) == code("WORKSPACE") and call(nbytes=need - 1) == code("WORKSPACE")
+    assert call(workspace=ctypes.c_void_p(0x1008)) == code("WORKSPACE")
+    for name in ("x", "weight_proj", "weight", "weight_c", "bias", "h", "c_last"):
+        assert call(**{name: None}) == code("NULL_POINTER"), name
+    for name in ("weight_proj", "weight", "weight_c", "bias"):      # ... and one layer's
+        assert call(**{name: pointers(0x1000, None, 0x1000)}) == code("NULL_POINTER"), name
+    for name, at in (("x", 0x1008), ("h", 0x1008), ("c_init", 0x1002), ("c_last", 0x1002)):
+        assert call(**{name: ctypes.c_void_p(at)}) == code("MISALIGNED"), name
+    for name, at in (("weight_proj", 0x1008), ("weight", 0x1008), ("weight_c", 0x1002), ("bias", 0x1002), ("scale_x", 0x1002)):
+        assert call(**{name: pointers(0x1000, 0x1000, at)}) == code("MISALIGNED"), name
+    every = _lib.SMALL_WEIGHT_C | _lib.SMALL_BIAS | _lib.SMALL_INIT | _lib.SMALL_SCALE | _lib.SMALL_LAST      # 16 bits: two-byte alignment, which leaves x to refuse
+    odd = ctypes.c_void_p(0x1002)
+    assert call(small16=every, c_init=odd, c_last=odd, weight_c=pointers(*[0x1002] * 3), bias=pointers(*[0x1002] * 3), scale_x=pointers(*[0x1002] * 3),
+                x=None) == code("NULL_POINTER")
+    assert call(small16=every, weight_c=pointers(0x1001, 0x1000, 0x1000)) == code("MISALIGNED")
+    assert call(small16=1 << 20) == code("BAD_FLAGS")
+    # what there is no kernel for
+    other = lambda **kw: _lib.Shape(*[kw.get(f[0], getattr(shape, f[0])) for f in _lib.Shape._fields_])
+    for bad in (other(dtype=_lib.F32), other(k=4, skip_type=2), other(is_custom=1), other(batch=65), other(hidden=48), other(length=2), other(length=64, dirs=2, hidden=32)):
+        assert lib.sru_amd_stack_workspace_bytes(ctypes.byref(bad), layers, n_proj) == 0
+        assert call(shape=bad) == code("BAD_SHAPE")
+    for n, p in ((1, n_proj), (17, n_proj), (-1, n_proj), (layers, -32), (layers, 64), (layers, 33)):
+        assert lib.sru_amd_stack_workspace_bytes(ctypes.byref(shape), n, p) == 0 and call(layers=n, n_proj=p) == code("BAD_SHAPE")
+    assert call(shape=other(dirs=3)) == code("BAD_FLAGS") and call(shape=other(batch=0)) == code("BAD_SHAPE")
