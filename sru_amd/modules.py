@@ -167,9 +167,11 @@ class SRUCell(nn.Module):
                       mask_pad: Optional[Tensor]) -> Optional[Tuple[Tensor, Tensor]]:
         """compute_UV and apply_recurrence with gradients, as one node of the graph, where the layer projects with its own
         weights, no step is overridden or replaced, and nothing watches, transforms or compiles torch's calls."""
+        if torch.compiler.is_compiling():
+            return None
         # (what rules most calls out first: a layer of 16-bit parameters, of which the node reads the small ones in float only, or a frozen one)
-        bias = None if torch.compiler.is_compiling() else self._parameters.get("bias")
-        if bias is None or bias.dtype is not torch.float32 or not self._recorded(input, residual, c0):
+        bias = self._parameters.get("bias")      # (none: a replica's, or one made anew for each call)
+        if bias is not None and (bias.dtype is not torch.float32 or not self._recorded(input, residual, c0)):
             return None
         if (self.custom_m is not None or not getattr(self, "native_16bit", True) or input.size(-1) != self.input_size
                 or getattr(self.compute_UV, "__func__", None) is not _COMPUTE_UV or getattr(self.compute_U, "__func__", None) is not _COMPUTE_U
@@ -181,9 +183,10 @@ class SRUCell(nn.Module):
                                                   self.hidden_size, self.bidirectional, self.has_skip_term, scale_val, mask_c, mask_pad)
 
     def _recorded(self, *inputs: Optional[Tensor]) -> bool:
-        for t in (*inputs, *self._parameters.values()):
-            if t is not None and t.requires_grad:
-                return True
+        for tensors in (self._parameters.values(), inputs):
+            for t in tensors:
+                if t is not None and t.requires_grad:
+                    return True
         return False
 
     def _whole_layer(self, input: Tensor, residual: Tensor) -> bool:

@@ -231,7 +231,8 @@ def test_a_stack_in_one_call_stands_for_cells_as_torch_calls_them(name, monkeypa
         assert model._whole_stack(x, None, None) is None
 
 
-@pytest.mark.parametrize("kind,asked", [("plain", True), ("16-bit", False), ("frozen", False), ("frozen, the input's gradient", True), ("frozen, the state's gradient", True)])
+@pytest.mark.parametrize("kind,asked", [("plain", True), ("16-bit", False), ("frozen", False), ("frozen, the input's gradient", True), ("frozen, the state's gradient", True),
+                                        ("a replica's", True)])
 def test_a_layers_node_is_asked_for_where_it_can_be(kind, asked, monkeypatch):
     from sru_amd import _lib
     cell, x, c0, calls = SRUCell(8, 8), torch.zeros(2, 2, 8), torch.zeros(2, 8), []
@@ -240,6 +241,10 @@ def test_a_layers_node_is_asked_for_where_it_can_be(kind, asked, monkeypatch):
     cell.requires_grad_("frozen" not in kind)
     x.requires_grad_("input" in kind)
     c0.requires_grad_("state" in kind)
+    if "replica" in kind:        # (torch.nn.DataParallel gives it its parameters as attributes)
+        for name, p in list(cell._parameters.items()):
+            del cell._parameters[name]
+            cell.__dict__[name] = p
     monkeypatch.setattr(_lib, "host", lambda: type("Host", (), {"layer": staticmethod(lambda *a: calls.append(1))}))
     assert cell._native_layer(x, x, c0, cell.scale_x, None, None) is None
     assert bool(calls) == asked
