@@ -259,11 +259,12 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
                           void *h, void *c_last, void *stream);
 
 /* A stack of such layers, each of the width of its input, in one launch (two with the clearing of the workspace): one time
- * step of up to 64 rows, or a sequence of one or two batch rows in one direction, through up to SRU_AMD_STACK_MAX_LAYERS layers of
- * one form (sru/modules.py:617-652, a loop over the layers there). `shape` is that of each layer's recurrence (16-bit streams, k 3,
- * skip_type 0 or 1, is_custom 0).
+ * step of up to 64 rows through two layers or more, or a sequence of 32 to 4096 steps of one to four batch rows in one direction
+ * through three or more, SRU_AMD_STACK_MAX_LAYERS at the most and all of one form (sru/modules.py:617-652, a loop over the
+ * layers there). `shape` is that of each layer's recurrence (16-bit streams, k 3, skip_type 0 or 1, is_custom 0).
  *
- * sru_amd_stack_workspace_bytes: 0 where there is no kernel for the stack or the layers one by one are the faster way.
+ * sru_amd_stack_workspace_bytes: 0 where there is no kernel for the stack, the layers one by one are the faster way, or what all layers hand
+ * over, 2 L B (layers (D' + n_proj) - D') bytes and a little, is more than 192 MB. The call writes all of it.
  * sru_amd_stack_wanted_in_graph: whether the one launch is the faster way in a recorded graph too, where a launch costs its host nothing.
  *   x            (L, B, D') in shape->dtype
  *   weight_proj  `layers` pointers to (D', n_proj); NULL iff n_proj is 0
@@ -272,7 +273,8 @@ int sru_amd_layer_forward(const sru_amd_shape *shape, uint32_t small16, int64_t 
  *   c_init       (layers, B, D') or NULL; c_last (layers, B, D')
  *   h            (L, B, D'), the last layer's
  *   workspace    16-byte aligned; contents before and after are undefined
- * Streams, weights and the workspace are 16-byte aligned. */
+ * Streams, weights and the workspace are 16-byte aligned. Workgroups wait for each other's results, and every wait ends by itself; should one
+ * last some seconds all the same it is given up, the call has returned SRU_AMD_OK, and h and c_last hold NaNs. */
 #define SRU_AMD_STACK_MAX_LAYERS 16
 size_t sru_amd_stack_workspace_bytes(const sru_amd_shape *shape, int64_t layers, int64_t n_proj);
 int sru_amd_stack_wanted_in_graph(const sru_amd_shape *shape, int64_t layers, int64_t n_proj);

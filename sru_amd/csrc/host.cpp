@@ -6,8 +6,8 @@
 //
 // Why: a forward and backward pass of the recurrence cost the host 145-175 us in Python, more than the
 // kernels of most sizes take. 128 x 32 x 1024 f32 with padding, 53 us of kernels: 159 us a pass then,
-// 90-94 us through here (with Python's autograd around it); one token through ten layers of 2048: 221
-// and 133 us.
+// 90-94 us through here with Python's autograd around it and 73 with a node of the graph that is native as
+// well; one token through ten layers of 2048: 221 us, 133 and, as one call for the stack, 71.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -286,8 +286,8 @@ at::Tensor product(const at::Tensor &x, const at::Tensor &weight, int32_t dtype,
 
 // ---------------------------------------------------------------- autograd
 // The graph's own nodes in the plain case. Python's autograd Functions cost some 25 us of host time a pass more for the
-// recurrence and 60 for a layer: two float layers of 256, 32 steps of 32 rows, 320 -> 163-220 us a training step with 105 us of
-// kernels; the recurrence alone, 128 x 32 x 1024 float padded, 96 -> 76 us with 53. A layer that knows both of its parts also adds the
+// recurrence and 60 for a layer: two float layers of 256, 32 steps of 32 rows, 320 -> 188-223 us a training step (one or the other
+// of two times, by process) with 93 us of kernels; the recurrence alone, 128 x 32 x 1024 float padded, 96 -> 76 us with 53. A layer that knows both of its parts also adds the
 // skip term's gradient in the product that makes the rest of it: 512 x 16 rows, ten layers of 2048 under autocast 4246 -> 4091 us.
 
 using torch::autograd::SavedVariable;

@@ -5,7 +5,8 @@
 // wait for each other, 5.4 and 7.9 us each, of which the weights' way from memory is a quarter. Here a workgroup takes
 // pieces of work in the order in which they depend on each other and has a piece's weights on their way before what
 // the piece reads exists: 134 -> 69 us a pass, 49 with one row (134), 174 with 64 (236); 2048 features without a projection, 8 layers, 95 -> 65;
-// six layers of 512 features 63 -> 21. Recorded in a graph 109 -> 67 (8 layers), two layers without a projection level.
+// six layers of 512 features 64 -> 22. Recorded in a graph 106 -> 65 (8 layers); few narrow layers without projections are
+// slower so and go one by one there (stack_wanted_in_graph).
 // What bounds it now, per layer and 16 rows, 6.2 us: handing 64 KB of outputs and 16 KB of projected rows over, 1.5 and 1.0 us;
 // from the arrival to the store 1.2 us each, of which the matrix instructions are a tenth and the partial sums' way through LDS half.
 //

@@ -10,8 +10,8 @@
 //
 // Pieces. A chunk is a number of time steps of all batch rows, 64 rows at the most. Per layer and chunk there are n_proj / 32
 // pieces that project 32 columns each (sru_stack.h), and Dp / 64 that make U for 64 cells, float and never in memory, and walk
-// the chunk's steps. A piece only reads what pieces of smaller numbers write; how they are drawn and how they hand results over
-// is layer_stack.hip's.
+// the chunk's steps. A piece only reads what pieces of smaller numbers write (prompt_piece in sru_layer.h has the numbers); how they are
+// drawn and how they hand results over is layer_stack.hip's.
 //
 // Their order. From a layer to the next it is three times as far as from a chunk to the next, which waits for a walk alone, so a
 // layer's projection of a chunk is numbered with what is `stride` chunks further on in the layer before, and its walk `delay`

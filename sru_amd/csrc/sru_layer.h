@@ -115,15 +115,16 @@ struct StackParams {
     int32_t projecting_last;
 };
 // Where the step kernels take each of the layers, of which there have to be two. Layer by layer / in one launch, bf16, us a pass,
-// launched one by one and in a graph (8 layers unless another number is given; 256 workgroups, fewer and up to 0.88 of the time since):
+// launched one by one and in a graph (8 layers unless another number is given):
 //                          1 row                  16 rows                 64 rows
-//   64                  81/24   30/25          82/23   30/29           81/53   55/60
-//   1024                86/32   57/38          86/38   64/45          111/87  115/92
-//   2048                85/60   89/68          95/72   99/78          162/134 167/139
-//   2048 -> 512        112/43   96/49         107/61  109/68          189/145 193/151
-//   3072               189/139 193/149        211/165 216/173         233/267 233/272 (past the step kernels' sizes)
-//   two of 64           30/18   18/21          28/16   16/17           27/15   21/22
-//   two of 2048         27/20   29/27          28/22   32/30           45/38   49/45
+//   64                  82/21   27/25          82/23   29/29           81/48   51/53
+//   1024                81/26   54/32          81/32   61/38          102/79  106/86
+//   2048                84/56   87/62          93/64   96/70          154/127 157/134
+//   2048 -> 512        108/41   94/47         109/59  106/65          181/143 184/149
+//   2048 -> 512, ten   133/49  115/56         136/71  130/77          225/177 228/182
+//   3072               187/142 191/147        209/167 212/172         (past the step kernels' sizes)
+//   two of 64           27/15   18/18          27/15   19/19           28/16   19/21
+//   two of 2048         27/20   28/27          28/23   30/29           42/37   46/44
 inline bool stack_sizes_ok(int64_t layers, int64_t rows, int64_t Dp, int64_t n_proj) {
     return layers >= 2 && layers <= kStackMaxLayers && n_proj < Dp && step_sizes_ok(rows, Dp, Dp, n_proj);
 }
