@@ -286,8 +286,8 @@ at::Tensor product(const at::Tensor &x, const at::Tensor &weight, int32_t dtype,
 
 // ---------------------------------------------------------------- autograd
 // The graph's own nodes in the plain case. Python's autograd Functions cost some 25 us of host time a pass more for the
-// recurrence and 60 for a layer: two float layers of 256, 32 steps of 32 rows, 320 -> 188-223 us a training step (one or the other
-// of two times, by process) with 93 us of kernels; the recurrence alone, 128 x 32 x 1024 float padded, 96 -> 76 us with 53. A layer that knows both of its parts also adds the
+// recurrence and 60 for a layer: two float layers of 256, 32 steps of 32 rows, 320 -> 152-165 or 213-223 us a training step (the
+// host takes one time or the other, by process) with 93 us of kernels; the recurrence alone, 128 x 32 x 1024 float padded, 96 -> 76 us with 53. A layer that knows both of its parts also adds the
 // skip term's gradient in the product that makes the rest of it: 512 x 16 rows, ten layers of 2048 under autocast 4246 -> 4091 us.
 
 using torch::autograd::SavedVariable;
