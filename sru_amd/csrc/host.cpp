@@ -19,6 +19,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/PyInterpreter.h>
+#include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -466,6 +467,7 @@ struct LayerNode : torch::autograd::Node {
         const auto self = shared_from_this();
         at::Tensor grads[kGradients];
         gradients_of(kept, self, out[0], out[1], grads);
+        if (!torch::autograd::get_current_graph_task_keep_graph()) kept.release();   // (room for the products' results)
         const c10::DeviceGuard guard(grads[0].device());
         variable_list result(7);
         result[WeightC] = grads[2];

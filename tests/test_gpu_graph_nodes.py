@@ -94,6 +94,33 @@ def test_graph_properties():
     assert float((again - full[0]).abs().max()) <= 1e-5 * float(full[0].abs().max())
 
 
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("kw", [{}, dict(n_proj=128)])
+def test_memory_of_a_backward_pass(kw, autocast, monkeypatch):
+    """What the recurrence's part has read is free before the products' results are made, as where they are nodes of their own; with the graph kept
+    it stays."""
+    cell, x = SRUCell(1024, 1024, **kw).cuda(), torch.randn(64, 64, 1024, device="cuda").requires_grad_()
+    with torch.no_grad():
+        probe = torch.randn(64, 64, 1024, device="cuda").to(torch.bfloat16 if autocast else torch.float32)
+    leaves = [x, *cell.parameters()]
+
+    def peak(keep=False):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            h, _ = cell(x)
+        torch.cuda.reset_peak_memory_stats()
+        grads = torch.autograd.grad(h, leaves, probe, retain_graph=keep)
+        most = torch.cuda.max_memory_allocated()
+        if keep:
+            assert all(torch.equal(a, b) for a, b in zip(grads, torch.autograd.grad(h, leaves, probe)))
+        return most
+
+    peak(), peak(True)
+    node = peak()
+    monkeypatch.setattr(functional, "replaced", lambda: True)
+    peak()
+    assert node <= peak() + (2 << 20)     # (allocations are rounded)
+
+
 def test_a_backward_pass_that_a_mode_watches_shows_its_products():
     from torch.utils._python_dispatch import TorchDispatchMode
 
